@@ -250,6 +250,20 @@ int kd_plan_build_tokens(const kd_token_args *t, void *plan, int64_t plan_bytes,
  * _flash_attn_fwd (original_kernel.py:1697-1778, kernel :279-626). */
 int kd_attn_fwd(const kd_attn_args *a, const void *plan, int64_t plan_bytes, void *stream);
 
+/* The same with a workspace.  Shapes with few row blocks (small B H T) leave
+ * most of the GPU idle when each block is one workgroup's; given a workspace
+ * of kd_attn_fwd_ws_bytes bytes the blocks' key lists are cut into pieces that
+ * run side by side, and a second kernel puts the fp32 partial results
+ * together.  kd_attn_fwd_ws_bytes is 0 where that would not pay (then, and
+ * with ws NULL, kd_attn_fwd_ws is kd_attn_fwd), -1 on bad arguments; it
+ * depends on a's B, H, T, D and dtype only.  The results are the same at every
+ * call (the pieces are added in a fixed order) and differ from kd_attn_fwd's
+ * by the rounding of fp32 sums.  ws is 16-byte aligned, used by this call
+ * alone until its work on the stream is done, and needs no initial contents. */
+int64_t kd_attn_fwd_ws_bytes(const kd_attn_args *a);
+int kd_attn_fwd_ws(const kd_attn_args *a, const void *plan, int64_t plan_bytes, void *ws, int64_t ws_bytes,
+                   void *stream);
+
 /* -Delta = -rowsum(O * dO) in fp32 into a->delta[0 : B*H*T], and -LSE / c
  * (the form kd_attn_bwd_dkdv starts its score accumulators from; -inf for
  * fully masked rows) into a->delta[B*H*T : 2*B*H*T].  Replaces
@@ -274,6 +288,13 @@ int kd_attn_bwd_dkdv(const kd_attn_args *a, const void *plan, int64_t plan_bytes
 /* Whole backward: dQ with Delta (kd_attn_bwd_dq_delta), then dK/dV.  Replaces
  * attention_backward_adapter (original_kernel.py:1806-1898). */
 int kd_attn_bwd(const kd_attn_args *a, const void *plan, int64_t plan_bytes, void *stream);
+
+/* The same with a workspace, as kd_attn_fwd_ws (dQ over pieces of the key
+ * lists, dK and dV over pieces of the query lists; one workspace serves both
+ * in turn).  a->delta is required as for kd_attn_bwd. */
+int64_t kd_attn_bwd_ws_bytes(const kd_attn_args *a);
+int kd_attn_bwd_ws(const kd_attn_args *a, const void *plan, int64_t plan_bytes, void *ws, int64_t ws_bytes,
+                   void *stream);
 
 /* The whole backward as kd_attn_bwd, with a->delta ignored: its workspace
  * (2 * B*H*T floats) lives in a library-owned device array of

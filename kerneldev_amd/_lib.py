@@ -126,6 +126,10 @@ SIGNATURES = {
     "kd_plan_layout": (c_int, [c_int32, c_int32, c_int32, POINTER(c_int64)]),
     "kd_plan_build": (c_int, [POINTER(MetaArgs), c_void_p, c_int64, c_void_p]),
     "kd_attn_fwd": (c_int, [POINTER(AttnArgs), c_void_p, c_int64, c_void_p]),
+    "kd_attn_fwd_ws_bytes": (c_int64, [POINTER(AttnArgs)]),
+    "kd_attn_fwd_ws": (c_int, [POINTER(AttnArgs), c_void_p, c_int64, c_void_p, c_int64, c_void_p]),
+    "kd_attn_bwd_ws_bytes": (c_int64, [POINTER(AttnArgs)]),
+    "kd_attn_bwd_ws": (c_int, [POINTER(AttnArgs), c_void_p, c_int64, c_void_p, c_int64, c_void_p]),
     "kd_attn_bwd_delta": (c_int, [POINTER(AttnArgs), c_void_p]),
     "kd_attn_bwd_dq": (c_int, [POINTER(AttnArgs), c_void_p, c_int64, c_void_p]),
     "kd_attn_bwd_dq_delta": (c_int, [POINTER(AttnArgs), c_void_p, c_int64, c_void_p]),

@@ -178,6 +178,17 @@ def _attn_args(q, k, v, sm_scale, prec=_lib.KD_PREC_SPLIT) -> AttnArgs:
 
 
 # ----------------------------------------------------------------- custom ops
+def _workspace(nbytes: int, device):
+    """Scratch for the partial results of a call whose work lists are cut into pieces, or None."""
+    if nbytes < 0:
+        raise ValueError(_lib.load().kd_last_error_string().decode(errors="replace"))
+    return torch.empty(nbytes, dtype=torch.uint8, device=device) if nbytes else None
+
+
+def _ws_ref(ws) -> tuple:
+    return (None, 0) if ws is None else (ctypes.c_void_p(ws.data_ptr()), ws.numel())
+
+
 def _new_out(B, H, T, D, q, bthd: bool) -> torch.Tensor:
     """O as [B, H, T, D]: contiguous, or a view of [B, T, H, D] memory (bthd)."""
     if bthd:
@@ -248,7 +259,9 @@ def _fwd_op(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, lens: torch.Tenso
     a.o, a.o_strides = o.data_ptr(), _strides3(o)
     a.lse = lse.data_ptr()
     a.o_lo = o_lo.data_ptr() if need_lo else None
-    _lib.check(_lib.load().kd_attn_fwd(ctypes.byref(a), *_lib.plan_ref(plan), _stream(q.device)), "kd_attn_fwd")
+    lib = _lib.load()
+    ws = _workspace(lib.kd_attn_fwd_ws_bytes(ctypes.byref(a)), q.device)
+    _lib.check(lib.kd_attn_fwd_ws(ctypes.byref(a), *_lib.plan_ref(plan), *_ws_ref(ws), _stream(q.device)), "kd_attn_fwd")
     return o, lse, (plan if plan_in is None else plan.new_empty(0)), o_lo, q_r, k_r, q8_o, k8_o, qs_o, ks_o
 
 
@@ -294,7 +307,9 @@ def _bwd_op(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: torch.Tensor, 
     a.o_lo = o_lo.data_ptr() if o_lo.numel() > 0 else None
     _set_fp8(a, _fp8_tuple(q8, k8, q_scale, k_scale))
     a.dqk_signs = dqk_signs.data_ptr() if dqk_signs is not None else None
-    _lib.check(_lib.load().kd_attn_bwd(ctypes.byref(a), *_lib.plan_ref(plan), _stream(q.device)), "kd_attn_bwd")
+    lib = _lib.load()
+    ws = _workspace(lib.kd_attn_bwd_ws_bytes(ctypes.byref(a)), q.device)
+    _lib.check(lib.kd_attn_bwd_ws(ctypes.byref(a), *_lib.plan_ref(plan), *_ws_ref(ws), _stream(q.device)), "kd_attn_bwd")
     return dq, dk, dv
 
 

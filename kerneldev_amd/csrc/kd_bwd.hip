@@ -202,7 +202,7 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void k_dq(AttnArgs a, const 
                                                const uint32_t* __restrict__ list,
                                                const int32_t* __restrict__ count,
                                                const uint32_t* __restrict__ order, int nT, int nQB,
-                                               bool fuse_delta) {
+                                               bool fuse_delta, SplitArgs sp) {
   constexpr bool SP = NSP >= 2, S3 = NSP == 3;
   using TL = Tile<D>;
   using SO = ScoreOp<E, D, Q8>;  // S^T = K Q^T (16-bit, or fp8 from the K8 tile)
@@ -232,8 +232,10 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void k_dq(AttnArgs a, const 
             c = lane & 31;
   const int T = a.T, H = a.H;
   const int work = xcd_remap(blockIdx.x, gridDim.x);
-  const int h = work / (a.B * nQB);  // head-major, then the plan's longest-first order
-  const int item = int(order[work - h * (a.B * nQB)]);
+  const int h = work / (a.B * nQB * sp.ns);  // head-major, then the plan's longest-first order
+  int rank = work - h * (a.B * nQB * sp.ns);
+  const int piece = split_piece(sp.ns, &rank);
+  const int item = int(order[rank]);
   const int b = item / nQB, qblock = item - b * nQB, bh = b * H + h;
 
   const uint16_t* qg = static_cast<const uint16_t*>(a.q) + b * a.q_strides[0] + h * a.q_strides[1];
@@ -326,8 +328,9 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void k_dq(AttnArgs a, const 
   uint32_t qcode = qvalid ? codes_b[qrow] : 0u;
 
   const int lbase = item;  // b nQB + qblock
-  const int n = count[lbase];
+  int n = count[lbase];
   const uint32_t* ent = list + int64_t(lbase) * nT;
+  split_list(sp.ns, piece, &ent, &n);
 
   uint32_t koff[NLK], voff[NL], k8off[NL8];
   TLK::load_offsets(wave, lane, krb, koff, KHALF ? uint32_t(DH) * 2u : dbytes);
@@ -518,7 +521,9 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void k_dq(AttnArgs a, const 
     if (e + 1 < n) step(e + 1, std::integral_constant<int, 1>{});
   }
 
-  if (qvalid) {
+  if (sp.ns > 1) {  // a piece of the list: the sum as it stands (kd_combine.hip)
+    if (qvalid) store_part<DH>(sp.part + ((int64_t(piece) * a.B * H + bh) * T + qrow) * a.D + D0, acc, hf, DH == D ? a.D : DH);
+  } else if (qvalid) {
     uint16_t* g = static_cast<uint16_t*>(a.dq) + b * a.dq_strides[0] + h * a.dq_strides[1] + qrow * a.dq_strides[2];
     void* glo = lo_row(a.dq_lo, (int64_t(b) * a.H + h) * a.T + qrow, a.D, S3);
     if constexpr (DH == D) {
@@ -551,7 +556,7 @@ template <class E, int D, bool Q8, int NSP>
 __global__ __launch_bounds__(512, 1) void k_dkdv(AttnArgs a, const uint32_t* __restrict__ codes,
                                                  const uint32_t* __restrict__ list,
                                                  const int32_t* __restrict__ count,
-                                                 const uint32_t* __restrict__ order, int nT, int nKB) {
+                                                 const uint32_t* __restrict__ order, int nT, int nKB, SplitArgs sp) {
   constexpr bool SP = NSP >= 2, S3 = NSP == 3;
   constexpr int NW = 8;
   using TL = Tile<D, NW>;
@@ -584,8 +589,10 @@ __global__ __launch_bounds__(512, 1) void k_dkdv(AttnArgs a, const uint32_t* __r
   const int pair = wave & 3, role = wave >> 2;
   const int T = a.T, H = a.H;
   const int work = xcd_remap(blockIdx.x, gridDim.x);
-  const int h = work / (a.B * nKB);  // head-major, then the plan's longest-first dK/dV order
-  const int item = int(order[work - h * (a.B * nKB)]);
+  const int h = work / (a.B * nKB * sp.ns);  // head-major, then the plan's longest-first dK/dV order
+  int rank = work - h * (a.B * nKB * sp.ns);
+  const int piece = split_piece(sp.ns, &rank);
+  const int item = int(order[rank]);
   const int b = item / nKB, kblock = item - b * nKB, bh = b * H + h;
 
   const uint16_t* qg = static_cast<const uint16_t*>(a.q) + b * a.q_strides[0] + h * a.q_strides[1];
@@ -629,8 +636,9 @@ __global__ __launch_bounds__(512, 1) void k_dkdv(AttnArgs a, const uint32_t* __r
   uint32_t kcode = kvalid ? codes[int64_t(b) * T + krow] : 0u;
 
   const int lbase = b * nKB + kblock;
-  const int n = count[lbase];
+  int n = count[lbase];
   const uint32_t* ent = list + int64_t(lbase) * nT;
+  split_list(sp.ns, piece, &ent, &n);
 
   // The P waves make every copy (the four of them share each tile): the dS
   // waves carry the longer chain of a step, the P waves wait for them at the
@@ -948,7 +956,10 @@ __global__ __launch_bounds__(512, 1) void k_dkdv(AttnArgs a, const uint32_t* __r
     sl = ahead(sl, 1);
   }
 
-  if (kvalid) {
+  if (sp.ns > 1) {  // a piece of the list: the sum as it stands, dV's then dK's (kd_combine.hip)
+    if (kvalid)
+      store_part<D>(sp.part + ((int64_t(role * sp.ns + piece) * a.B * H + bh) * T + krow) * D, acc, hf, D);
+  } else if (kvalid) {
     uint16_t* g = role == 0
         ? static_cast<uint16_t*>(a.dv) + b * a.dv_strides[0] + h * a.dv_strides[1] + krow * a.dv_strides[2]
         : static_cast<uint16_t*>(a.dk) + b * a.dk_strides[0] + h * a.dk_strides[1] + krow * a.dk_strides[2];
@@ -979,7 +990,7 @@ template <class E, int D, int NSP, int DH, int D0, bool Q8 = false>
 __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void k_dkdv_wide(AttnArgs a, const uint32_t* __restrict__ codes,
                                                       const uint32_t* __restrict__ list,
                                                       const int32_t* __restrict__ count,
-                                                      const uint32_t* __restrict__ order, int nT, int nKB) {
+                                                      const uint32_t* __restrict__ order, int nT, int nKB, SplitArgs sp) {
   constexpr bool SP = NSP >= 2, S3 = NSP == 3;
   using TL = Tile<D, 4>;
   // fp8 scores (Q8): S^T comes from the e4m3 Q8 tile and this lane's K8 row,
@@ -1003,8 +1014,10 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void k_dkdv_wide(AttnArgs a, 
             c = lane & 31;
   const int T = a.T, H = a.H;
   const int work = xcd_remap(blockIdx.x, gridDim.x);
-  const int h = work / (a.B * nKB);  // head-major, then the plan's longest-first dK/dV order
-  const int item = int(order[work - h * (a.B * nKB)]);
+  const int h = work / (a.B * nKB * sp.ns);  // head-major, then the plan's longest-first dK/dV order
+  int rank = work - h * (a.B * nKB * sp.ns);
+  const int piece = split_piece(sp.ns, &rank);
+  const int item = int(order[rank]);
   const int b = item / nKB, kblock = item - b * nKB, bh = b * H + h;
 
   const uint16_t* qg = static_cast<const uint16_t*>(a.q) + b * a.q_strides[0] + h * a.q_strides[1];
@@ -1049,8 +1062,9 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void k_dkdv_wide(AttnArgs a, 
   uint32_t kcode = kvalid ? codes[int64_t(b) * T + krow] : 0u;
 
   const int lbase = b * nKB + kblock;
-  const int n = count[lbase];
+  int n = count[lbase];
   const uint32_t* ent = list + int64_t(lbase) * nT;
+  split_list(sp.ns, piece, &ent, &n);
 
   uint32_t qoff[NLQ], dooff[NL], q8off[NL8];
   TLQ::load_offsets(wave, lane, qrb, qoff, QHALF ? uint32_t(DH) * 2u : dbytes);
@@ -1255,7 +1269,13 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void k_dkdv_wide(AttnArgs a, 
     }
   }
 
-  if (kvalid) {
+  if (sp.ns > 1) {  // a piece of the list: the sums as they stand, dV's then dK's (kd_combine.hip)
+    if (kvalid) {
+      const int dlim = DH == D ? a.D : DH;
+      store_part<DH>(sp.part + ((int64_t(piece) * a.B * H + bh) * T + krow) * a.D + D0, acc_v, hf, dlim);
+      store_part<DH>(sp.part + ((int64_t(sp.ns + piece) * a.B * H + bh) * T + krow) * a.D + D0, acc_k, hf, dlim);
+    }
+  } else if (kvalid) {
     uint16_t* gv = static_cast<uint16_t*>(a.dv) + b * a.dv_strides[0] + h * a.dv_strides[1] + krow * a.dv_strides[2];
     uint16_t* gk = static_cast<uint16_t*>(a.dk) + b * a.dk_strides[0] + h * a.dk_strides[1] + krow * a.dk_strides[2];
     const int64_t row = (int64_t(b) * a.H + h) * a.T + krow;
@@ -1284,68 +1304,68 @@ static void launch_delta_t(const AttnArgs& a, hipStream_t st) {
   hipLaunchKernelGGL((k_delta<E, D>), dim3(unsigned((rows + RPB - 1) / RPB)), dim3(256), 0, st, a);
 }
 template <class E, int D, bool Q8, int NSP>
-static void launch_dq_s(const AttnArgs& a, const uint8_t* plan, hipStream_t st, bool fuse_delta) {
+static void launch_dq_s(const AttnArgs& a, const uint8_t* plan, const SplitArgs& sp, hipStream_t st, bool fuse_delta) {
   const PlanLayout L = plan_layout(a.B, a.T, a.D);
-  const unsigned grid = unsigned(a.B) * a.H * L.n_dq_blocks;
+  const unsigned grid = unsigned(a.B) * a.H * L.n_dq_blocks * sp.ns;
   auto* codes = reinterpret_cast<const uint32_t*>(plan + L.codes);
   auto* list = reinterpret_cast<const uint32_t*>(plan + L.dq_list);
   auto* cnt = reinterpret_cast<const int32_t*>(plan + L.dq_count);
   auto* order = reinterpret_cast<const uint32_t*>(plan + L.dq_order);
   if constexpr (D == 256) {  // two launches, the column halves of dQ; the first forms Delta
     hipLaunchKernelGGL((k_dq<E, D, Q8, NSP, 128, 0>), dim3(grid), dim3(256), 0, st, a, codes, list, cnt, order, L.nT,
-                       L.n_dq_blocks, fuse_delta);
+                       L.n_dq_blocks, fuse_delta, sp);
     hipLaunchKernelGGL((k_dq<E, D, Q8, NSP, 128, 128>), dim3(grid), dim3(256), 0, st, a, codes, list, cnt, order, L.nT,
-                       L.n_dq_blocks, false);
+                       L.n_dq_blocks, false, sp);
   } else {
     hipLaunchKernelGGL((k_dq<E, D, Q8, NSP>), dim3(grid), dim3(256), 0, st, a, codes, list, cnt, order, L.nT,
-                       L.n_dq_blocks, fuse_delta);
+                       L.n_dq_blocks, fuse_delta, sp);
   }
 }
 template <class E, int D, bool Q8 = false>
-static void launch_dq_t(const AttnArgs& a, const uint8_t* plan, hipStream_t st, bool fuse_delta) {
+static void launch_dq_t(const AttnArgs& a, const uint8_t* plan, const SplitArgs& sp, hipStream_t st, bool fuse_delta) {
   switch (parts_of(a.precision)) {
-    case 1: launch_dq_s<E, D, Q8, 1>(a, plan, st, fuse_delta); break;
-    case 2: launch_dq_s<E, D, Q8, 2>(a, plan, st, fuse_delta); break;
+    case 1: launch_dq_s<E, D, Q8, 1>(a, plan, sp, st, fuse_delta); break;
+    case 2: launch_dq_s<E, D, Q8, 2>(a, plan, sp, st, fuse_delta); break;
     default:
-      if constexpr (!Q8) launch_dq_s<E, D, Q8, 3>(a, plan, st, fuse_delta);  // (refused with fp8 by the C ABI)
+      if constexpr (!Q8) launch_dq_s<E, D, Q8, 3>(a, plan, sp, st, fuse_delta);  // (refused with fp8 by the C ABI)
       break;
   }
 }
 template <class E, int D, bool Q8, int NSP>
-static void launch_dkdv_s(const AttnArgs& a, const uint8_t* plan, hipStream_t st) {
+static void launch_dkdv_s(const AttnArgs& a, const uint8_t* plan, const SplitArgs& sp, hipStream_t st) {
   const PlanLayout L = plan_layout(a.B, a.T, a.D);
-  const unsigned grid = unsigned(a.B) * a.H * L.n_dkdv_blocks;
+  const unsigned grid = unsigned(a.B) * a.H * L.n_dkdv_blocks * sp.ns;
   if constexpr (D == 64) {  // one launch, all four products per wave (fp8 scores too)
     hipLaunchKernelGGL((k_dkdv_wide<E, D, NSP, 64, 0, Q8>), dim3(grid), dim3(256), 0, st, a,
                        reinterpret_cast<const uint32_t*>(plan + L.codes),
                        reinterpret_cast<const uint32_t*>(plan + L.dkdv_list),
                        reinterpret_cast<const int32_t*>(plan + L.dkdv_count),
-                       reinterpret_cast<const uint32_t*>(plan + L.dkdv_order), L.nT, L.n_dkdv_blocks);
+                       reinterpret_cast<const uint32_t*>(plan + L.dkdv_order), L.nT, L.n_dkdv_blocks, sp);
   } else if constexpr (D == 256) {  // two launches, the column halves of dK and dV (fp8 scores too)
     auto* codes = reinterpret_cast<const uint32_t*>(plan + L.codes);
     auto* list = reinterpret_cast<const uint32_t*>(plan + L.dkdv_list);
     auto* cnt = reinterpret_cast<const int32_t*>(plan + L.dkdv_count);
     auto* order = reinterpret_cast<const uint32_t*>(plan + L.dkdv_order);
     hipLaunchKernelGGL((k_dkdv_wide<E, D, NSP, 128, 0, Q8>), dim3(grid), dim3(256), 0, st, a, codes, list, cnt, order,
-                       L.nT, L.n_dkdv_blocks);
+                       L.nT, L.n_dkdv_blocks, sp);
     hipLaunchKernelGGL((k_dkdv_wide<E, D, NSP, 128, 128, Q8>), dim3(grid), dim3(256), 0, st, a, codes, list, cnt,
-                       order, L.nT, L.n_dkdv_blocks);
+                       order, L.nT, L.n_dkdv_blocks, sp);
   } else {
     hipLaunchKernelGGL((k_dkdv<E, D, Q8, NSP>), dim3(grid), dim3(512), 0, st, a,
                        reinterpret_cast<const uint32_t*>(plan + L.codes),
                        reinterpret_cast<const uint32_t*>(plan + L.dkdv_list),
                        reinterpret_cast<const int32_t*>(plan + L.dkdv_count),
-                       reinterpret_cast<const uint32_t*>(plan + L.dkdv_order), L.nT, L.n_dkdv_blocks);
+                       reinterpret_cast<const uint32_t*>(plan + L.dkdv_order), L.nT, L.n_dkdv_blocks, sp);
   }
 }
 
 template <class E, int D, bool Q8 = false>
-static void launch_dkdv_t(const AttnArgs& a, const uint8_t* plan, hipStream_t st) {
+static void launch_dkdv_t(const AttnArgs& a, const uint8_t* plan, const SplitArgs& sp, hipStream_t st) {
   switch (parts_of(a.precision)) {
-    case 1: launch_dkdv_s<E, D, Q8, 1>(a, plan, st); break;
-    case 2: launch_dkdv_s<E, D, Q8, 2>(a, plan, st); break;
+    case 1: launch_dkdv_s<E, D, Q8, 1>(a, plan, sp, st); break;
+    case 2: launch_dkdv_s<E, D, Q8, 2>(a, plan, sp, st); break;
     default:
-      if constexpr (!Q8) launch_dkdv_s<E, D, Q8, 3>(a, plan, st);  // (refused with fp8 by the C ABI)
+      if constexpr (!Q8) launch_dkdv_s<E, D, Q8, 3>(a, plan, sp, st);  // (refused with fp8 by the C ABI)
       break;
   }
 }
@@ -1376,33 +1396,41 @@ static void launch_delta_e(const AttnArgs& a, hipStream_t st) {
 }
 
 int launch_delta(const AttnArgs& a, hipStream_t st) {
-  if (use_simt(a)) return launch_simt_kernel(1, a, nullptr, st);
+  if (use_simt(a)) return launch_simt_kernel(1, a, nullptr, SplitArgs{nullptr, 1}, st);
   if (a.dtype == KD_BF16) launch_delta_e<BF16>(a, st);
   else launch_delta_e<F16>(a, st);
   return hipGetLastError() == hipSuccess ? KD_OK : KD_ERR_LAUNCH;
 }
-int launch_dq(const AttnArgs& a, const uint8_t* plan, hipStream_t st, bool fuse_delta) {
+int launch_dq(const AttnArgs& a, const uint8_t* plan, float* ws, hipStream_t st, bool fuse_delta) {
+  const SplitArgs sp{ws, ws == nullptr ? 1 : split_pieces(a, SPLIT_DQ)};
   if (use_simt(a)) {
-    const int r = fuse_delta ? launch_simt_kernel(1, a, plan, st) : KD_OK;
-    return r ? r : launch_simt_kernel(2, a, plan, st);
+    int r = fuse_delta ? launch_simt_kernel(1, a, plan, sp, st) : KD_OK;
+    if (!r) r = launch_simt_kernel(2, a, plan, sp, st);
+    return r || sp.ns == 1 ? r : launch_combine_dq(a, sp, st);
   }
   if (a.q8 != nullptr) {  // fp8 QK^T: bf16 at head dim 64, 128 or 256 (checked by the C ABI)
-    if (a.D == 64) launch_dq_t<BF16, 64, true>(a, plan, st, fuse_delta);
-    else if (a.D == 128) launch_dq_t<BF16, 128, true>(a, plan, st, fuse_delta);
-    else launch_dq_t<BF16, 256, true>(a, plan, st, fuse_delta);
+    if (a.D == 64) launch_dq_t<BF16, 64, true>(a, plan, sp, st, fuse_delta);
+    else if (a.D == 128) launch_dq_t<BF16, 128, true>(a, plan, sp, st, fuse_delta);
+    else launch_dq_t<BF16, 256, true>(a, plan, sp, st, fuse_delta);
   }
-  else KD_DISPATCH(launch_dq_t, a, plan, st, fuse_delta);
-  return hipGetLastError() == hipSuccess ? KD_OK : KD_ERR_LAUNCH;
+  else KD_DISPATCH(launch_dq_t, a, plan, sp, st, fuse_delta);
+  if (hipGetLastError() != hipSuccess) return KD_ERR_LAUNCH;
+  return sp.ns == 1 ? KD_OK : launch_combine_dq(a, sp, st);
 }
-int launch_dkdv(const AttnArgs& a, const uint8_t* plan, hipStream_t st) {
-  if (use_simt(a)) return launch_simt_kernel(3, a, plan, st);
-  if (a.q8 != nullptr) {  // fp8 QK^T: bf16 at head dim 64, 128 or 256 (checked by the C ABI)
-    if (a.D == 64) launch_dkdv_t<BF16, 64, true>(a, plan, st);
-    else if (a.D == 128) launch_dkdv_t<BF16, 128, true>(a, plan, st);
-    else launch_dkdv_t<BF16, 256, true>(a, plan, st);
+int launch_dkdv(const AttnArgs& a, const uint8_t* plan, float* ws, hipStream_t st) {
+  const SplitArgs sp{ws, ws == nullptr ? 1 : split_pieces(a, SPLIT_DKDV)};
+  if (use_simt(a)) {
+    const int r = launch_simt_kernel(3, a, plan, sp, st);
+    return r || sp.ns == 1 ? r : launch_combine_dkdv(a, sp, st);
   }
-  else KD_DISPATCH(launch_dkdv_t, a, plan, st);
-  return hipGetLastError() == hipSuccess ? KD_OK : KD_ERR_LAUNCH;
+  if (a.q8 != nullptr) {  // fp8 QK^T: bf16 at head dim 64, 128 or 256 (checked by the C ABI)
+    if (a.D == 64) launch_dkdv_t<BF16, 64, true>(a, plan, sp, st);
+    else if (a.D == 128) launch_dkdv_t<BF16, 128, true>(a, plan, sp, st);
+    else launch_dkdv_t<BF16, 256, true>(a, plan, sp, st);
+  }
+  else KD_DISPATCH(launch_dkdv_t, a, plan, sp, st);
+  if (hipGetLastError() != hipSuccess) return KD_ERR_LAUNCH;
+  return sp.ns == 1 ? KD_OK : launch_combine_dkdv(a, sp, st);
 }
 
 }  // namespace kd

@@ -118,7 +118,7 @@ int check_plan(const void* plan, int64_t plan_bytes, int B, int T, int D) {
 
 extern "C" {
 
-int kd_version(void) { return 30300; }
+int kd_version(void) { return 30400; }
 
 const char* kd_last_error_string(void) { return g_err.c_str(); }
 
@@ -271,7 +271,31 @@ static int check_fp8(const kd_attn_args* a) {
   return KD_OK;
 }
 
+// A caller's workspace: NULL (none), or 16-byte aligned and as large as the shape needs
+static int check_ws(const void* ws, int64_t ws_bytes, int64_t need) {
+  if (ws == nullptr) return KD_OK;
+  if (!aligned16(ws)) return fail(KD_ERR_INVALID, "ws must be 16-byte aligned");
+  if (ws_bytes < need) {
+    g_err = "ws is " + std::to_string(ws_bytes) + " bytes; this shape needs " + std::to_string(need);
+    return KD_ERR_INVALID;
+  }
+  return KD_OK;
+}
+
+int64_t kd_attn_fwd_ws_bytes(const kd_attn_args* a) {
+  return check_common(a) ? -1 : 4 * kd::split_floats(*a, kd::SPLIT_FWD);
+}
+
+int64_t kd_attn_bwd_ws_bytes(const kd_attn_args* a) {  // (dQ's pieces are put together before dK/dV's are made)
+  return check_common(a) ? -1 : 4 * std::max(kd::split_floats(*a, kd::SPLIT_DQ), kd::split_floats(*a, kd::SPLIT_DKDV));
+}
+
 int kd_attn_fwd(const kd_attn_args* a, const void* plan, int64_t plan_bytes, void* stream) {
+  return kd_attn_fwd_ws(a, plan, plan_bytes, nullptr, 0, stream);
+}
+
+int kd_attn_fwd_ws(const kd_attn_args* a, const void* plan, int64_t plan_bytes, void* ws, int64_t ws_bytes,
+                   void* stream) {
   int r = check_common(a);
   if (r) return r;
   if ((r = check_fp8(a))) return r;
@@ -280,7 +304,10 @@ int kd_attn_fwd(const kd_attn_args* a, const void* plan, int64_t plan_bytes, voi
       (r = check_tensor(a->v, a->v_strides, "v", a->T, a->D, esz(a))) || (r = check_tensor(a->o, a->o_strides, "o", a->T, a->D, esz(a))))
     return r;
   if ((r = check_o_lo(a))) return r;
-  r = kd::launch_fwd(*a, static_cast<const uint8_t*>(plan), as_stream(stream));
+  const int64_t need = kd_attn_fwd_ws_bytes(a);
+  if ((r = check_ws(ws, ws_bytes, need))) return r;
+  r = kd::launch_fwd(*a, static_cast<const uint8_t*>(plan), need > 0 ? static_cast<float*>(ws) : nullptr,
+                     as_stream(stream));
   return r ? fail(r, "kernel launch failed (forward)") : KD_OK;
 }
 
@@ -319,7 +346,7 @@ int kd_attn_bwd_dq(const kd_attn_args* a, const void* plan, int64_t plan_bytes, 
   int r = check_bwd(a, plan, plan_bytes);
   if (r) return r;
   if ((r = check_tensor(a->dq, a->dq_strides, "dq", a->T, a->D, esz(a)))) return r;
-  r = kd::launch_dq(*a, static_cast<const uint8_t*>(plan), as_stream(stream), false);
+  r = kd::launch_dq(*a, static_cast<const uint8_t*>(plan), nullptr, as_stream(stream), false);
   return r ? fail(r, "kernel launch failed (dq)") : KD_OK;
 }
 
@@ -327,7 +354,7 @@ int kd_attn_bwd_dkdv(const kd_attn_args* a, const void* plan, int64_t plan_bytes
   int r = check_bwd(a, plan, plan_bytes);
   if (r) return r;
   if ((r = check_tensor(a->dk, a->dk_strides, "dk", a->T, a->D, esz(a))) || (r = check_tensor(a->dv, a->dv_strides, "dv", a->T, a->D, esz(a)))) return r;
-  r = kd::launch_dkdv(*a, static_cast<const uint8_t*>(plan), as_stream(stream));
+  r = kd::launch_dkdv(*a, static_cast<const uint8_t*>(plan), nullptr, as_stream(stream));
   return r ? fail(r, "kernel launch failed (dkdv)") : KD_OK;
 }
 
@@ -337,7 +364,7 @@ int kd_attn_bwd_dq_delta(const kd_attn_args* a, const void* plan, int64_t plan_b
   if ((r = check_tensor(a->o, a->o_strides, "o", a->T, a->D, esz(a))) || (r = check_tensor(a->dq, a->dq_strides, "dq", a->T, a->D, esz(a))))
     return r;
   if ((r = check_o_lo(a))) return r;
-  r = kd::launch_dq(*a, static_cast<const uint8_t*>(plan), as_stream(stream), true);
+  r = kd::launch_dq(*a, static_cast<const uint8_t*>(plan), nullptr, as_stream(stream), true);
   return r ? fail(r, "kernel launch failed (dq)") : KD_OK;
 }
 
@@ -355,10 +382,20 @@ static int check_bwd_all(const kd_attn_args* a, const void* plan, int64_t plan_b
 }
 
 int kd_attn_bwd(const kd_attn_args* a, const void* plan, int64_t plan_bytes, void* stream) {
+  return kd_attn_bwd_ws(a, plan, plan_bytes, nullptr, 0, stream);
+}
+
+int kd_attn_bwd_ws(const kd_attn_args* a, const void* plan, int64_t plan_bytes, void* ws, int64_t ws_bytes,
+                   void* stream) {
   int r = check_bwd_all(a, plan, plan_bytes);
   if (r) return r;
-  r = kd_attn_bwd_dq_delta(a, plan, plan_bytes, stream);
-  return r ? r : kd_attn_bwd_dkdv(a, plan, plan_bytes, stream);
+  if ((r = check_ws(ws, ws_bytes, kd_attn_bwd_ws_bytes(a)))) return r;
+  const uint8_t* p = static_cast<const uint8_t*>(plan);
+  auto part = [&](kd::SplitPass pass) { return kd::split_floats(*a, pass) > 0 ? static_cast<float*>(ws) : nullptr; };
+  r = kd::launch_dq(*a, p, part(kd::SPLIT_DQ), as_stream(stream), true);
+  if (r) return fail(r, "kernel launch failed (dq)");
+  r = kd::launch_dkdv(*a, p, part(kd::SPLIT_DKDV), as_stream(stream));
+  return r ? fail(r, "kernel launch failed (dkdv)") : KD_OK;
 }
 
 int kd_attn_bwd_noalloc(const kd_attn_args* a, const void* plan, int64_t plan_bytes, void* stream) {

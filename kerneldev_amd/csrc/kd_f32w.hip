@@ -235,15 +235,17 @@ KD_DEV float group_sum(float x) {
 
 // Work item of this workgroup: head hh, plan item (batch row, block) and member.
 struct Item {
-  int hh, b, blk, member;
+  int hh, b, blk, member, piece;
 };
-KD_DEV Item item_of(const AttnArgs& a, int nblk, const uint32_t* order) {
+KD_DEV Item item_of(const AttnArgs& a, int nblk, const uint32_t* order, int ns) {
   const int work = xcd_remap(blockIdx.x, gridDim.x);  // head-major
-  const int per_head = 2 * a.B * nblk;
-  const int hh = work / per_head, r = work - hh * per_head;
+  const int per_head = 2 * a.B * nblk * ns;
+  const int hh = work / per_head;
+  int r = work - hh * per_head;
+  const int piece = split_piece(ns, &r);
   const int item = int(order[r >> 1]);  // the plan's longest-first order, both members together
   const int b = item / nblk;
-  return Item{hh, b, item - b * nblk, r & 1};
+  return Item{hh, b, item - b * nblk, r & 1, piece};
 }
 
 // index of the first entry at or after e whose class is not EMPTY for member
@@ -257,7 +259,7 @@ template <int WD>
 __global__ __launch_bounds__(256, Geo<WD>::WAVES) void k_fwd_f32w(AttnArgs a, const uint32_t* __restrict__ codes,
                                                      const uint32_t* __restrict__ list,
                                                      const int32_t* __restrict__ count, int nT, int nblk,
-                                                     const uint32_t* __restrict__ order) {
+                                                     const uint32_t* __restrict__ order, SplitArgs sp) {
   using G = Geo<WD>;
   constexpr int NR = G::NR, NDB = G::NDB;
   const uint32_t dbytes = uint32_t(a.D) * 4u;  // a row of a.D <= WD floats (16 on the WD = 32 kernels)
@@ -266,7 +268,7 @@ __global__ __launch_bounds__(256, Geo<WD>::WAVES) void k_fwd_f32w(AttnArgs a, co
   __shared__ __attribute__((aligned(256))) uint32_t s_kc[2][64];
   const int tid = threadIdx.x, lane = tid & 63, i = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const Item it = item_of(a, nblk, order);
+  const Item it = item_of(a, nblk, order, sp.ns);
   const int T = a.T, bh = it.b * a.H + it.hh;
   const int q = it.blk * 128 + it.member * 64 + wave * 16 + i;  // this lane's query
   const bool qvalid = q < T;
@@ -284,8 +286,9 @@ __global__ __launch_bounds__(256, Geo<WD>::WAVES) void k_fwd_f32w(AttnArgs a, co
   load_row16<WD>(qg, a.q_strides[2], q, qvalid, g, cs, qr, a.D);
 
   const int lb = it.b * nblk + it.blk;
-  const int n = count[lb];
+  int n = count[lb];
   const uint32_t* ent = list + int64_t(lb) * nT;
+  split_list(sp.ns, it.piece, &ent, &n);
   // chunk (entry e, half hf): keys 64 tile + 32 hf .. + 31
   auto copy = [&](int e, int hf, int slot) {
     const uint32_t r0 = entry_tile(ent[e]) * 64u + uint32_t(32 * hf);
@@ -350,6 +353,12 @@ __global__ __launch_bounds__(256, Geo<WD>::WAVES) void k_fwd_f32w(AttnArgs a, co
     slot ^= 1;
   }
   if (!qvalid) return;
+  if (sp.ns > 1) {  // a piece of the list: O as it stands, the maximum and the sum (kd_combine.hip)
+    const int64_t at = (int64_t(it.piece) * a.B * a.H + bh) * T + q;
+    store16<WD>(sp.part + at * a.D, o, g, 1.f, a.D);
+    if (g == 0) *reinterpret_cast<f32x2*>(sp.part + int64_t(sp.ns) * a.B * a.H * T * a.D + 2 * at) = f32x2{m, l};
+    return;
+  }
   const float inv = l > 0.f ? 1.f / l : 0.f;
   store16<WD>(static_cast<float*>(a.o) + it.b * a.o_strides[0] + it.hh * a.o_strides[1] + int64_t(q) * a.o_strides[2], o,
           g, inv, a.D);
@@ -361,7 +370,7 @@ template <int WD>
 __global__ __launch_bounds__(256, Geo<WD>::WAVES) void k_dq_f32w(AttnArgs a, const uint32_t* __restrict__ codes,
                                                     const uint32_t* __restrict__ list,
                                                     const int32_t* __restrict__ count, int nT, int nblk,
-                                                    const uint32_t* __restrict__ order) {
+                                                    const uint32_t* __restrict__ order, SplitArgs sp) {
   using G = Geo<WD>;
   constexpr int NR = G::NR, NDB = G::NDB;
   const uint32_t dbytes = uint32_t(a.D) * 4u;  // a row of a.D <= WD floats (16 on the WD = 32 kernels)
@@ -370,7 +379,7 @@ __global__ __launch_bounds__(256, Geo<WD>::WAVES) void k_dq_f32w(AttnArgs a, con
   __shared__ __attribute__((aligned(256))) uint32_t s_kc[2][64];
   const int tid = threadIdx.x, lane = tid & 63, i = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const Item it = item_of(a, nblk, order);
+  const Item it = item_of(a, nblk, order, sp.ns);
   const int T = a.T, bh = it.b * a.H + it.hh;
   const int q = it.blk * 128 + it.member * 64 + wave * 16 + i;
   const bool qvalid = q < T;
@@ -394,8 +403,9 @@ __global__ __launch_bounds__(256, Geo<WD>::WAVES) void k_dq_f32w(AttnArgs a, con
   load_row16<WD>(dog, a.do_strides[2], q, qvalid, g, 1.f, dr, a.D);
 
   const int lb = it.b * nblk + it.blk;
-  const int n = count[lb];
+  int n = count[lb];
   const uint32_t* ent = list + int64_t(lb) * nT;
+  split_list(sp.ns, it.piece, &ent, &n);
   auto copy = [&](int e, int hf, int slot) {
     const uint32_t r0 = entry_tile(ent[e]) * 64u + uint32_t(32 * hf);
     copy_chunk<WD>(rs_k, r0, krb, lds_addr(s_k[slot]), wave, lane, dbytes);
@@ -452,6 +462,10 @@ __global__ __launch_bounds__(256, Geo<WD>::WAVES) void k_dq_f32w(AttnArgs a, con
     slot ^= 1;
   }
   if (!qvalid) return;
+  if (sp.ns > 1) {  // a piece of the list: the sum as it stands (kd_combine.hip)
+    store16<WD>(sp.part + ((int64_t(it.piece) * a.B * a.H + bh) * T + q) * a.D, dq, g, 1.f, a.D);
+    return;
+  }
   store16<WD>(static_cast<float*>(a.dq) + it.b * a.dq_strides[0] + it.hh * a.dq_strides[1] + int64_t(q) * a.dq_strides[2],
           dq, g, a.sm_scale, a.D);
 }
@@ -461,7 +475,7 @@ template <int WD>
 __global__ __launch_bounds__(256, Geo<WD>::WAVES) void k_dkdv_f32w(AttnArgs a, const uint32_t* __restrict__ codes,
                                                       const uint32_t* __restrict__ list,
                                                       const int32_t* __restrict__ count, int nT, int nblk,
-                                                      const uint32_t* __restrict__ order) {
+                                                      const uint32_t* __restrict__ order, SplitArgs sp) {
   using G = Geo<WD>;
   constexpr int NR = G::NR, NDB = G::NDB;
   const uint32_t dbytes = uint32_t(a.D) * 4u;  // a row of a.D <= WD floats (16 on the WD = 32 kernels)
@@ -472,7 +486,7 @@ __global__ __launch_bounds__(256, Geo<WD>::WAVES) void k_dkdv_f32w(AttnArgs a, c
   __shared__ __attribute__((aligned(256))) uint32_t s_qc[2][64];
   const int tid = threadIdx.x, lane = tid & 63, i = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const Item it = item_of(a, nblk, order);
+  const Item it = item_of(a, nblk, order, sp.ns);
   const int T = a.T, bh = it.b * a.H + it.hh;
   const int k = it.blk * 128 + it.member * 64 + wave * 16 + i;  // this lane's key
   const bool kvalid = k < T;
@@ -494,8 +508,9 @@ __global__ __launch_bounds__(256, Geo<WD>::WAVES) void k_dkdv_f32w(AttnArgs a, c
   load_row16<WD>(vg, a.v_strides[2], k, kvalid, g, 1.f, vr, a.D);
 
   const int lb = it.b * nblk + it.blk;
-  const int n = count[lb];
+  int n = count[lb];
   const uint32_t* ent = list + int64_t(lb) * nT;
+  split_list(sp.ns, it.piece, &ent, &n);
   // chunk (entry e, half hf): queries 64 tile + 32 hf .. + 31, with their
   // codes, LSE and -Delta (64 values copied, the first 32 used)
   auto copy = [&](int e, int hf, int slot) {
@@ -564,6 +579,12 @@ __global__ __launch_bounds__(256, Geo<WD>::WAVES) void k_dkdv_f32w(AttnArgs a, c
     slot ^= 1;
   }
   if (!kvalid) return;
+  if (sp.ns > 1) {  // a piece of the list: the sums as they stand, dV's then dK's (kd_combine.hip)
+    const int64_t at = (int64_t(it.piece) * a.B * a.H + bh) * T + k;
+    store16<WD>(sp.part + at * a.D, dv, g, 1.f, a.D);
+    store16<WD>(sp.part + (int64_t(sp.ns) * a.B * a.H * T + at) * a.D, dk, g, 1.f, a.D);
+    return;
+  }
   store16<WD>(static_cast<float*>(a.dk) + it.b * a.dk_strides[0] + it.hh * a.dk_strides[1] + int64_t(k) * a.dk_strides[2],
           dk, g, a.sm_scale, a.D);
   store16<WD>(static_cast<float*>(a.dv) + it.b * a.dv_strides[0] + it.hh * a.dv_strides[1] + int64_t(k) * a.dv_strides[2],
@@ -571,32 +592,32 @@ __global__ __launch_bounds__(256, Geo<WD>::WAVES) void k_dkdv_f32w(AttnArgs a, c
 }
 
 template <int WD>
-void launch_f32w_d(int which, const AttnArgs& a, const uint8_t* plan, hipStream_t st) {
+void launch_f32w_d(int which, const AttnArgs& a, const uint8_t* plan, const SplitArgs& sp, hipStream_t st) {
   const PlanLayout L = plan_layout(a.B, a.T, a.D);
   const uint32_t* codes = reinterpret_cast<const uint32_t*>(plan + L.codes);
   auto lst = [&](size_t off) { return reinterpret_cast<const uint32_t*>(plan + off); };
   auto cnt = [&](size_t off) { return reinterpret_cast<const int32_t*>(plan + off); };
-  const unsigned bh2 = 2u * unsigned(a.B) * unsigned(a.H);  // two member workgroups per block
+  const unsigned bh2 = 2u * unsigned(a.B) * unsigned(a.H) * sp.ns;  // two member workgroups per block (and piece)
   if (which == 0)
     hipLaunchKernelGGL(k_fwd_f32w<WD>, dim3(bh2 * unsigned(L.n_fwd_blocks)), dim3(256), 0, st, a, codes,
-                       lst(L.fwd_list), cnt(L.fwd_count), L.nT, L.n_fwd_blocks, lst(L.fwd_order));
+                       lst(L.fwd_list), cnt(L.fwd_count), L.nT, L.n_fwd_blocks, lst(L.fwd_order), sp);
   else if (which == 2)
     hipLaunchKernelGGL(k_dq_f32w<WD>, dim3(bh2 * unsigned(L.n_dq_blocks)), dim3(256), 0, st, a, codes,
-                       lst(L.dq_list), cnt(L.dq_count), L.nT, L.n_dq_blocks, lst(L.dq_order));
+                       lst(L.dq_list), cnt(L.dq_count), L.nT, L.n_dq_blocks, lst(L.dq_order), sp);
   else
     hipLaunchKernelGGL(k_dkdv_f32w<WD>, dim3(bh2 * unsigned(L.n_dkdv_blocks)), dim3(256), 0, st, a, codes,
-                       lst(L.dkdv_list), cnt(L.dkdv_count), L.nT, L.n_dkdv_blocks, lst(L.dkdv_order));
+                       lst(L.dkdv_list), cnt(L.dkdv_count), L.nT, L.n_dkdv_blocks, lst(L.dkdv_order), sp);
 }
 
 }  // namespace
 
-int launch_f32mma(int which, const AttnArgs& a, const uint8_t* plan, hipStream_t st) {
+int launch_f32mma(int which, const AttnArgs& a, const uint8_t* plan, const SplitArgs& sp, hipStream_t st) {
   switch (a.D) {
     case 16:  // on the WD = 32 kernels: columns 16-31 read as zeros, not stored
-    case 32: launch_f32w_d<32>(which, a, plan, st); break;
-    case 64: launch_f32w_d<64>(which, a, plan, st); break;
-    case 128: launch_f32w_d<128>(which, a, plan, st); break;
-    default: launch_f32w_d<256>(which, a, plan, st); break;
+    case 32: launch_f32w_d<32>(which, a, plan, sp, st); break;
+    case 64: launch_f32w_d<64>(which, a, plan, sp, st); break;
+    case 128: launch_f32w_d<128>(which, a, plan, sp, st); break;
+    default: launch_f32w_d<256>(which, a, plan, sp, st); break;
   }
   return hipGetLastError() == hipSuccess ? KD_OK : KD_ERR_LAUNCH;
 }

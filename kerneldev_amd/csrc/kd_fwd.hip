@@ -54,7 +54,8 @@ template <class E, int D, bool Q8, int NSP>
 __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void k_fwd(AttnArgs a, const uint32_t* __restrict__ codes,
                                                              const uint32_t* __restrict__ list,
                                                              const int32_t* __restrict__ count,
-                                                             const uint32_t* __restrict__ order, int nT, int nQB) {
+                                                             const uint32_t* __restrict__ order, int nT, int nQB,
+                                                             SplitArgs sp) {
   constexpr bool SP = NSP >= 2, S3 = NSP == 3;
   constexpr int NW = 4;             // waves per 128-row q-block; each owns 32 rows
   using TL = Tile<D, NW>;           // V tiles (and K tiles on the 16-bit path)
@@ -74,7 +75,8 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void k_fwd(AttnArgs a, const
             c = lane & 31;
   const int T = a.T, H = a.H;
   int h, rank;  // (fwd_work: per XCD, the plan's longest-first order)
-  fwd_work(blockIdx.x, gridDim.x, a.B * nQB, &h, &rank);
+  fwd_work(blockIdx.x, gridDim.x, a.B * nQB * sp.ns, &h, &rank);
+  const int piece = split_piece(sp.ns, &rank);
   const int item = int(order[rank]);
   const int b = item / nQB, qblock = item - b * nQB, bh = b * H + h;
 
@@ -112,8 +114,9 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void k_fwd(AttnArgs a, const
   uint32_t qcode = qvalid ? codes[int64_t(b) * T + qrow] : 0u;
 
   const int lbase = item;  // b nQB + qblock
-  const int n = count[lbase];
+  int n = count[lbase];
   const uint32_t* ent = list + int64_t(lbase) * nT;
+  split_list(sp.ns, piece, &ent, &n);
 
   uint32_t koff[NLK], voff[NL];
   TK::load_offsets(wave, lane, krb, koff, Q8 ? uint32_t(TK::ROWB) : dbytes);
@@ -317,7 +320,15 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void k_fwd(AttnArgs a, const
   {
     const float l_tot = xhalf_sum(l0 + l1);
     const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-    if (qvalid) {
+    if (sp.ns > 1) {  // a piece of the row's list: O as it stands, the maximum and the sum (kd_combine.hip)
+      if (qvalid) {
+        const int64_t at = (int64_t(piece) * a.B * H + bh) * T + qrow;
+        store_part<D>(sp.part + at * a.D, o, hf, a.D);
+        if (hf == 0)
+          *reinterpret_cast<f32x2*>(sp.part + int64_t(sp.ns) * a.B * H * T * a.D + 2 * at) =
+              f32x2{m_ref == NEG_INF ? NEG_INF : m_ref * sl2, l_tot};
+      }
+    } else if (qvalid) {
       const int row = qrow;
       uint16_t* og = static_cast<uint16_t*>(a.o) + b * a.o_strides[0] + h * a.o_strides[1] + row * a.o_strides[2];
       // optional rounding residual O - bf16(O), so the backward's Delta can be
@@ -355,44 +366,49 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void k_fwd(AttnArgs a, const
 }
 
 template <class E, int D, bool Q8, int NSP>
-static void launch_fwd_t(const AttnArgs& a, const uint8_t* plan, hipStream_t st) {
+static void launch_fwd_t(const AttnArgs& a, const uint8_t* plan, const SplitArgs& sp, hipStream_t st) {
   const PlanLayout L = plan_layout(a.B, a.T, a.D);
   const int nQB = L.n_fwd_blocks;
-  const unsigned grid = unsigned(a.B) * a.H * nQB;
+  const unsigned grid = unsigned(a.B) * a.H * nQB * sp.ns;
   hipLaunchKernelGGL((k_fwd<E, D, Q8, NSP>), dim3(grid), dim3(256), 0, st, a,
                      reinterpret_cast<const uint32_t*>(plan + L.codes),
                      reinterpret_cast<const uint32_t*>(plan + L.fwd_list),
                      reinterpret_cast<const int32_t*>(plan + L.fwd_count),
-                     reinterpret_cast<const uint32_t*>(plan + L.fwd_order), L.nT, nQB);
+                     reinterpret_cast<const uint32_t*>(plan + L.fwd_order), L.nT, nQB, sp);
 }
 
 template <class E, int D, bool Q8 = false>
-static void launch_fwd_p(const AttnArgs& a, const uint8_t* plan, hipStream_t st) {
+static void launch_fwd_p(const AttnArgs& a, const uint8_t* plan, const SplitArgs& sp, hipStream_t st) {
   switch (parts_of(a.precision)) {
-    case 1: launch_fwd_t<E, D, Q8, 1>(a, plan, st); break;
-    case 2: launch_fwd_t<E, D, Q8, 2>(a, plan, st); break;
+    case 1: launch_fwd_t<E, D, Q8, 1>(a, plan, sp, st); break;
+    case 2: launch_fwd_t<E, D, Q8, 2>(a, plan, sp, st); break;
     default:
-      if constexpr (!Q8) launch_fwd_t<E, D, Q8, 3>(a, plan, st);  // (the C ABI refuses it with fp8 scores)
+      if constexpr (!Q8) launch_fwd_t<E, D, Q8, 3>(a, plan, sp, st);  // (the C ABI refuses it with fp8 scores)
       break;
   }
 }
 
-int launch_fwd(const AttnArgs& a, const uint8_t* plan, hipStream_t st) {
-  if (use_simt(a)) return launch_simt_kernel(0, a, plan, st);
-  if (a.q8 != nullptr) {  // fp8 QK^T: bf16 at head dim 64, 128 or 256 (checked by the C ABI)
-    if (a.D == 64) launch_fwd_p<BF16, 64, true>(a, plan, st);
-    else if (a.D == 128) launch_fwd_p<BF16, 128, true>(a, plan, st);
-    else launch_fwd_p<BF16, 256, true>(a, plan, st);
-  } else if (a.dtype == KD_BF16) {  // head dims 16 and 32 on the D = 64 kernel
-    if (a.D <= 64) launch_fwd_p<BF16, 64>(a, plan, st);
-    else if (a.D == 128) launch_fwd_p<BF16, 128>(a, plan, st);
-    else launch_fwd_p<BF16, 256>(a, plan, st);
-  } else {
-    if (a.D <= 64) launch_fwd_p<F16, 64>(a, plan, st);
-    else if (a.D == 128) launch_fwd_p<F16, 128>(a, plan, st);
-    else launch_fwd_p<F16, 256>(a, plan, st);
+int launch_fwd(const AttnArgs& a, const uint8_t* plan, float* ws, hipStream_t st) {
+  const SplitArgs sp{ws, ws == nullptr ? 1 : split_pieces(a, SPLIT_FWD)};
+  if (use_simt(a)) {
+    const int r = launch_simt_kernel(0, a, plan, sp, st);
+    return r || sp.ns == 1 ? r : launch_combine_fwd(a, sp, st);
   }
-  return hipGetLastError() == hipSuccess ? KD_OK : KD_ERR_LAUNCH;
+  if (a.q8 != nullptr) {  // fp8 QK^T: bf16 at head dim 64, 128 or 256 (checked by the C ABI)
+    if (a.D == 64) launch_fwd_p<BF16, 64, true>(a, plan, sp, st);
+    else if (a.D == 128) launch_fwd_p<BF16, 128, true>(a, plan, sp, st);
+    else launch_fwd_p<BF16, 256, true>(a, plan, sp, st);
+  } else if (a.dtype == KD_BF16) {  // head dims 16 and 32 on the D = 64 kernel
+    if (a.D <= 64) launch_fwd_p<BF16, 64>(a, plan, sp, st);
+    else if (a.D == 128) launch_fwd_p<BF16, 128>(a, plan, sp, st);
+    else launch_fwd_p<BF16, 256>(a, plan, sp, st);
+  } else {
+    if (a.D <= 64) launch_fwd_p<F16, 64>(a, plan, sp, st);
+    else if (a.D == 128) launch_fwd_p<F16, 128>(a, plan, sp, st);
+    else launch_fwd_p<F16, 256>(a, plan, sp, st);
+  }
+  if (hipGetLastError() != hipSuccess) return KD_ERR_LAUNCH;
+  return sp.ns == 1 ? KD_OK : launch_combine_fwd(a, sp, st);
 }
 
 }  // namespace kd

@@ -39,18 +39,37 @@ struct PlanLayout {
   int nT, fwd_group, dq_group, dkdv_group, n_fwd_blocks, n_dq_blocks, n_dkdv_blocks;
 };
 
+// How a launch cuts its blocks' work lists: into ns pieces, one workgroup
+// each, whose partial results go to `part` and are put together by
+// kd_combine.hip (ns == 1: no pieces, the kernel writes the results itself).
+struct SplitArgs {
+  float* part;
+  int ns;
+};
+enum SplitPass { SPLIT_FWD, SPLIT_DQ, SPLIT_DKDV };
+int split_pieces(const AttnArgs& a, SplitPass pass);
+int64_t split_floats(const AttnArgs& a, SplitPass pass);
+// forward: the pieces' (row maximum in log2 units, row sum), [ns][rows][2], behind their O
+inline float* split_ml(const AttnArgs& a, const SplitArgs& sp) {
+  return sp.part + int64_t(sp.ns) * a.B * a.H * a.T * a.D;
+}
+int launch_combine_fwd(const AttnArgs& a, const SplitArgs& sp, hipStream_t st);
+int launch_combine_dq(const AttnArgs& a, const SplitArgs& sp, hipStream_t st);
+int launch_combine_dkdv(const AttnArgs& a, const SplitArgs& sp, hipStream_t st);
+
 PlanLayout plan_layout(int B, int T, int D);
 int launch_plan(const MetaArgs& m, uint8_t* plan, hipStream_t st);
 int launch_plan_tokens(const kd_token_args& t, uint8_t* plan, hipStream_t st);
 int launch_tile_masks(const uint8_t* plan, int B, int T, int D, uint64_t* rows, uint64_t* cols, hipStream_t st);
 int launch_mask_dense(const uint32_t* codes, int B, int H, int T, uint8_t* out, const int64_t* strides,
                       hipStream_t st);
-int launch_fwd(const AttnArgs& a, const uint8_t* plan, hipStream_t st);
+// ws: NULL (no pieces), or split_floats of the pass
+int launch_fwd(const AttnArgs& a, const uint8_t* plan, float* ws, hipStream_t st);
 int launch_delta(const AttnArgs& a, hipStream_t st);
 // fuse_delta: the dQ kernel also computes Delta and the LSE copy (k_delta's
 // job) for its rows and stores them for the dK/dV kernel
-int launch_dq(const AttnArgs& a, const uint8_t* plan, hipStream_t st, bool fuse_delta);
-int launch_dkdv(const AttnArgs& a, const uint8_t* plan, hipStream_t st);
+int launch_dq(const AttnArgs& a, const uint8_t* plan, float* ws, hipStream_t st, bool fuse_delta);
+int launch_dkdv(const AttnArgs& a, const uint8_t* plan, float* ws, hipStream_t st);
 int launch_hadamard(const kd_rot_args& a, hipStream_t st);
 int launch_quant(const kd_quant_args& a, hipStream_t st);
 int launch_absmax(const kd_quant_args& a, float* amax, hipStream_t st);
@@ -59,10 +78,10 @@ int launch_span_bwd(const kd_span_args& a, hipStream_t st);
 // fp32 inputs (kd_simt.hip): Delta on the vector ALUs and the fp32 MFMA
 // kernels; which: 0 forward, 1 Delta, 2 dQ, 3 dK/dV
 bool use_simt(const AttnArgs& a);
-int launch_simt_kernel(int which, const AttnArgs& a, const uint8_t* plan, hipStream_t st);
+int launch_simt_kernel(int which, const AttnArgs& a, const uint8_t* plan, const SplitArgs& sp, hipStream_t st);
 // fp32 attention at head dims 16 (on the 32 kernels), 32, 64, 128, 256 on the
 // fp32 MFMA (kd_f32w.hip); which: 0 forward, 2 dQ, 3 dK/dV
-int launch_f32mma(int which, const AttnArgs& a, const uint8_t* plan, hipStream_t st);
+int launch_f32mma(int which, const AttnArgs& a, const uint8_t* plan, const SplitArgs& sp, hipStream_t st);
 // Device address of the no-allocation workspace on the current device
 // (kd_noalloc.hip); KD_OK, or a status with *err set.
 int noalloc_workspace(float** out, const char** err);

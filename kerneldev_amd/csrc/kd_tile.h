@@ -145,6 +145,21 @@ struct Tile {
   }
 };
 
+// The piece of a block's list that this workgroup takes (SplitArgs): rank
+// counts pieces of blocks and becomes the block's rank
+KD_DEV int split_piece(int ns, int* rank) {
+  if (ns == 1) return 0;
+  const int r = *rank / ns, piece = *rank - r * ns;
+  *rank = r;
+  return piece;
+}
+KD_DEV void split_list(int ns, int piece, const uint32_t** ent, int* n) {
+  if (ns == 1) return;
+  const int e0 = *n * piece / ns;
+  *n = *n * (piece + 1) / ns - e0;
+  *ent += e0;
+}
+
 // 32 lanes of one half-wave exchange with the other half: returns op(x, x of lane ^ 32).
 KD_DEV float xhalf_max(float x) {
   const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
@@ -303,6 +318,21 @@ struct ScoreOp<E, D, true> {
     for (int st = 0; st < NK; ++st) asm volatile("" : "+v"(b[st]));
   }
 };
+
+// A transposed accumulator's rows as they are, in fp32 (a piece's partial
+// result); dlim: columns from there on are not stored
+template <int D>
+KD_DEV void store_part(float* g, const f32x16 (&acc)[D / 32], int hf, int dlim) {
+#pragma unroll
+  for (int db = 0; db < D / 32; ++db)
+#pragma unroll
+    for (int gg = 0; gg < 4; ++gg) {
+      const int d0 = 32 * db + 8 * gg + 4 * hf;
+      if (d0 < dlim)
+        *reinterpret_cast<f32x4*>(g + d0) =
+            f32x4{acc[db][4 * gg], acc[db][4 * gg + 1], acc[db][4 * gg + 2], acc[db][4 * gg + 3]};
+    }
+}
 
 // Sum of a packed pair of 16-bit floats into an fp32 accumulator (v_dot2).
 template <class E> KD_DEV float acc_pair(uint32_t w, float acc);
