@@ -181,6 +181,31 @@ def load():
     return lib
 
 
+_native = None
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
+
+
+def native():
+    """The C++ eager route (``_kd_torch.so``, csrc/kd_torch.cpp), loaded once; raises if it is not built."""
+    global _native
+    if _native is None:
+        load()
+        from . import _kd_torch  # (an ImportError names the missing file)
+
+        _kd_torch.set_kernel_error(KernelError)
+        _native = _kd_torch
+    return _native
+
+
+def eager(*tensors) -> bool:
+    """Whether the C++ route may take a call on these tensors (None: absent): no
+    compiler is tracing and none is of a subclass.  (The route itself declines,
+    with None, under dispatch modes, transforms and the like.)"""
+    if torch.compiler.is_compiling():
+        return False
+    return all(t is None or type(t) in _PLAIN for t in tensors)
+
+
 def check(status: int, what: str):
     if status != KD_OK:
         msg = load().kd_last_error_string().decode(errors="replace")

@@ -1,10 +1,12 @@
 """``flash_attention()`` -- the drop-in boundary (original_kernel.py:2096-2168).
 
 Keeps the reference's signature, defaults and return forms, and adds three
-optional keyword arguments for the incoherent-processing path.  The work goes
-through two torch custom ops in the ``kdattn`` namespace (the reference uses
-``flash_attention::forward`` / ``::backward``, :1697, :1806), each a thin
-shim over the C ABI of ``libkdattn.so``:
+optional keyword arguments for the incoherent-processing path.  A plain
+eager call goes to the C ABI of ``libkdattn.so`` through one C++ autograd node
+(csrc/kd_torch.cpp); under torch.compile, dispatch or function modes, transforms
+and for tensor subclasses the same work goes through two torch custom ops in the
+``kdattn`` namespace (the reference uses ``flash_attention::forward`` /
+``::backward``, :1697, :1806), each a thin shim over the same C ABI:
 
 * ``kdattn::fwd``  -> plan (codes, tile map, work lists) + forward kernel,
   returns ``(O, LSE2, plan)``; the plan is saved for the backward.
@@ -99,6 +101,10 @@ def _mode(in_span, span_id, is_prefix, has_attention_mask, causal) -> int:
 def build_plan(B, T, D, device, mode, in_span=None, span_id=None, is_prefix=None, lens=None):
     """Run ``kd_plan_build`` and return the plan as a uint8 device tensor."""
     lib = _lib.load()
+    if _lib.eager(in_span, span_id, is_prefix, lens):
+        plan = _lib.native().plan_from_metadata(B, T, D, mode, torch.device(device), lens, in_span, span_id, is_prefix)
+        if plan is not None:
+            return plan
     # zero-filled: the build leaves the bit masks of non-PARTIAL tiles and the
     # section padding unwritten, and an op's outputs should not carry stale bytes
     plan = torch.zeros(_lib.plan_bytes(B, T, D), dtype=torch.uint8, device=device)
@@ -151,6 +157,10 @@ def build_plan_from_tokens(tokens: torch.Tensor, head_dim: int, rule: str = "col
     if lens is not None and (lens.dtype != torch.int32 or lens.dim() != 1 or lens.shape[0] != tokens.shape[0]):
         raise ValueError("lens must be an int32 tensor of shape [batch]")
     B, T = tokens.shape
+    if _lib.eager(tokens, lens):
+        plan = _lib.native().plan_from_tokens(tokens, head_dim, RULES[rule], lens)
+        if plan is not None:
+            return AttentionPlan(plan, B, T, head_dim)
     plan = torch.zeros(_lib.plan_bytes(B, T, head_dim), dtype=torch.uint8, device=tokens.device)
     t = _lib.TokenArgs()
     t.tokens = tokens.data_ptr()
@@ -641,10 +651,15 @@ def flash_attention(
         # O's rounding residual, kept for the backward's Delta (16-bit O only)
         need_lo = (q.dtype != torch.float32 and torch.is_grad_enabled()
                    and any(x.requires_grad for x in (q, k, v)))
-        o, lse, plan_t, *_ = _fwd_op(q, k, v, lens, in_span, span_id, is_prefix, float(sm_scale), int(mode),
-                                     need_lo, bthd=out_layout == "bthd",
-                                     plan_in=None if plan is None else plan.tensor, signs=fused_signs,
-                                     quant_fp8=qk_dtype == "fp8_e4m3", prec=PRECISIONS[precision])
+        bthd, plan_in, fp8 = out_layout == "bthd", None if plan is None else plan.tensor, qk_dtype == "fp8_e4m3"
+        got = None
+        if _lib.eager(q, k, v, lens, in_span, span_id, is_prefix, plan_in):
+            got = _lib.native().flash(q, k, v, lens, in_span, span_id, is_prefix, float(sm_scale), int(mode), need_lo,
+                                      bthd, plan_in, fused_signs, fp8, PRECISIONS[precision])
+        if got is None:  # traced, under a mode, or a subclass: the custom op, with the same kernels
+            got = _fwd_op(q, k, v, lens, in_span, span_id, is_prefix, float(sm_scale), int(mode), need_lo, bthd=bthd,
+                          plan_in=plan_in, signs=fused_signs, quant_fp8=fp8, prec=PRECISIONS[precision])
+        o, lse, plan_t, *_ = got
     if plan is not None:
         plan_t = plan.tensor
     if in_dtype == torch.float32:

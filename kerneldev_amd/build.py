@@ -66,6 +66,31 @@ def build_library(verbose: bool = False) -> str:
     return LIB
 
 
+NATIVE_SRC = os.path.join(CSRC, "kd_torch.cpp")
+NATIVE = os.path.join(PKG, "_kd_torch.so")
+
+
+def build_native(verbose: bool = False) -> str:
+    """The C++ eager route from torch to libkdattn.so (host code only), linked
+    against torch's own libraries and, through its rpath, the library beside it."""
+    import sysconfig
+
+    from torch.utils import cpp_extension
+
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    inc = [f"-I{p}" for p in (*cpp_extension.include_paths(), f"{rocm}/include", sysconfig.get_paths()["include"])]
+    libdirs = [f"-L{p}" for p in cpp_extension.library_paths()]
+    tmp = NATIVE + ".tmp"
+    _run(["g++", "-std=c++17", "-O2", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+          "-DTORCH_API_INCLUDE_EXTENSION_H", "-DTORCH_EXTENSION_NAME=_kd_torch", *inc, NATIVE_SRC, "-o", tmp,
+          f"-L{PKG}", "-lkdattn", *libdirs, "-lc10", "-lc10_hip", "-ltorch", "-ltorch_cpu", "-ltorch_python",
+          "-Wl,-rpath,$ORIGIN"])
+    os.replace(tmp, NATIVE)
+    if verbose:
+        print(f"built {NATIVE}")
+    return NATIVE
+
+
 C_ABI_SRC = os.path.join(ROOT, "tests", "c_abi", "attn_from_c.c")
 C_ABI_BIN = os.path.join(ROOT, "tests", "c_abi", "attn_from_c")
 
@@ -84,5 +109,6 @@ def build_c_abi_check(verbose: bool = False) -> str:
 
 if __name__ == "__main__":
     build_library(verbose=True)
+    build_native(verbose=True)
     build_c_abi_check(verbose=True)
     sys.exit(0)

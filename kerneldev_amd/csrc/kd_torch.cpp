@@ -1,0 +1,406 @@
+// The eager route of flash_attention, build_plan, build_plan_from_tokens and
+// span_scores from torch to the C ABI of libkdattn.so, in C++.
+//
+// The Python custom ops (attention.py, span_head.py) stay the ones that
+// torch.compile, torch.export, dispatch and function modes, functorch
+// transforms, tracing and forward-mode AD see.  For a plain eager call their
+// Python dispatch, schema and autograd layers take most of the time of a small
+// step: 309 us a forward and backward at fp32 B2 H4 T256 d64, whose kernels
+// run for 78 us.  The same work here -- the same checks, allocations, kernels
+// and saved tensors, under a C++ autograd::Function -- takes 104 us (fp16 B4
+// H8 T777 d32: 322 -> 88; span_scores of B8 T2048 D768: 226 -> 96).  Every entry returns None where the call is not plain (see
+// plain()), and the caller then goes through the custom op.
+#include <ATen/ATen.h>
+#include <ATen/record_function.h>
+#include <ATen/PythonTorchFunctionTLS.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/forward_grad.h>
+#include <torch/csrc/autograd/functions/basic_ops.h>
+#include <torch/csrc/autograd/functions/utils.h>
+#include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
+#include <torch/csrc/utils/pybind.h>
+
+#include "../../include/kdattn.h"
+
+namespace {
+
+using at::Tensor;
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
+using OptTensor = std::optional<Tensor>;
+
+PyObject* g_kernel_error = nullptr;  // _lib.KernelError
+
+// A status as the Python layer raises it (_lib.check): ValueError for refused
+// arguments, KernelError for the rest
+void check(int status, const char* what) {
+  if (status == KD_OK) return;
+  pybind11::gil_scoped_acquire gil;
+  std::string msg = std::string(what) + ": " + kd_last_error_string();
+  const bool refused = status == KD_ERR_INVALID || status == KD_ERR_UNSUPPORTED;
+  if (!refused) msg += " (status " + std::to_string(status) + ")";
+  PyErr_SetString(refused ? PyExc_ValueError : g_kernel_error, msg.c_str());
+  python_error e;
+  e.persist();
+  throw e;
+}
+
+void* stream_on(c10::Device d) { return c10::hip::getCurrentHIPStream(d.index()).stream(); }
+void* stream_of(const Tensor& t) { return stream_on(t.device()); }
+
+// Plain eager tensors: strided GPU tensors with nothing between them and their
+// memory (no subclass or mode dispatch, transform, lazy negation or zero, no
+// tangent).
+bool plain(const Tensor& t) {
+  using K = c10::DispatchKey;
+  static const c10::DispatchKeySet other({K::Python, K::PythonTLSSnapshot, K::Negative, K::Conjugate, K::ZeroTensor,
+                                          K::FuncTorchBatched, K::FuncTorchGradWrapper, K::Functionalize});
+  return t.defined() && t.is_cuda() && t.layout() == at::kStrided && !t.is_nested() &&
+         (t.key_set() & other).empty() && !t._fw_grad(0).defined();
+}
+bool plain(const OptTensor& t) { return !t.has_value() || plain(*t); }
+bool plain_mode() {
+  using K = c10::DispatchKey;
+  return !c10::impl::TorchDispatchModeTLS::any_modes_set() && at::impl::PythonTorchFunctionTLS::stack_len() == 0 &&
+         !c10::impl::tls_is_dispatch_key_included(K::FuncTorchDynamicLayerFrontMode) &&
+         !c10::impl::tls_is_dispatch_key_included(K::Functionalize) && !torch::jit::tracer::isTracing();
+}
+
+// Unit d-stride, 16-byte aligned base, 8-element-multiple strides, rows that
+// do not overlap (attention._kernel_ready)
+Tensor kernel_ready(const Tensor& x) {
+  const auto s = x.strides();
+  const bool ok = s[3] == 1 && reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 && s[0] % 8 == 0 && s[1] % 8 == 0 &&
+                  s[2] % 8 == 0 && s[2] >= x.size(3) && x.size(2) * s[2] * x.element_size() < (int64_t(1) << 31);
+  return ok ? x : x.contiguous();
+}
+
+int dtype_code(at::ScalarType t) {
+  if (t == at::kBFloat16) return KD_BF16;
+  if (t == at::kHalf) return KD_F16;
+  TORCH_CHECK_VALUE(t == at::kFloat, "kernel dtype must be bf16, fp16 or fp32");
+  return KD_F32;
+}
+
+void set3(int64_t (&to)[3], const Tensor& t) {
+  for (int i = 0; i < 3; ++i) to[i] = t.stride(i);
+}
+
+int64_t plan_size(int64_t B, int64_t T, int64_t D) {
+  const int64_t n = kd_plan_bytes(int32_t(B), int32_t(T), int32_t(D));
+  TORCH_CHECK_VALUE(n >= 0, "invalid plan shape");
+  return n;
+}
+
+Tensor bytes_on(c10::Device device, int64_t n, bool zero) {
+  const auto o = at::TensorOptions().dtype(at::kByte).device(device);
+  return zero ? at::zeros({n}, o) : at::empty({n}, o);
+}
+
+struct Meta {
+  OptTensor lens, in_span, span_id, is_prefix;
+};
+
+Tensor plan_of(int64_t B, int64_t T, int64_t D, c10::Device on, int64_t mode, const Meta& x) {
+  Tensor plan = bytes_on(on, plan_size(B, T, D), true);
+  kd_meta_args m{};
+  m.B = int32_t(B), m.T = int32_t(T), m.D = int32_t(D), m.mode = int32_t(mode);
+  auto two = [](int64_t (&to)[2], const Tensor& t) { to[0] = t.stride(0), to[1] = t.stride(1); };
+  if (x.in_span) m.in_span = static_cast<const uint8_t*>(x.in_span->data_ptr()), two(m.in_span_strides, *x.in_span);
+  if (x.is_prefix)
+    m.is_prefix = static_cast<const uint8_t*>(x.is_prefix->data_ptr()), two(m.is_prefix_strides, *x.is_prefix);
+  if (x.span_id) {
+    m.span_id = x.span_id->data_ptr();
+    two(m.span_id_strides, *x.span_id);
+    m.span_id_dtype = x.span_id->scalar_type() == at::kLong ? KD_I64 : KD_I32;
+  }
+  if (x.lens) m.lens = static_cast<const int32_t*>(x.lens->data_ptr()), m.lens_stride = x.lens->stride(0);
+  check(kd_plan_build(&m, plan.data_ptr(), plan.numel(), stream_on(on)), "kd_plan_build");
+  return plan;
+}
+
+kd_attn_args attn_args(const Tensor& q, const Tensor& k, const Tensor& v, double sm_scale, int64_t prec) {
+  kd_attn_args a{};
+  a.B = int32_t(q.size(0)), a.H = int32_t(q.size(1)), a.T = int32_t(q.size(2)), a.D = int32_t(q.size(3));
+  a.dtype = dtype_code(q.scalar_type());
+  a.sm_scale = float(sm_scale);
+  a.precision = int32_t(prec);
+  a.q = q.data_ptr(), a.k = k.data_ptr(), a.v = v.data_ptr();
+  set3(a.q_strides, q), set3(a.k_strides, k), set3(a.v_strides, v);
+  return a;
+}
+
+// kd_hadamard of a kernel-ready tensor, with amax [B, H] where given
+Tensor rotate(const Tensor& x, const Tensor& signs, const Tensor& amax) {
+  Tensor y = at::empty(x.sizes(), x.options());
+  kd_rot_args a{};
+  a.x = x.data_ptr(), a.y = y.data_ptr();
+  set3(a.x_strides, x), set3(a.y_strides, y);
+  a.signs = static_cast<const float*>(signs.data_ptr());
+  a.amax = amax.defined() ? static_cast<float*>(amax.data_ptr()) : nullptr;
+  a.B = int32_t(x.size(0)), a.H = int32_t(x.size(1)), a.T = int32_t(x.size(2)), a.D = int32_t(x.size(3));
+  a.dtype = dtype_code(x.scalar_type());
+  check(kd_hadamard(&a, stream_of(x)), "kd_hadamard");
+  return y;
+}
+
+// e4m3 copy and scale of a kernel-ready tensor; amax [B, H] as the rotation
+// left it, or filled here
+std::pair<Tensor, Tensor> quantise(const Tensor& x, const Tensor& amax, bool fill) {
+  Tensor y = at::empty(x.sizes(), x.options().dtype(at::kByte));
+  Tensor scale = at::empty({x.size(0), x.size(1)}, x.options().dtype(at::kFloat));
+  kd_quant_args a{};
+  a.x = x.data_ptr();
+  set3(a.x_strides, x);
+  a.y = static_cast<uint8_t*>(y.data_ptr());
+  a.amax = static_cast<const float*>(amax.data_ptr());
+  a.scale = static_cast<float*>(scale.data_ptr());
+  a.B = int32_t(x.size(0)), a.H = int32_t(x.size(1)), a.T = int32_t(x.size(2)), a.D = int32_t(x.size(3));
+  a.dtype = dtype_code(x.scalar_type());
+  if (fill) check(kd_absmax(&a, static_cast<float*>(amax.data_ptr()), stream_of(x)), "kd_absmax");
+  check(kd_quant_fp8(&a, stream_of(x)), "kd_quant_fp8");
+  return {y, scale};
+}
+
+void set_fp8(kd_attn_args& a, const Tensor& q8, const Tensor& k8, const Tensor& qs, const Tensor& ks) {
+  a.q8 = static_cast<const uint8_t*>(q8.data_ptr()), a.k8 = static_cast<const uint8_t*>(k8.data_ptr());
+  a.q_scale = static_cast<const float*>(qs.data_ptr()), a.k_scale = static_cast<const float*>(ks.data_ptr());
+}
+
+// Gradients made under create_graph depend on `from` through an op without a
+// derivative: going back through them raises, as the custom op does
+void refuse_second(variable_list& grads, const char* op, const variable_list& from) {
+  const auto node = std::make_shared<torch::autograd::Error>(
+      std::string("Trying to backward through ") + op + " but no autograd formula was registered.",
+      torch::autograd::collect_next_edges(from));
+  for (Tensor& g : grads) torch::autograd::set_history(g, node);
+}
+
+struct AttnOpts {
+  Meta meta;
+  OptTensor plan, signs;
+  double sm_scale;
+  int64_t mode, prec;
+  bool need_lo, bthd, fp8;
+  Tensor* built;  // the plan used, for the caller
+};
+
+// kdattn::fwd and kdattn::bwd (attention.py) as one C++ node
+struct Attention : torch::autograd::Function<Attention> {
+  static variable_list forward(AutogradContext* ctx, const Tensor& q_in, const Tensor& k_in, const Tensor& v_in,
+                               const AttnOpts& x) {
+    RECORD_FUNCTION("kdattn::fwd", std::vector<c10::IValue>());
+    const c10::DeviceGuard on(q_in.device());
+    const int64_t B = q_in.size(0), H = q_in.size(1), T = q_in.size(2), D = q_in.size(3);
+    Tensor q = kernel_ready(q_in), k = kernel_ready(k_in), v = kernel_ready(v_in);
+    const Tensor plan = x.plan ? *x.plan : plan_of(B, T, D, q.device(), x.mode, x.meta);
+    *x.built = plan;
+    const auto f32 = q.options().dtype(at::kFloat);
+    Tensor amax[2], q8, k8, qs, ks;
+    if (x.fp8) {  // (the rotation folds its absmax into amax with atomics: zeroed first)
+      const Tensor both = x.signs ? at::zeros({2, B, H}, f32) : at::empty({2, B, H}, f32);
+      amax[0] = both[0], amax[1] = both[1];
+    }
+    if (x.signs) q = rotate(q, *x.signs, amax[0]), k = rotate(k, *x.signs, amax[1]);
+    if (x.fp8) std::tie(q8, qs) = quantise(q, amax[0], !x.signs), std::tie(k8, ks) = quantise(k, amax[1], !x.signs);
+    Tensor o = x.bthd ? at::empty_strided({B, H, T, D}, {T * H * D, D, H * D, 1}, q.options())
+                      : at::empty({B, H, T, D}, q.options());
+    Tensor lse = at::empty({B, H, T}, f32), o_lo;
+    if (x.need_lo) o_lo = at::empty({B, H, T, D}, x.prec == KD_PREC_SPLIT3 ? f32 : q.options());
+    kd_attn_args a = attn_args(q, k, v, x.sm_scale, x.prec);
+    if (x.fp8) set_fp8(a, q8, k8, qs, ks);
+    a.o = o.data_ptr();
+    set3(a.o_strides, o);
+    a.lse = static_cast<float*>(lse.data_ptr());
+    a.o_lo = x.need_lo ? o_lo.data_ptr() : nullptr;
+    const int64_t need = kd_attn_fwd_ws_bytes(&a);
+    Tensor ws = need > 0 ? bytes_on(q.device(), need, false) : Tensor();
+    check(kd_attn_fwd_ws(&a, plan.data_ptr(), plan.numel(), need > 0 ? ws.data_ptr() : nullptr, need, stream_of(q)),
+          "kd_attn_fwd");
+    // with a rotation the backward recomputes from the rotated operands
+    variable_list keep{x.signs ? q : q_in, x.signs ? k : k_in, v_in, o, lse, plan, o_lo};
+    if (x.signs) keep.push_back(*x.signs);
+    if (x.fp8) keep.insert(keep.end(), {q8, k8, qs, ks});
+    ctx->save_for_backward(std::move(keep));
+    ctx->set_materialize_grads(false);  // LSE's gradient is ignored: no zeros made for it
+    ctx->saved_data["sm_scale"] = x.sm_scale;
+    ctx->saved_data["prec"] = x.prec;
+    ctx->saved_data["rot"] = x.signs.has_value();
+    ctx->saved_data["fp8"] = x.fp8;
+    return {o, lse};
+  }
+
+  static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
+    variable_list out(4);
+    if (!grads[0].defined()) return out;  // O did not reach the loss
+    RECORD_FUNCTION("kdattn::bwd", std::vector<c10::IValue>());
+    const variable_list s = ctx->get_saved_variables();
+    const bool rot = ctx->saved_data["rot"].toBool(), fp8 = ctx->saved_data["fp8"].toBool();
+    bool differentiable = false;  // (create_graph: the op has no second derivative, which its use must report)
+    if (at::GradMode::is_enabled())
+      for (const Tensor& t : {s[0], s[1], s[2], s[3], s[4], grads[0]}) differentiable |= t.requires_grad();
+    variable_list g(3);
+    {
+      at::AutoDispatchBelowADInplaceOrView below;
+      const c10::DeviceGuard on(s[0].device());
+      Tensor d_o = grads[0];
+      if (d_o.is_neg()) d_o = d_o.resolve_neg();
+      if (d_o._is_zerotensor()) d_o = at::zeros(d_o.sizes(), s[3].options());
+      const Tensor q = kernel_ready(s[0]), k = kernel_ready(s[1]), v = kernel_ready(s[2]), o = kernel_ready(s[3]);
+      d_o = kernel_ready(d_o);
+      const Tensor &lse = s[4], &plan = s[5], &o_lo = s[6];
+      const int64_t B = q.size(0), H = q.size(1), T = q.size(2), D = q.size(3);
+      for (Tensor& t : g) t = at::empty({B, H, T, D}, q.options());
+      const Tensor delta = at::empty({2, B, H, T}, q.options().dtype(at::kFloat));
+      kd_attn_args a = attn_args(q, k, v, ctx->saved_data["sm_scale"].toDouble(), ctx->saved_data["prec"].toInt());
+      a.o = o.data_ptr();
+      set3(a.o_strides, o);
+      a.lse = static_cast<float*>(lse.data_ptr());
+      a.dout = d_o.data_ptr();
+      set3(a.do_strides, d_o);
+      a.dq = g[0].data_ptr(), a.dk = g[1].data_ptr(), a.dv = g[2].data_ptr();
+      set3(a.dq_strides, g[0]), set3(a.dk_strides, g[1]), set3(a.dv_strides, g[2]);
+      a.delta = static_cast<float*>(delta.data_ptr());
+      a.o_lo = o_lo.defined() ? o_lo.data_ptr() : nullptr;
+      if (fp8) {
+        const size_t i = rot ? 8 : 7;
+        set_fp8(a, s[i], s[i + 1], s[i + 2], s[i + 3]);
+      }
+      a.dqk_signs = rot ? static_cast<const float*>(s[7].data_ptr()) : nullptr;
+      const int64_t need = kd_attn_bwd_ws_bytes(&a);
+      const Tensor ws = need > 0 ? bytes_on(q.device(), need, false) : Tensor();
+      check(kd_attn_bwd_ws(&a, plan.data_ptr(), plan.numel(), need > 0 ? ws.data_ptr() : nullptr, need, stream_of(q)),
+            "kd_attn_bwd");
+    }
+    if (differentiable) refuse_second(g, "kdattn.bwd.default", {s[0], s[1], s[2], s[3], s[4], grads[0]});
+    for (int i = 0; i < 3; ++i) out[i] = g[i];
+    return out;
+  }
+};
+
+// (o, lse, plan), or None where the call is not a plain eager one
+pybind11::object flash(const Tensor& q, const Tensor& k, const Tensor& v, const OptTensor& lens, const OptTensor& in_span,
+                       const OptTensor& span_id, const OptTensor& is_prefix, double sm_scale, int64_t mode, bool need_lo,
+                       bool bthd, const OptTensor& plan, const OptTensor& signs, bool fp8, int64_t prec) {
+  if (!plain_mode() || !plain(q) || !plain(k) || !plain(v) || !plain(lens) || !plain(in_span) || !plain(span_id) ||
+      !plain(is_prefix) || !plain(plan) || !plain(signs) || q.scalar_type() != k.scalar_type() ||
+      q.scalar_type() != v.scalar_type() || q.numel() == 0)
+    return pybind11::none();
+  Tensor used;
+  const AttnOpts x{{lens, in_span, span_id, is_prefix}, plan, signs, sm_scale, mode, prec, need_lo, bthd, fp8, &used};
+  const variable_list r = Attention::apply(q, k, v, x);
+  return pybind11::make_tuple(r[0], r[1], used);
+}
+
+pybind11::object plan_from_metadata(int64_t B, int64_t T, int64_t D, int64_t mode, c10::Device on, const OptTensor& lens,
+                                    const OptTensor& in_span, const OptTensor& span_id, const OptTensor& is_prefix) {
+  if (!plain_mode() || !on.is_cuda() || !plain(lens) || !plain(in_span) || !plain(span_id) || !plain(is_prefix))
+    return pybind11::none();
+  const c10::DeviceGuard guard(on);
+  return pybind11::cast(plan_of(B, T, D, on, mode, Meta{lens, in_span, span_id, is_prefix}));
+}
+
+pybind11::object plan_from_tokens(const Tensor& tokens, int64_t D, int64_t rule, const OptTensor& lens) {
+  if (!plain_mode() || !plain(tokens) || !plain(lens)) return pybind11::none();
+  const c10::DeviceGuard guard(tokens.device());
+  const int64_t B = tokens.size(0), T = tokens.size(1);
+  Tensor plan = bytes_on(tokens.device(), plan_size(B, T, D), true);
+  kd_token_args t{};
+  t.tokens = tokens.data_ptr();
+  t.tokens_strides[0] = tokens.stride(0), t.tokens_strides[1] = tokens.stride(1);
+  t.tokens_dtype = tokens.scalar_type() == at::kLong ? KD_I64 : KD_I32;
+  t.rule = int32_t(rule);
+  if (lens) t.lens = static_cast<const int32_t*>(lens->data_ptr()), t.lens_stride = lens->stride(0);
+  t.B = int32_t(B), t.T = int32_t(T), t.D = int32_t(D);
+  check(kd_plan_build_tokens(&t, plan.data_ptr(), plan.numel(), stream_of(tokens)), "kd_plan_build_tokens");
+  return pybind11::cast(plan);
+}
+
+// ---------------------------------------------------------------- span head
+kd_span_args span_args(const Tensor& tokens, const Tensor& h, int64_t n) {
+  kd_span_args a{};
+  a.tokens = tokens.data_ptr();
+  a.tokens_strides[0] = tokens.stride(0), a.tokens_strides[1] = tokens.stride(1);
+  a.tokens_dtype = tokens.scalar_type() == at::kLong ? KD_I64 : KD_I32;
+  a.dtype = dtype_code(h.scalar_type());
+  a.h = h.data_ptr();
+  a.h_strides[0] = h.stride(0), a.h_strides[1] = h.stride(1);
+  a.B = int32_t(h.size(0)), a.T = int32_t(h.size(1)), a.D = int32_t(h.size(2));
+  a.n_spans = int32_t(n);
+  return a;
+}
+
+void set_span(kd_span_args& a, const Tensor& h_ctx, const Tensor& h_spans, const Tensor& lo, const Tensor& hi,
+              const Tensor& mpos) {
+  a.h_ctx = static_cast<float*>(h_ctx.data_ptr()), a.h_spans = static_cast<float*>(h_spans.data_ptr());
+  a.span_lo = static_cast<int32_t*>(lo.data_ptr()), a.span_hi = static_cast<int32_t*>(hi.data_ptr());
+  a.mask_pos = static_cast<int32_t*>(mpos.data_ptr());
+}
+
+// kdattn::span_fwd and kdattn::span_bwd (span_head.py) as one C++ node
+struct SpanHead : torch::autograd::Function<SpanHead> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& h_in, const Tensor& tokens, int64_t n) {
+    RECORD_FUNCTION("kdattn::span_fwd", std::vector<c10::IValue>());
+    const c10::DeviceGuard on(h_in.device());
+    const Tensor h = h_in.stride(2) != 1 ? h_in.contiguous() : h_in;
+    const int64_t B = h.size(0), D = h.size(2);
+    const auto f32 = h.options().dtype(at::kFloat), i32 = h.options().dtype(at::kInt);
+    Tensor scores = at::empty({B, n}, f32), h_ctx = at::empty({B, D}, f32), h_spans = at::empty({B, n, D}, f32);
+    Tensor lo = at::empty({B, n}, i32), hi = at::empty({B, n}, i32), mpos = at::empty({B}, i32);
+    kd_span_args a = span_args(tokens, h, n);
+    a.scores = static_cast<float*>(scores.data_ptr());
+    set_span(a, h_ctx, h_spans, lo, hi, mpos);
+    check(kd_span_scores(&a, stream_of(h)), "kd_span_scores");
+    ctx->save_for_backward({tokens, h_in, h_ctx, h_spans, lo, hi, mpos});
+    ctx->set_materialize_grads(false);
+    return scores;
+  }
+  static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
+    variable_list out(3);
+    if (!grads[0].defined()) return out;
+    RECORD_FUNCTION("kdattn::span_bwd", std::vector<c10::IValue>());
+    const variable_list s = ctx->get_saved_variables();
+    const bool differentiable = at::GradMode::is_enabled() && (s[1].requires_grad() || grads[0].requires_grad());
+    variable_list dh(1);
+    {
+      at::AutoDispatchBelowADInplaceOrView below;
+      const Tensor &tokens = s[0], &h = s[1];
+      const c10::DeviceGuard on(h.device());
+      Tensor ds = grads[0];
+      if (ds.is_neg()) ds = ds.resolve_neg();
+      if (ds._is_zerotensor()) ds = at::zeros(ds.sizes(), s[2].options());
+      ds = ds.to(at::kFloat).contiguous();
+      dh[0] = at::empty(h.sizes(), h.options());
+      kd_span_args a = span_args(tokens, h, ds.size(1));
+      set_span(a, s[2], s[3], s[4], s[5], s[6]);
+      a.dscores = static_cast<const float*>(ds.data_ptr());
+      a.dh = dh[0].data_ptr();
+      a.dh_strides[0] = dh[0].stride(0), a.dh_strides[1] = dh[0].stride(1);
+      check(kd_span_scores_bwd(&a, stream_of(h)), "kd_span_scores_bwd");
+    }
+    if (differentiable) refuse_second(dh, "kdattn.span_bwd.default", {s[1], grads[0]});
+    out[0] = dh[0];
+    return out;
+  }
+};
+
+pybind11::object span(const Tensor& tokens, const Tensor& h, int64_t n) {
+  if (!plain_mode() || !plain(tokens) || !plain(h) || h.numel() == 0) return pybind11::none();
+  return pybind11::cast(SpanHead::apply(h, tokens, n));
+}
+
+}  // namespace
+
+PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+  m.def("set_kernel_error", [](pybind11::object e) { g_kernel_error = e.release().ptr(); });
+  m.def("flash", torch::wrap_pybind_function(flash));
+  m.def("plan_from_metadata", torch::wrap_pybind_function(plan_from_metadata));
+  m.def("plan_from_tokens", torch::wrap_pybind_function(plan_from_tokens));
+  m.def("span", torch::wrap_pybind_function(span));
+}

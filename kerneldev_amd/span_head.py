@@ -145,6 +145,10 @@ def span_scores(tokens: torch.Tensor, h: torch.Tensor, n_spans: int | None = Non
     n = max_spans(tokens) if n_spans is None else int(n_spans)
     if n < 1:
         raise ValueError("no [SPAN] token in the batch (the reference returns an empty result there)")
+    if _lib.eager(tokens, h):
+        scores = _lib.native().span(tokens, h, n)
+        if scores is not None:
+            return scores
     return _span_fwd_op(tokens, h, n)[0]
 
 
