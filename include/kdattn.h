@@ -344,6 +344,10 @@ int kd_quant_fp8(const kd_quant_args *a, void *stream);
  * counterpart in the reference, which has no fp8 path. */
 int kd_absmax(const kd_quant_args *a, float *amax, void *stream);
 
+/* [SPAN] tokens of each row: counts [B] int32, from a's tokens, B and T only
+ * (their maximum is the reference's max_spans, model.py:274). */
+int kd_span_count(const kd_span_args *a, int32_t *counts, void *stream);
+
 /* Cocktail-party head forward: span_lo/hi, mask_pos, h_ctx, h_spans and
  * scores.  Replaces the Python double loop and einsum of GPTModel.forward
  * (model.py:263-298). */

@@ -116,6 +116,7 @@ SIGNATURES = {
     "kd_struct_sizes2": (None, [POINTER(c_size_t), POINTER(c_size_t)]),
     "kd_struct_sizes3": (None, [POINTER(c_size_t)]),
     "kd_struct_sizes4": (None, [POINTER(c_size_t)]),
+    "kd_span_count": (c_int, [POINTER(SpanArgs), c_void_p, c_void_p]),
     "kd_span_scores": (c_int, [POINTER(SpanArgs), c_void_p]),
     "kd_span_scores_bwd": (c_int, [POINTER(SpanArgs), c_void_p]),
     "kd_plan_build_tokens": (c_int, [POINTER(TokenArgs), c_void_p, c_int64, c_void_p]),

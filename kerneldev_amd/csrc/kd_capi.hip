@@ -140,6 +140,16 @@ void kd_struct_sizes4(size_t* span) {
   if (span) *span = sizeof(kd_span_args);
 }
 
+int kd_span_count(const kd_span_args* a, int32_t* counts, void* stream) {
+  if (a == nullptr) return fail(KD_ERR_INVALID, "args is NULL");
+  if (a->B < 1 || a->T < 1) return fail(KD_ERR_INVALID, "B and T must be >= 1");
+  if (a->tokens_dtype != KD_I64 && a->tokens_dtype != KD_I32) return fail(KD_ERR_INVALID, "bad tokens dtype");
+  if (a->tokens == nullptr || counts == nullptr) return fail(KD_ERR_INVALID, "tokens and counts are required");
+  if (a->tokens_strides[0] < 0 || a->tokens_strides[1] < 0) return fail(KD_ERR_INVALID, "negative token strides");
+  const int r = kd::launch_span_count(*a, counts, as_stream(stream));
+  return r ? fail(r, "kernel launch failed (span count)") : KD_OK;
+}
+
 int kd_span_scores(const kd_span_args* a, void* stream) {
   int r;
   if ((r = check_span(a))) return r;

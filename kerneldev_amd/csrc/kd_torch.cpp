@@ -395,6 +395,22 @@ pybind11::object span(const Tensor& tokens, const Tensor& h, int64_t n) {
   return pybind11::cast(SpanHead::apply(h, tokens, n));
 }
 
+// [SPAN] tokens of each row of tokens [B, T], int32 [B] on its device
+pybind11::object span_counts(const Tensor& tokens) {
+  if (!plain_mode() || !plain(tokens) || tokens.dim() != 2 || tokens.numel() == 0 ||
+      (tokens.scalar_type() != at::kLong && tokens.scalar_type() != at::kInt))
+    return pybind11::none();
+  const c10::DeviceGuard guard(tokens.device());
+  Tensor counts = at::empty({tokens.size(0)}, tokens.options().dtype(at::kInt));
+  kd_span_args a{};
+  a.tokens = tokens.data_ptr();
+  a.tokens_strides[0] = tokens.stride(0), a.tokens_strides[1] = tokens.stride(1);
+  a.tokens_dtype = tokens.scalar_type() == at::kLong ? KD_I64 : KD_I32;
+  a.B = int32_t(tokens.size(0)), a.T = int32_t(tokens.size(1));
+  check(kd_span_count(&a, static_cast<int32_t*>(counts.data_ptr()), stream_of(tokens)), "kd_span_count");
+  return pybind11::cast(counts);
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -402,5 +418,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("flash", torch::wrap_pybind_function(flash));
   m.def("plan_from_metadata", torch::wrap_pybind_function(plan_from_metadata));
   m.def("plan_from_tokens", torch::wrap_pybind_function(plan_from_tokens));
+  m.def("span_counts", torch::wrap_pybind_function(span_counts));
   m.def("span", torch::wrap_pybind_function(span));
 }

@@ -126,3 +126,23 @@ def test_public_entry_and_errors(dev):
         span_scores(torch.tensor([[MASK, X, X]], device=dev), torch.randn(1, 3, 8, device=dev).bfloat16())
     with pytest.raises(ValueError):
         span_scores(tokens, h.float())
+
+
+@pytest.mark.parametrize("T,D", [(16384, 128), (16385, 128), (1500, 2048), (1500, 2052), (511, 4), (513, 130)])
+def test_routes_of_the_head(dev, T, D):
+    """Both sides of the one-launch route's limits (16384 tokens, 2048 columns), and widths that allow 16-byte,
+    8-byte and no vector accesses."""
+    rows = [[X] * 7 + [MASK] + [X] * (T // 2 - 20) + [SPAN] + [X] * 9 + [ES] + [X] * (T - T // 2 - 1 - 3 - 6 - 4) + [SPAN, X, ES],
+            [SPAN, X, X, ES] + [X] * (T - 6) + [MASK, X]]
+    tokens = torch.tensor([r[:T] + [X] * (T - len(r)) for r in rows], dtype=torch.int64)
+    h = torch.randn(2, T, D, generator=torch.Generator().manual_seed(T + D)).to(torch.bfloat16)
+    _check(tokens, h, dev, seed=D)
+
+
+@pytest.mark.parametrize("dtype", [torch.int64, torch.int32])
+def test_span_count(dev, dtype):
+    g = torch.Generator().manual_seed(3)
+    for B, T in ((1, 1), (3, 63), (5, 64), (9, 1000)):
+        tokens = torch.randint(0, 6, (B, T), generator=g).to(dtype)
+        assert max_spans(tokens.to(dev)) == max_spans(tokens)
+        assert max_spans(tokens.T.contiguous().T.to(dev)) == max_spans(tokens)
