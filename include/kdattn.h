@@ -326,6 +326,11 @@ int kd_tile_masks(const void *plan, int64_t plan_bytes, int32_t B, int32_t T, in
 int kd_mask_dense(const void *plan, int64_t plan_bytes, int32_t B, int32_t H, int32_t T, int32_t D, uint8_t *out,
                   const int64_t *strides, void *stream);
 
+/* d signs (+1 where bit i % 64 of bits[i / 64] is set, else -1) written to the
+ * device array signs; d <= 256.  bits is host memory, read before the call
+ * returns, and nothing is waited for. */
+int kd_signs(const uint64_t *bits, int32_t d, float *signs, void *stream);
+
 /* y = x R with R = diag(signs) H_D / sqrt(D) (or x R^T when inverse), per
  * row, in a fixed fp32 evaluation order (bit-reproducible); optionally
  * max |y| per (b, h) into amax.  The reference only names this operation

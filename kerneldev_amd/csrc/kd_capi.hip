@@ -140,6 +140,13 @@ void kd_struct_sizes4(size_t* span) {
   if (span) *span = sizeof(kd_span_args);
 }
 
+int kd_signs(const uint64_t* bits, int32_t d, float* signs, void* stream) {
+  if (bits == nullptr || signs == nullptr) return fail(KD_ERR_INVALID, "bits and signs are required");
+  if (d < 1 || d > 256) return fail(KD_ERR_UNSUPPORTED, "d must be in 1 .. 256");
+  const int r = kd::launch_signs(bits, d, signs, as_stream(stream));
+  return r ? fail(r, "kernel launch failed (signs)") : KD_OK;
+}
+
 int kd_span_count(const kd_span_args* a, int32_t* counts, void* stream) {
   if (a == nullptr) return fail(KD_ERR_INVALID, "args is NULL");
   if (a->B < 1 || a->T < 1) return fail(KD_ERR_INVALID, "B and T must be >= 1");

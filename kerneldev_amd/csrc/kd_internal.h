@@ -73,6 +73,7 @@ int launch_dkdv(const AttnArgs& a, const uint8_t* plan, float* ws, hipStream_t s
 int launch_hadamard(const kd_rot_args& a, hipStream_t st);
 int launch_quant(const kd_quant_args& a, hipStream_t st);
 int launch_absmax(const kd_quant_args& a, float* amax, hipStream_t st);
+int launch_signs(const uint64_t* bits, int d, float* out, hipStream_t st);
 int launch_span_count(const kd_span_args& a, int32_t* counts, hipStream_t st);
 int launch_span(const kd_span_args& a, hipStream_t st);
 int launch_span_bwd(const kd_span_args& a, hipStream_t st);

@@ -395,6 +395,21 @@ pybind11::object span(const Tensor& tokens, const Tensor& h, int64_t n) {
   return pybind11::cast(SpanHead::apply(h, tokens, n));
 }
 
+// draws (0 or 1, int64 on the host, at most 256 of them) as signs -1 or +1, fp32 on the device
+pybind11::object signs(const Tensor& draws, c10::Device on) {
+  if (!plain_mode() || !on.is_cuda() || !draws.is_cpu() || draws.scalar_type() != at::kLong || !draws.is_contiguous() ||
+      draws.numel() < 1 || draws.numel() > 256)
+    return pybind11::none();
+  const c10::DeviceGuard guard(on);
+  const int64_t* x = static_cast<const int64_t*>(draws.data_ptr());
+  uint64_t bits[4] = {};
+  for (int64_t i = 0; i < draws.numel(); ++i) bits[i / 64] |= uint64_t(x[i] & 1) << (i % 64);
+  Tensor out = at::empty({draws.numel()}, at::TensorOptions().dtype(at::kFloat).device(on));
+  check(kd_signs(bits, int32_t(draws.numel()), static_cast<float*>(out.data_ptr()),
+                 stream_on(out.device())), "kd_signs");
+  return pybind11::cast(out);
+}
+
 // [SPAN] tokens of each row of tokens [B, T], int32 [B] on its device
 pybind11::object span_counts(const Tensor& tokens) {
   if (!plain_mode() || !plain(tokens) || tokens.dim() != 2 || tokens.numel() == 0 ||
@@ -418,6 +433,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("flash", torch::wrap_pybind_function(flash));
   m.def("plan_from_metadata", torch::wrap_pybind_function(plan_from_metadata));
   m.def("plan_from_tokens", torch::wrap_pybind_function(plan_from_tokens));
+  m.def("signs", torch::wrap_pybind_function(signs));
   m.def("span_counts", torch::wrap_pybind_function(span_counts));
   m.def("span", torch::wrap_pybind_function(span));
 }

@@ -26,7 +26,12 @@ def generate_hadamard_signs(d: int, seed: int | None = None, device=None) -> tor
     if d <= 0 or d & (d - 1):
         raise ValueError(f"d must be a power of two, got {d}")
     g = torch.Generator("cpu").manual_seed(0 if seed is None else int(seed))
-    s = torch.randint(0, 2, (d,), generator=g, dtype=torch.int64).to(torch.float32) * 2 - 1
+    s = torch.randint(0, 2, (d,), generator=g, dtype=torch.int64)
+    if device is not None and torch.device(device).type == "cuda" and d <= 256 and _lib.eager(s):
+        on_device = _lib.native().signs(s, torch.device(device))  # in a launch's arguments: no copy waits
+        if on_device is not None:
+            return on_device
+    s = s.to(torch.float32) * 2 - 1
     return s if device is None else s.to(device)
 
 

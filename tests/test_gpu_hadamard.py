@@ -154,3 +154,21 @@ def test_attention_with_hadamard_fp16_ragged_lens(dev, D):
     assert_close("dq", qd.grad, ref["dq"])
     assert_close("dk", kd.grad, ref["dk"])
     assert_close("dv", vd.grad, ref["dv"])
+
+
+@pytest.mark.parametrize("d", [1, 2, 16, 64, 128, 256, 512])
+def test_signs_on_the_device(dev, d):
+    """The same signs as on the host, and nothing is waited for: they can be made inside a graph capture
+    (up to 256, where they travel in the launch's arguments)."""
+    for seed in (None, 0, 7):
+        want = generate_hadamard_signs(d, seed)
+        got = generate_hadamard_signs(d, seed, device=dev)
+        assert got.device.type == "cuda" and torch.equal(got.cpu(), want)
+        if d <= 256:
+            g = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(g):
+                again = generate_hadamard_signs(d, seed, device="cuda")
+            for _ in range(2):
+                g.replay()
+                torch.cuda.synchronize()
+                assert torch.equal(again.cpu(), want)
