@@ -326,6 +326,20 @@ int kd_tile_masks(const void *plan, int64_t plan_bytes, int32_t B, int32_t T, in
 int kd_mask_dense(const void *plan, int64_t plan_bytes, int32_t B, int32_t H, int32_t T, int32_t D, uint8_t *out,
                   const int64_t *strides, void *stream);
 
+/* y = x rsqrt(mean(x^2) + eps) over contiguous rows of D bf16 / fp16 elements
+ * (D a multiple of 8, at most 2048), fp32 inside (model.py:31-39); rstd [rows]
+ * (may be NULL) receives the factor, which the backward
+ * dx = rstd (dy - x rstd^2 mean(dy x)) reads.  All 16-byte aligned. */
+int kd_rms_norm(const void *x, void *y, float *rstd, int64_t rows, int32_t D, int32_t dtype, float eps, void *stream);
+int kd_rms_norm_bwd(const void *x, const void *dy, const float *rstd, void *dx, int64_t rows, int32_t D,
+                    int32_t dtype, void *stream);
+
+/* y = silu(a) b over n contiguous bf16 / fp16 elements, fp32 inside
+ * (model.py:42-52), and its gradients.  All 16-byte aligned. */
+int kd_swiglu(const void *a, const void *b, void *y, int64_t n, int32_t dtype, void *stream);
+int kd_swiglu_bwd(const void *a, const void *b, const void *dy, void *da, void *db, int64_t n, int32_t dtype,
+                  void *stream);
+
 /* d signs (+1 where bit i % 64 of bits[i / 64] is set, else -1) written to the
  * device array signs; d <= 256.  bits is host memory, read before the call
  * returns, and nothing is waited for. */

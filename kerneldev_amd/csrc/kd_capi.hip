@@ -3,6 +3,7 @@
 // shape or stride never reaches a kernel.
 #include <cmath>
 #include <cstdio>
+#include <initializer_list>
 #include <string>
 
 #include "kd_internal.h"
@@ -138,6 +139,54 @@ void kd_struct_sizes3(size_t* tokens) {
 
 void kd_struct_sizes4(size_t* span) {
   if (span) *span = sizeof(kd_span_args);
+}
+
+static int check_rms(int64_t rows, int32_t D, int32_t dtype) {
+  if (rows < 1 || rows > (int64_t(1) << 32)) return fail(KD_ERR_INVALID, "rows must be in 1 .. 2^32");
+  if (D < 8 || D > 2048 || D % 8 != 0) return fail(KD_ERR_UNSUPPORTED, "D must be a multiple of 8 in 8 .. 2048");
+  if (dtype != KD_BF16 && dtype != KD_F16) return fail(KD_ERR_UNSUPPORTED, "dtype must be bf16 or fp16");
+  return KD_OK;
+}
+static int check_flat(std::initializer_list<const void*> ps) {
+  for (const void* p : ps)
+    if (p == nullptr || !aligned16(p)) return fail(KD_ERR_INVALID, "operands must be given and 16-byte aligned");
+  return KD_OK;
+}
+static int check_gate(int64_t n, int32_t dtype) {
+  if (n < 1 || n > (int64_t(1) << 40)) return fail(KD_ERR_INVALID, "n must be in 1 .. 2^40");
+  if (dtype != KD_BF16 && dtype != KD_F16) return fail(KD_ERR_UNSUPPORTED, "dtype must be bf16 or fp16");
+  return KD_OK;
+}
+
+int kd_rms_norm(const void* x, void* y, float* rstd, int64_t rows, int32_t D, int32_t dtype, float eps, void* stream) {
+  int r;
+  if ((r = check_rms(rows, D, dtype)) || (r = check_flat({x, y}))) return r;
+  r = kd::launch_rms_fwd(x, y, rstd, rows, D, dtype, eps, as_stream(stream));
+  return r ? fail(r, "kernel launch failed (rms norm)") : KD_OK;
+}
+
+int kd_rms_norm_bwd(const void* x, const void* dy, const float* rstd, void* dx, int64_t rows, int32_t D, int32_t dtype,
+                    void* stream) {
+  int r;
+  if ((r = check_rms(rows, D, dtype)) || (r = check_flat({x, dy, dx}))) return r;
+  if (rstd == nullptr) return fail(KD_ERR_INVALID, "rstd is required");
+  r = kd::launch_rms_bwd(x, dy, rstd, dx, rows, D, dtype, as_stream(stream));
+  return r ? fail(r, "kernel launch failed (rms norm backward)") : KD_OK;
+}
+
+int kd_swiglu(const void* a, const void* b, void* y, int64_t n, int32_t dtype, void* stream) {
+  int r;
+  if ((r = check_gate(n, dtype)) || (r = check_flat({a, b, y}))) return r;
+  r = kd::launch_gate_fwd(a, b, y, n, dtype, as_stream(stream));
+  return r ? fail(r, "kernel launch failed (swiglu)") : KD_OK;
+}
+
+int kd_swiglu_bwd(const void* a, const void* b, const void* dy, void* da, void* db, int64_t n, int32_t dtype,
+                  void* stream) {
+  int r;
+  if ((r = check_gate(n, dtype)) || (r = check_flat({a, b, dy, da, db}))) return r;
+  r = kd::launch_gate_bwd(a, b, dy, da, db, n, dtype, as_stream(stream));
+  return r ? fail(r, "kernel launch failed (swiglu backward)") : KD_OK;
 }
 
 int kd_signs(const uint64_t* bits, int32_t d, float* signs, void* stream) {

@@ -73,6 +73,12 @@ int launch_dkdv(const AttnArgs& a, const uint8_t* plan, float* ws, hipStream_t s
 int launch_hadamard(const kd_rot_args& a, hipStream_t st);
 int launch_quant(const kd_quant_args& a, hipStream_t st);
 int launch_absmax(const kd_quant_args& a, float* amax, hipStream_t st);
+int launch_rms_fwd(const void* x, void* y, float* rstd, int64_t rows, int D, int dtype, float eps, hipStream_t st);
+int launch_rms_bwd(const void* x, const void* dy, const float* rstd, void* dx, int64_t rows, int D, int dtype,
+                   hipStream_t st);
+int launch_gate_fwd(const void* a, const void* b, void* y, int64_t n, int dtype, hipStream_t st);
+int launch_gate_bwd(const void* a, const void* b, const void* dy, void* da, void* db, int64_t n, int dtype,
+                    hipStream_t st);
 int launch_signs(const uint64_t* bits, int d, float* out, hipStream_t st);
 int launch_span_count(const kd_span_args& a, int32_t* counts, hipStream_t st);
 int launch_span(const kd_span_args& a, hipStream_t st);

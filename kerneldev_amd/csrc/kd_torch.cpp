@@ -11,6 +11,7 @@
 // H8 T777 d32: 322 -> 88; span_scores of B8 T2048 D768: 226 -> 96).  Every entry returns None where the call is not plain (see
 // plain()), and the caller then goes through the custom op.
 #include <ATen/ATen.h>
+#include <ATen/autocast_mode.h>
 #include <ATen/record_function.h>
 #include <ATen/PythonTorchFunctionTLS.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
@@ -79,6 +80,16 @@ Tensor kernel_ready(const Tensor& x) {
   const bool ok = s[3] == 1 && reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 && s[0] % 8 == 0 && s[1] % 8 == 0 &&
                   s[2] % 8 == 0 && s[2] >= x.size(3) && x.size(2) * s[2] * x.element_size() < (int64_t(1) << 31);
   return ok ? x : x.contiguous();
+}
+
+// A gradient of x [B, H, T, D] (`ready`: x as the kernels read it): contiguous,
+// or in [B, T, H, D] memory where x is, so that a projection's backward reads
+// it without a copy (attention._grad_like)
+Tensor grad_like(const Tensor& x, const Tensor& ready) {
+  const int64_t H = x.size(1), T = x.size(2), D = x.size(3);
+  if (x.is_same(ready) && x.strides() == at::IntArrayRef({T * H * D, D, H * D, 1}))
+    return at::empty_strided(x.sizes(), x.strides(), x.options());
+  return at::empty(x.sizes(), x.options());
 }
 
 int dtype_code(at::ScalarType t) {
@@ -256,7 +267,8 @@ struct Attention : torch::autograd::Function<Attention> {
       d_o = kernel_ready(d_o);
       const Tensor &lse = s[4], &plan = s[5], &o_lo = s[6];
       const int64_t B = q.size(0), H = q.size(1), T = q.size(2), D = q.size(3);
-      for (Tensor& t : g) t = at::empty({B, H, T, D}, q.options());
+      const Tensor* ready[3] = {&q, &k, &v};
+      for (int i = 0; i < 3; ++i) g[i] = grad_like(s[i], *ready[i]);
       const Tensor delta = at::empty({2, B, H, T}, q.options().dtype(at::kFloat));
       kd_attn_args a = attn_args(q, k, v, ctx->saved_data["sm_scale"].toDouble(), ctx->saved_data["prec"].toInt());
       a.o = o.data_ptr();
@@ -395,6 +407,94 @@ pybind11::object span(const Tensor& tokens, const Tensor& h, int64_t n) {
   return pybind11::cast(SpanHead::apply(h, tokens, n));
 }
 
+// ------------------------------------------------------- transformer block
+// Under create_graph the backward of both is formed with differentiable torch
+// operations, so that second derivatives exist as they do for the eager forms.
+bool flat16(const Tensor& t) {
+  return plain(t) && t.is_contiguous() && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 &&
+         (t.scalar_type() == at::kBFloat16 || t.scalar_type() == at::kHalf) && t.numel() > 0;
+}
+bool second_order(const Tensor& d, const Tensor& a, const Tensor& b) {
+  return at::GradMode::is_enabled() && (d.requires_grad() || a.requires_grad() || (b.defined() && b.requires_grad()));
+}
+Tensor ready_grad(Tensor d, const Tensor& like) {
+  if (d.is_neg()) d = d.resolve_neg();
+  if (d._is_zerotensor()) d = at::zeros(d.sizes(), like.options());
+  d = d.contiguous();
+  return reinterpret_cast<uintptr_t>(d.data_ptr()) % 16 ? d.clone() : d;
+}
+
+struct RmsNorm : torch::autograd::Function<RmsNorm> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& x, double eps) {
+    const c10::DeviceGuard on(x.device());
+    const int64_t D = x.size(-1), rows = x.numel() / D;
+    Tensor y = at::empty(x.sizes(), x.options()), rstd = at::empty({rows}, x.options().dtype(at::kFloat));
+    check(kd_rms_norm(x.data_ptr(), y.data_ptr(), static_cast<float*>(rstd.data_ptr()), rows, int32_t(D),
+                      dtype_code(x.scalar_type()), float(eps), stream_of(x)), "kd_rms_norm");
+    ctx->save_for_backward({x, rstd});
+    ctx->saved_data["eps"] = eps;
+    return y;
+  }
+  static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
+    const variable_list s = ctx->get_saved_variables();
+    const Tensor &x = s[0], &rstd = s[1];
+    if (second_order(grads[0], x, Tensor())) {
+      const Tensor f = x.to(at::kFloat), d = grads[0].to(at::kFloat);
+      const Tensor r = at::rsqrt(f.pow(2).mean(-1, true) + ctx->saved_data["eps"].toDouble());
+      return {(r * (d - f * (r * r * (d * f).mean(-1, true)))).to(x.scalar_type()), Tensor()};
+    }
+    at::AutoDispatchBelowADInplaceOrView below;
+    const c10::DeviceGuard on(x.device());
+    const Tensor d = ready_grad(grads[0], x);
+    const int64_t D = x.size(-1);
+    Tensor dx = at::empty(x.sizes(), x.options());
+    check(kd_rms_norm_bwd(x.data_ptr(), d.data_ptr(), static_cast<const float*>(rstd.data_ptr()), dx.data_ptr(),
+                          x.numel() / D, int32_t(D), dtype_code(x.scalar_type()), stream_of(x)), "kd_rms_norm_bwd");
+    return {dx, Tensor()};
+  }
+};
+
+struct Gate : torch::autograd::Function<Gate> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& a, const Tensor& b) {
+    const c10::DeviceGuard on(a.device());
+    Tensor y = at::empty(a.sizes(), a.options());
+    check(kd_swiglu(a.data_ptr(), b.data_ptr(), y.data_ptr(), a.numel(), dtype_code(a.scalar_type()), stream_of(a)),
+          "kd_swiglu");
+    ctx->save_for_backward({a, b});
+    return y;
+  }
+  static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
+    const variable_list s = ctx->get_saved_variables();
+    const Tensor &a = s[0], &b = s[1];
+    if (second_order(grads[0], a, b)) {
+      const Tensor u = a.to(at::kFloat), v = b.to(at::kFloat), d = grads[0].to(at::kFloat), g = at::sigmoid(u);
+      return {(d * v * g * (1 + u * (1 - g))).to(a.scalar_type()), (d * (u * g)).to(a.scalar_type())};
+    }
+    at::AutoDispatchBelowADInplaceOrView below;
+    const c10::DeviceGuard on(a.device());
+    const Tensor d = ready_grad(grads[0], a);
+    Tensor da = at::empty(a.sizes(), a.options()), db = at::empty(a.sizes(), a.options());
+    check(kd_swiglu_bwd(a.data_ptr(), b.data_ptr(), d.data_ptr(), da.data_ptr(), db.data_ptr(), a.numel(),
+                        dtype_code(a.scalar_type()), stream_of(a)), "kd_swiglu_bwd");
+    return {da, db};
+  }
+};
+
+// (autocast takes the eager forms through other types)
+bool block_mode() { return plain_mode() && !at::autocast::is_autocast_enabled(at::kCUDA); }
+
+pybind11::object rms_norm(const Tensor& x, double eps) {
+  if (!block_mode() || x.dim() < 1 || !flat16(x) || x.size(-1) % 8 != 0 || x.size(-1) > 2048) return pybind11::none();
+  return pybind11::cast(RmsNorm::apply(x, eps));
+}
+
+pybind11::object swiglu(const Tensor& a, const Tensor& b) {
+  if (!block_mode() || !flat16(a) || !flat16(b) || a.sizes() != b.sizes() || a.scalar_type() != b.scalar_type() ||
+      a.device() != b.device())
+    return pybind11::none();
+  return pybind11::cast(Gate::apply(a, b));
+}
+
 // draws (0 or 1, int64 on the host, at most 256 of them) as signs -1 or +1, fp32 on the device
 pybind11::object signs(const Tensor& draws, c10::Device on) {
   if (!plain_mode() || !on.is_cuda() || !draws.is_cpu() || draws.scalar_type() != at::kLong || !draws.is_contiguous() ||
@@ -433,6 +533,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("flash", torch::wrap_pybind_function(flash));
   m.def("plan_from_metadata", torch::wrap_pybind_function(plan_from_metadata));
   m.def("plan_from_tokens", torch::wrap_pybind_function(plan_from_tokens));
+  m.def("rms_norm", torch::wrap_pybind_function(rms_norm));
+  m.def("swiglu", torch::wrap_pybind_function(swiglu));
   m.def("signs", torch::wrap_pybind_function(signs));
   m.def("span_counts", torch::wrap_pybind_function(span_counts));
   m.def("span", torch::wrap_pybind_function(span));

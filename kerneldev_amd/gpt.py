@@ -27,6 +27,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from . import _lib
 from .attention import AttentionPlan, build_plan, build_plan_from_tokens, flash_attention, mask_mode
 from .metadata import CLS, MASKQ, SPAN, derive_metadata
 from .span_head import has_cocktail_layout, span_scores
@@ -42,6 +43,10 @@ class RMSNorm(nn.Module):
         self.eps = eps
 
     def forward(self, x):
+        if x.is_cuda and _lib.eager(x):
+            y = _lib.native().rms_norm(x, self.eps)  # bf16 / fp16 rows in one kernel, fp32 inside
+            if y is not None:
+                return y
         return x * torch.rsqrt(x.pow(2).mean(-1, keepdim=True) + self.eps)
 
 
@@ -55,7 +60,9 @@ class SwiGLU(nn.Module):
         self.w3 = nn.Linear(dim, hidden, bias=False)
 
     def forward(self, x):
-        return self.w2(F.silu(self.w1(x)) * self.w3(x))
+        a, b = self.w1(x), self.w3(x)
+        y = _lib.native().swiglu(a, b) if a.is_cuda and _lib.eager(a, b) else None  # silu(a) b in one kernel, fp32 inside
+        return self.w2(F.silu(a) * b if y is None else y)
 
 
 class MultiHeadAttention(nn.Module):

@@ -1,0 +1,104 @@
+"""GPU: RMSNorm and the SwiGLU gate of gpt.py on their kernels (kd_block.hip).
+
+Against the same formulas in fp64 on the same 16-bit inputs.  The kernels work
+in fp32 and round once, so an output is within half an ulp of the exact value
+plus the fp32 arithmetic's error: 2^-8 |ref| (bf16, half of 2^-7) or 2^-11
+|ref| (fp16), and 2^-19 of the largest term that enters it (fp32 sums of up to
+2048 terms, exp2 and one division).
+"""
+import pytest
+import torch
+import torch.nn.functional as F
+
+from kerneldev_amd import _lib
+from kerneldev_amd.gpt import RMSNorm, SwiGLU
+
+pytestmark = pytest.mark.gpu
+
+
+def _close(got, ref, dtype, scale):
+    ulp = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    tiny = 0.0 if dtype == torch.bfloat16 else 2.0 ** -25  # fp16's subnormal spacing
+    err = (got.double() - ref).abs()
+    assert bool((err <= ulp * 1.01 * ref.abs() + 2.0 ** -19 * scale + tiny).all()), (err / (ref.abs() + 1e-30)).max().item()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("shape", [(1, 8), (3, 5, 504), (2, 7, 512), (9, 520), (1, 4, 1024), (5, 1032), (2, 3, 2048)])
+def test_rms_norm(dev, shape, dtype):
+    g = torch.Generator("cpu").manual_seed(sum(shape))
+    x = (torch.randn(shape, generator=g) * 3).to(dtype).to(dev).requires_grad_(True)
+    dy = torch.randn(shape, generator=g).to(dtype).to(dev)
+    y = RMSNorm()(x)
+    assert "CppFunction" in type(y.grad_fn).__name__
+    dx, = torch.autograd.grad(y, x, dy)
+    x64 = x.detach().double().requires_grad_(True)
+    r = torch.rsqrt(x64.pow(2).mean(-1, keepdim=True) + 1e-6)
+    y64 = x64 * r
+    want, = torch.autograd.grad(y64, x64, dy.double())
+    _close(y.detach(), y64.detach(), dtype, y64.detach().abs())
+    d = dy.double()
+    terms = (r * (d.abs() + y64.abs() * (d * y64).abs().mean(-1, keepdim=True))).detach()
+    _close(dx, want, dtype, terms)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n", [1, 7, 8, 2048, 2055, 40000])
+def test_gate(dev, n, dtype):
+    g = torch.Generator("cpu").manual_seed(n)
+    a, b, dy = ((torch.randn(n, generator=g) * s).to(dtype).to(dev) for s in (6, 2, 1))
+    a[0] = -80.0  # exp(80) is finite in fp32; the gate is about -80 e^-80
+    a.requires_grad_(True), b.requires_grad_(True)
+    y = _lib.native().swiglu(a, b)
+    da, db = torch.autograd.grad(y, (a, b), dy)
+    a64, b64 = a.detach().double().requires_grad_(True), b.detach().double().requires_grad_(True)
+    y64 = F.silu(a64) * b64
+    wa, wb = torch.autograd.grad(y64, (a64, b64), dy.double())
+    _close(y.detach(), y64.detach(), dtype, y64.detach().abs())
+    # silu' = s + a s (1 - s): its two terms may cancel
+    s = torch.sigmoid(a64.detach())
+    _close(da, wa, dtype, (dy.double() * b64.detach()).abs() * (s + a64.detach().abs() * s * (1 - s)))
+    _close(db, wb, dtype, wb.abs())
+
+
+def test_the_eager_forms_where_the_kernels_do_not_apply(dev):
+    x = torch.randn(4, 36, device=dev)
+    for y in (x, x.bfloat16(), x.bfloat16()[:, :24], torch.randn(2, 4096, device=dev).bfloat16(), x.cpu().half()):
+        assert RMSNorm()(y).shape == y.shape  # fp32, a width of 36, strided rows, wide rows, the CPU
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert RMSNorm()(x.bfloat16()[:, :32].contiguous()).dtype == torch.float32  # pow runs in fp32 there
+    # second derivatives exist as for the eager forms
+    m = SwiGLU(64, 128).to(dev).bfloat16()
+    z = torch.randn(3, 64, device=dev).bfloat16().requires_grad_(True)
+    out = m(RMSNorm()(z)).float().pow(2).sum()
+    gz, = torch.autograd.grad(out, z, create_graph=True)
+    gg, = torch.autograd.grad(gz.float().pow(2).sum(), z)
+    z64 = z.detach().double().requires_grad_(True)
+    w1, w2, w3 = (w.weight.detach().double() for w in (m.w1, m.w2, m.w3))
+    n = z64 * torch.rsqrt(z64.pow(2).mean(-1, keepdim=True) + 1e-6)
+    o64 = ((F.silu(n @ w1.T) * (n @ w3.T)) @ w2.T).pow(2).sum()
+    g64, = torch.autograd.grad(o64, z64, create_graph=True)
+    gg64, = torch.autograd.grad(g64.pow(2).sum(), z64)
+    # bf16 activations and gradients between the layers: a few per cent of a second derivative
+    assert (gg.double() - gg64).norm() <= 0.1 * gg64.norm()
+    compiled = torch.compile(RMSNorm(), fullgraph=True)
+    w = torch.randn(8, 64, device=dev).bfloat16()
+    assert torch.allclose(compiled(w).float(), RMSNorm()(w).float(), rtol=2 ** -6)
+    # forward-mode AD and vmap through the eager forms
+    import torch.autograd.forward_ad as fw
+    with fw.dual_level():
+        t = fw.unpack_dual(RMSNorm()(fw.make_dual(w, torch.ones_like(w)))).tangent
+        assert t is not None and t.shape == w.shape
+    assert torch.vmap(RMSNorm())(w[None]).shape == (1, 8, 64)
+
+
+def test_gradient_layout_follows_the_operand(dev):
+    from kerneldev_amd import flash_attention
+
+    x = torch.randn(2, 100, 3, 64, device=dev).bfloat16()
+    q = x.transpose(1, 2).requires_grad_(True)  # [B, H, T, d] in [B, T, H, d] memory
+    c = x.transpose(1, 2).contiguous().requires_grad_(True)
+    do = torch.randn_like(c)
+    gq, = torch.autograd.grad(flash_attention(q, q, q), q, do)
+    gc, = torch.autograd.grad(flash_attention(c, c, c), c, do)
+    assert torch.equal(gq, gc) and gq.stride() == q.stride() and gc.is_contiguous()
