@@ -340,6 +340,14 @@ int kd_swiglu(const void *a, const void *b, void *y, int64_t n, int32_t dtype, v
 int kd_swiglu_bwd(const void *a, const void *b, const void *dy, void *da, void *db, int64_t n, int32_t dtype,
                   void *stream);
 
+/* dW [N, K] = dY^T X of contiguous bf16 / fp16 dY [M, N] and X [M, K], fp32
+ * sums, rounded once (the weight gradient of a projection y = x W^T over M
+ * tokens).  N and K are multiples of 8; everything is 16-byte aligned; ws holds
+ * kd_weight_grad_ws_bytes bytes, used by this call alone. */
+int64_t kd_weight_grad_ws_bytes(int32_t M, int32_t N, int32_t K, int32_t dtype);
+int kd_weight_grad(const void *dy, const void *x, void *dw, int32_t M, int32_t N, int32_t K, int32_t dtype,
+                   void *ws, int64_t ws_bytes, void *stream);
+
 /* d signs (+1 where bit i % 64 of bits[i / 64] is set, else -1) written to the
  * device array signs; d <= 256.  bits is host memory, read before the call
  * returns, and nothing is waited for. */

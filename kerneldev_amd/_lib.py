@@ -120,6 +120,9 @@ SIGNATURES = {
     "kd_span_scores": (c_int, [POINTER(SpanArgs), c_void_p]),
     "kd_span_scores_bwd": (c_int, [POINTER(SpanArgs), c_void_p]),
     "kd_plan_build_tokens": (c_int, [POINTER(TokenArgs), c_void_p, c_int64, c_void_p]),
+    "kd_weight_grad_ws_bytes": (c_int64, [c_int32, c_int32, c_int32, c_int32]),
+    "kd_weight_grad": (c_int, [c_void_p, c_void_p, c_void_p, c_int32, c_int32, c_int32, c_int32, c_void_p, c_int64,
+                               c_void_p]),
     "kd_rms_norm": (c_int, [c_void_p, c_void_p, c_void_p, c_int64, c_int32, c_int32, c_float, c_void_p]),
     "kd_rms_norm_bwd": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int32, c_int32, c_void_p]),
     "kd_swiglu": (c_int, [c_void_p, c_void_p, c_void_p, c_int64, c_int32, c_void_p]),

@@ -174,6 +174,28 @@ int kd_rms_norm_bwd(const void* x, const void* dy, const float* rstd, void* dx, 
   return r ? fail(r, "kernel launch failed (rms norm backward)") : KD_OK;
 }
 
+static int check_wgrad(int32_t M, int32_t N, int32_t K, int32_t dtype) {
+  if (M < 1 || N < 8 || K < 8) return fail(KD_ERR_INVALID, "M must be >= 1, N and K >= 8");
+  if (N % 8 != 0 || K % 8 != 0) return fail(KD_ERR_UNSUPPORTED, "N and K must be multiples of 8");
+  if (int64_t(M) * std::max(N, K) * 2 >= (int64_t(1) << 31) || int64_t(N) * K >= (int64_t(1) << 28))
+    return fail(KD_ERR_UNSUPPORTED, "operands must be < 2^31 bytes and dW < 2^28 elements");
+  if (dtype != KD_BF16 && dtype != KD_F16) return fail(KD_ERR_UNSUPPORTED, "dtype must be bf16 or fp16");
+  return KD_OK;
+}
+
+int64_t kd_weight_grad_ws_bytes(int32_t M, int32_t N, int32_t K, int32_t dtype) {
+  return check_wgrad(M, N, K, dtype) ? -1 : 4 * int64_t(kd::wgrad_pieces(M, N, K)) * N * K;
+}
+
+int kd_weight_grad(const void* dy, const void* x, void* dw, int32_t M, int32_t N, int32_t K, int32_t dtype, void* ws,
+                   int64_t ws_bytes, void* stream) {
+  int r;
+  if ((r = check_wgrad(M, N, K, dtype)) || (r = check_flat({dy, x, dw, ws}))) return r;
+  if (ws_bytes < kd_weight_grad_ws_bytes(M, N, K, dtype)) return fail(KD_ERR_INVALID, "ws is too small");
+  r = kd::launch_wgrad(dy, x, dw, static_cast<float*>(ws), M, N, K, dtype, as_stream(stream));
+  return r ? fail(r, "kernel launch failed (weight gradient)") : KD_OK;
+}
+
 int kd_swiglu(const void* a, const void* b, void* y, int64_t n, int32_t dtype, void* stream) {
   int r;
   if ((r = check_gate(n, dtype)) || (r = check_flat({a, b, y}))) return r;

@@ -50,14 +50,29 @@ class RMSNorm(nn.Module):
         return x * torch.rsqrt(x.pow(2).mean(-1, keepdim=True) + self.eps)
 
 
+class Projection(nn.Linear):
+    """A linear layer without bias whose weight gradient runs on the library's own
+    kernel (csrc/kd_wgrad.hip) where that is the faster one."""
+
+    def __init__(self, in_features: int, out_features: int):
+        super().__init__(in_features, out_features, bias=False)
+
+    def forward(self, x):
+        if x.is_cuda and _lib.eager(x, self.weight):
+            y = _lib.native().projection(x, self.weight)
+            if y is not None:
+                return y
+        return super().forward(x)
+
+
 class SwiGLU(nn.Module):
     """w2(silu(w1 x) * w3 x) (model.py:42-52)."""
 
     def __init__(self, dim: int, hidden: int):
         super().__init__()
-        self.w1 = nn.Linear(dim, hidden, bias=False)
-        self.w2 = nn.Linear(hidden, dim, bias=False)
-        self.w3 = nn.Linear(dim, hidden, bias=False)
+        self.w1 = Projection(dim, hidden)
+        self.w2 = Projection(hidden, dim)
+        self.w3 = Projection(dim, hidden)
 
     def forward(self, x):
         a, b = self.w1(x), self.w3(x)
@@ -71,10 +86,10 @@ class MultiHeadAttention(nn.Module):
     def __init__(self, dim: int, n_heads: int, causal: bool = True, attention=None):
         super().__init__()
         self.n_heads, self.head_dim, self.causal = n_heads, dim // n_heads, causal
-        self.q_proj = nn.Linear(dim, dim, bias=False)
-        self.k_proj = nn.Linear(dim, dim, bias=False)
-        self.v_proj = nn.Linear(dim, dim, bias=False)
-        self.o_proj = nn.Linear(dim, dim, bias=False)
+        self.q_proj = Projection(dim, dim)
+        self.k_proj = Projection(dim, dim)
+        self.v_proj = Projection(dim, dim)
+        self.o_proj = Projection(dim, dim)
         self.attention = attention or flash_attention
 
     def forward(self, x, in_span, span_id, is_prefix, plan=None):

@@ -102,3 +102,55 @@ def test_gradient_layout_follows_the_operand(dev):
     gq, = torch.autograd.grad(flash_attention(q, q, q), q, do)
     gc, = torch.autograd.grad(flash_attention(c, c, c), c, do)
     assert torch.equal(gq, gc) and gq.stride() == q.stride() and gc.is_contiguous()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,N,K", [(1, 8, 8), (63, 128, 136), (64, 120, 128), (65, 256, 8), (200, 264, 520),
+                                   (1000, 128, 128), (4097, 72, 200), (16384, 256, 256), (5000, 2048, 1024)])
+def test_weight_gradient(dev, M, N, K, dtype):
+    """Edges of the 64-token steps, the 128 x 128 tiles and the pieces of the tokens.  fp32 sums of M products
+    (each exact): 2^-24 sqrt(M) of the root of the sum of squares, four times that and one rounding allowed."""
+    from kerneldev_amd.gpt import Projection
+
+    g = torch.Generator("cpu").manual_seed(M + N + K)
+    x = torch.randn(M, K, generator=g).to(dtype).to(dev)
+    dy = torch.randn(M, N, generator=g).to(dtype).to(dev)
+    p = Projection(K, N).to(dev).to(dtype)
+    x.requires_grad_(True)
+    y = p(x)
+    assert "CppFunction" in type(y.grad_fn).__name__
+    dx, dw = torch.autograd.grad(y, (x, p.weight), dy)
+    ref = dy.double().t() @ x.detach().double()
+    size = (dy.double().square().t() @ x.detach().double().square()).sqrt()
+    ulp = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    err = (dw.double() - ref).abs()
+    assert bool((err <= 1.01 * ulp * ref.abs() + 2.0 ** -22 * M ** 0.5 * size + 2.0 ** -25).all())
+    want = dy.double() @ p.weight.detach().double()
+    assert (dx.double() - want).norm() <= 2 * ulp * want.norm()
+
+
+def test_projection_forms(dev):
+    """The library's linear where the kernel does not apply, hooks, frozen weights and second derivatives."""
+    from kerneldev_amd.gpt import Projection
+
+    p = Projection(64, 72).to(dev).bfloat16()
+    x = torch.randn(2, 5, 64, device=dev).bfloat16()
+    seen = []
+    p.register_forward_hook(lambda *a: seen.append(1))
+    assert torch.equal(p(x), F.linear(x, p.weight)) and seen == [1]
+    with torch.no_grad():
+        assert p(x).grad_fn is None
+    y = p(x.transpose(0, 1))
+    assert y.shape == (5, 2, 72) and y.requires_grad
+    with torch.autocast("cuda", dtype=torch.float16):
+        assert p(x).dtype == torch.float16
+    p.weight.requires_grad_(False)
+    z = x.clone().requires_grad_(True)
+    assert torch.autograd.grad(p(z).sum(), z)[0].shape == z.shape
+    p.weight.requires_grad_(True)
+    gz, = torch.autograd.grad(p(z).float().pow(2).sum(), z, create_graph=True)
+    gw, = torch.autograd.grad(gz.float().sum(), p.weight)
+    w64 = p.weight.detach().double().requires_grad_(True)
+    g64, = torch.autograd.grad((2 * (z.detach().double() @ w64.T) @ w64).sum(), w64)
+    assert (gw.double() - g64).norm() <= 0.05 * g64.norm()
+    assert set(p.state_dict()) == {"weight"}
