@@ -162,20 +162,24 @@ int launch(const AttnArgs& a, const CombineArgs& c, bool fwd, int outputs, hipSt
 // kernel's time.  Pieces shorten it, and cost the partial results' way through
 // memory (ns rows D floats written and read, at ~5.9 TB/s), a second launch and
 // each piece's own start (4 us together).  The lines below come from sweeps of
-// ns = 1 .. 8 on causal and full masks (us, forward / dQ / dK+dV; bf16 unless
-// said; W = workgroups without pieces):
+// ns = 1 .. 8 on causal and full masks (us, forward / dQ / dK+dV; bf16 and causal
+// unless said; W = workgroups without pieces):
 //   B1 H12 T1531 d64  (W 144):  37 / 36 / 39   -> 27.5 / 28 / 33  at 3
 //   B1 H8 T4095 d128  (W 256):  110 / 120 / 139 -> 82 / 96 / 116  at 2
 //   B1 H1 T8192 d64   (W 64):   132 / 134 / 160 -> 44 / 57 / 45   at 4
 //   B1 H8 T2048 d256  (W 128):  99 / 170 / 238 -> 61 / 108 / 128  at 3
-//   B2 H8 T1024 d64, full (W 128): 23 -> 22 at 2, 25.6 at 4
+//   B2 H8 T1531 d64, full (W 192): 35 -> 37 at 2 and 3, 35 at 4: no gain left
+//   B4 H8 T395 d128   (W 128):  17 -> 22 at 2: lists of 7 tiles are too short
 //   B2 H8 T4096 d64   (W 512):  80 -> 79 at 2, 81 at 3: no pieces from here on
-//   fp32 B1 H8 T2048 d128 (W 256): 170 / 230 / 296 -> 110 / 150 / 186 at 4
-//   fp32 B2 H8 T4096 d128 (W 1024): 647 -> 626 at 2, 634 at 3
+//   fp32 B1 H8 T2048 d128 (W 256): 170 / 230 / 296 -> 102 / 145 / 188 at 3
+//   fp32 B4 H8 T777 d64   (W 448): 60 / 77 / 90 -> 49 / 64 / 78 at 2
+//   fp32 B8 H8 T395 d128  (W 512): 59 -> 63 at 2, full 75 -> 95
+//   fp32 B2 H8 T4096 d128 (W 1024): 647 -> 626 at 2: long causal lists only
 // 16-bit: pieces of two tiles or more while each has a CU to itself, of six or
 // more up to two a CU (at d = 256, where one fills a CU, up to one and a half).
-// fp32 (two workgroups a block): a tile takes four times as long, so one tile a
-// piece, up to eight a CU.
+// fp32 (two workgroups a block, a tile takes four times as long): one tile a
+// piece, up to two (d = 256), three (128) or four workgroups a CU.  And what a
+// piece saves has to be 1.45 times what it costs.
 int split_pieces(const AttnArgs& a, SplitPass pass) {
   const bool f32 = use_simt(a);
   const int nT = (a.T + 63) / 64, nblk = (nT + 1) / 2;
@@ -184,15 +188,16 @@ int split_pieces(const AttnArgs& a, SplitPass pass) {
   // us a tile step takes a workgroup that has its CU to itself
   constexpr float step16[4] = {1.0f, 1.0f, 1.7f, 3.0f}, step32[4] = {2.0f, 3.0f, 5.3f, 10.6f};
   constexpr float pass16[3] = {1.0f, 1.1f, 1.25f}, pass32[3] = {1.0f, 1.3f, 1.8f};
+  constexpr int64_t room32[4] = {1024, 1024, 768, 512};
   const float step = f32 ? step32[d] * pass32[pass] : step16[d] * pass16[pass];
   const int outs = pass == SPLIT_DKDV ? 2 : 1;
-  for (int ns = f32 ? 8 : 4; ns > 1; --ns) {
+  for (int ns = f32 ? 6 : 4; ns > 1; --ns) {
     const int64_t wg = W * ns;
-    const bool room = f32 ? nT >= ns && wg <= (ns > 4 ? 512 : 2048)
+    const bool room = f32 ? nT >= ns && (wg <= (ns > 4 ? 256 : room32[d]) || (wg <= 2048 && nT >= 32 * ns))
                           : (wg <= 256 && nT >= 2 * ns) || (wg <= (a.D == 256 ? 384 : 512) && nT >= 6 * ns);
     const float saved = step * float(nT) * (1.f - 1.f / float(ns));
     const float cost = 4.f + 1.4e-6f * float(ns * outs) * float(rows) * float(a.D);
-    if (room && saved > 1.2f * cost) return ns;
+    if (room && saved > 1.45f * cost) return ns;
   }
   return 1;
 }
