@@ -195,6 +195,19 @@ typedef struct kd_span_args {
   int64_t dh_strides[2];    /* (b, t) in elements, unit d stride */
 } kd_span_args;
 
+/* Packing for the bf16x3 route (kd_x3_pack / kd_x3_unpack): n tensors at once. */
+typedef struct kd_x3_args {
+  const void *src[4];       /* pack: fp32 [B, H, T, d]; unpack: bf16 contiguous [B, H, T, Dp] */
+  int64_t src_strides[4][3];/* pack: (b, h, t) in elements, multiples of 8 */
+  const void *lo[4];        /* unpack: the rounding residuals of src, same shape */
+  void *dst[4];             /* pack: bf16 contiguous [B, H, T, Dp]; unpack: fp32 [B, H, T, d] */
+  int64_t dst_strides[4][3];/* unpack: (b, h, t) in elements, multiples of 8 */
+  int32_t sel[4];           /* pack: 0 rows [h, h, l], 1 rows [h, l, h]; unpack: the second block added (1 or 2) */
+  int32_t n;                /* 1 .. 4 */
+  int32_t B, H, T, d, Dp;   /* d 16, 32 or 64; 3 d <= Dp <= 256, a multiple of 8 */
+  int32_t pad_;
+} kd_x3_args;
+
 /* Library version (major*10000 + minor*100 + patch).  3.0.0: the plan's size
  * beside its pointer in every entry point that takes a plan.  3.1.0:
  * kd_plan_layout writes 20 offsets (the dK/dV work order added).  3.2.0:
@@ -347,6 +360,13 @@ int kd_swiglu_bwd(const void *a, const void *b, const void *dy, void *da, void *
 int64_t kd_weight_grad_ws_bytes(int32_t M, int32_t N, int32_t K, int32_t dtype);
 int kd_weight_grad(const void *dy, const void *x, void *dw, int32_t M, int32_t N, int32_t K, int32_t dtype,
                    void *ws, int64_t ws_bytes, void *stream);
+
+/* fp32 rows x as packed bf16 rows of h = bf16(x) and l = bf16(x - h), zeros
+ * behind (pack), and the fp32 sum of a packed result's blocks 0 and sel, each with
+ * its residual (unpack). */
+int kd_x3_pack(const kd_x3_args *a, void *stream);
+int kd_x3_unpack(const kd_x3_args *a, void *stream);
+void kd_struct_sizes5(size_t *x3);
 
 /* d signs (+1 where bit i % 64 of bits[i / 64] is set, else -1) written to the
  * device array signs; d <= 256.  bits is host memory, read before the call

@@ -108,6 +108,16 @@ class SpanArgs(ctypes.Structure):
     ]
 
 
+class X3Args(ctypes.Structure):
+    """Mirror of ``kd_x3_args``."""
+
+    _fields_ = [
+        ("src", c_void_p * 4), ("src_strides", I64x3 * 4), ("lo", c_void_p * 4), ("dst", c_void_p * 4),
+        ("dst_strides", I64x3 * 4), ("sel", c_int32 * 4), ("n", c_int32),
+        ("B", c_int32), ("H", c_int32), ("T", c_int32), ("d", c_int32), ("Dp", c_int32), ("pad_", c_int32),
+    ]
+
+
 # name -> (restype, argtypes); every symbol include/kdattn.h declares
 SIGNATURES = {
     "kd_version": (c_int, []),
@@ -123,6 +133,9 @@ SIGNATURES = {
     "kd_weight_grad_ws_bytes": (c_int64, [c_int32, c_int32, c_int32, c_int32]),
     "kd_weight_grad": (c_int, [c_void_p, c_void_p, c_void_p, c_int32, c_int32, c_int32, c_int32, c_void_p, c_int64,
                                c_void_p]),
+    "kd_struct_sizes5": (None, [POINTER(c_size_t)]),
+    "kd_x3_pack": (c_int, [POINTER(X3Args), c_void_p]),
+    "kd_x3_unpack": (c_int, [POINTER(X3Args), c_void_p]),
     "kd_rms_norm": (c_int, [c_void_p, c_void_p, c_void_p, c_int64, c_int32, c_int32, c_float, c_void_p]),
     "kd_rms_norm_bwd": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int32, c_int32, c_void_p]),
     "kd_swiglu": (c_int, [c_void_p, c_void_p, c_void_p, c_int64, c_int32, c_void_p]),
@@ -178,14 +191,18 @@ def load():
     ts, ss = c_size_t(), c_size_t()
     lib.kd_struct_sizes3(ctypes.byref(ts))
     lib.kd_struct_sizes4(ctypes.byref(ss))
+    xs = c_size_t()
+    lib.kd_struct_sizes5(ctypes.byref(xs))
     if (ms.value != ctypes.sizeof(MetaArgs) or as_.value != ctypes.sizeof(AttnArgs)
             or rs.value != ctypes.sizeof(RotArgs) or qs.value != ctypes.sizeof(QuantArgs)
-            or ts.value != ctypes.sizeof(TokenArgs) or ss.value != ctypes.sizeof(SpanArgs)):
+            or ts.value != ctypes.sizeof(TokenArgs) or ss.value != ctypes.sizeof(SpanArgs)
+            or xs.value != ctypes.sizeof(X3Args)):
         raise ImportError(
             f"struct layout mismatch: C meta={ms.value} attn={as_.value} rot={rs.value} quant={qs.value} "
-            f"tokens={ts.value} span={ss.value}, ctypes meta={ctypes.sizeof(MetaArgs)} "
+            f"tokens={ts.value} span={ss.value} x3={xs.value}, ctypes meta={ctypes.sizeof(MetaArgs)} "
             f"attn={ctypes.sizeof(AttnArgs)} rot={ctypes.sizeof(RotArgs)} quant={ctypes.sizeof(QuantArgs)} "
-            f"tokens={ctypes.sizeof(TokenArgs)} span={ctypes.sizeof(SpanArgs)}")
+            f"tokens={ctypes.sizeof(TokenArgs)} span={ctypes.sizeof(SpanArgs)} "
+            f"x3={ctypes.sizeof(X3Args)}")
     _lib = lib
     return lib
 

@@ -23,7 +23,6 @@ from __future__ import annotations
 import ctypes
 import math
 
-import numpy as np
 import torch
 
 from . import _lib
@@ -415,6 +414,29 @@ def _hi_lo(hi: torch.Tensor, lo: torch.Tensor, d: int, second: int) -> torch.Ten
     return x[..., :d] + x[..., second * d:(second + 1) * d]
 
 
+def _x3_call(pack: bool, tensors, B, H, T, d, Dp):
+    """kd_x3_pack of ``(x, y, pattern)`` or kd_x3_unpack of ``(hi, lo, out, second)``, all in one launch."""
+    a = _lib.X3Args()
+    a.n, a.B, a.H, a.T, a.d, a.Dp = len(tensors), B, H, T, d, Dp
+    for i, t in enumerate(tensors):
+        if pack:
+            x, y, pattern = t
+            a.src[i], a.src_strides[i], a.dst[i], a.sel[i] = x.data_ptr(), _strides3(x), y.data_ptr(), pattern == "hlh"
+        else:
+            hi, lo, out, second = t
+            a.src[i], a.lo[i], a.dst[i], a.dst_strides[i] = hi.data_ptr(), lo.data_ptr(), out.data_ptr(), _strides3(out)
+            a.sel[i] = second
+    fn = _lib.load().kd_x3_pack if pack else _lib.load().kd_x3_unpack
+    _lib.check(fn(ctypes.byref(a), _stream(tensors[0][0].device)), "kd_x3_pack" if pack else "kd_x3_unpack")
+
+
+def _x3_packed(tensors, patterns, B, H, T, d, Dp):
+    tensors = [_kernel_ready(x) for x in tensors]
+    out = [torch.empty((B, H, T, Dp), dtype=torch.bfloat16, device=x.device) for x in tensors]
+    _x3_call(True, list(zip(tensors, out, patterns)), B, H, T, d, Dp)
+    return out
+
+
 @torch.library.custom_op("kdattn::fwd_x3", mutates_args=(), device_types=("cuda",))
 def _fwd_x3_op(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, lens: torch.Tensor | None,
                in_span: torch.Tensor | None, span_id: torch.Tensor | None,
@@ -423,7 +445,7 @@ def _fwd_x3_op(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, lens: torch.Te
                ) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
     B, H, T, d = q.shape
     Dp = X3_HEAD_DIMS[d]
-    qx, kx, vx = _x3(q, "hhl", Dp), _x3(k, "hlh", Dp), _x3(v, "hlh", Dp)
+    qx, kx, vx = _x3_packed((q, k, v), ("hhl", "hlh", "hlh"), B, H, T, d, Dp)
     plan = plan_in if plan_in is not None else build_plan(B, T, Dp, q.device, mode, in_span, span_id, is_prefix, lens)
     ox = torch.empty((B, H, T, Dp), dtype=torch.bfloat16, device=q.device)
     ox_lo = torch.empty_like(ox)
@@ -432,9 +454,11 @@ def _fwd_x3_op(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, lens: torch.Te
     a.o, a.o_strides = ox.data_ptr(), _strides3(ox)
     a.lse = lse.data_ptr()
     a.o_lo = ox_lo.data_ptr()
-    _lib.check(_lib.load().kd_attn_fwd(ctypes.byref(a), *_lib.plan_ref(plan), _stream(q.device)), "kd_attn_fwd")
+    lib = _lib.load()
+    ws = _workspace(lib.kd_attn_fwd_ws_bytes(ctypes.byref(a)), q.device)
+    _lib.check(lib.kd_attn_fwd_ws(ctypes.byref(a), *_lib.plan_ref(plan), *_ws_ref(ws), _stream(q.device)), "kd_attn_fwd")
     o = _new_out(B, H, T, d, q, bthd)
-    o.copy_(_hi_lo(ox, ox_lo, d, 1))
+    _x3_call(False, [(ox, ox_lo, o, 1)], B, H, T, d, Dp)
     return o, lse, (plan if plan_in is None else plan.new_empty(0))
 
 
@@ -453,17 +477,18 @@ def _bwd_x3_op(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: torch.Tenso
                ) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
     B, H, T, d = q.shape
     Dp = X3_HEAD_DIMS[d]
-    qx, kx, vx, dox = _x3(q, "hhl", Dp), _x3(k, "hlh", Dp), _x3(v, "hlh", Dp), _x3(do, "hhl", Dp)
+    qx, kx, vx, dox = _x3_packed((q, k, v, do), ("hhl", "hlh", "hlh", "hhl"), B, H, T, d, Dp)
+    lib, st = _lib.load(), _stream(q.device)
     # the workspace of kd_attn_bwd_dq / kd_attn_bwd_dkdv (kd_attn_args.delta):
-    # -Delta with Delta = rowsum(dO O) in fp32, then -LSE / c (-inf where LSE is)
+    # -Delta with Delta = rowsum(dO O) in fp32, then -LSE / c (-inf where LSE is),
+    # from the fp32 O and dO
     ws = torch.empty((2, B, H, T), dtype=torch.float32, device=q.device)
-    torch.sum(do.to(torch.float32) * o.to(torch.float32), dim=-1, out=ws[0]).neg_()
-    # -1/c as the kernels form it, in fp32 on the host: a Python float (exactly that
-    # fp32 value) enters the product as a scalar, with no host-to-device copy, so the
-    # op stays capturable in a HIP graph
-    neg_inv_c = -float(np.float32(1.0) / (np.float32(sm_scale) * np.float32(LOG2E)))
-    ninf = torch.full_like(lse, -math.inf)
-    torch.where(lse == -math.inf, ninf, lse * neg_inv_c, out=ws[1])
+    o, do = _kernel_ready(o), _kernel_ready(do)
+    f = _attn_args(o, o, o, sm_scale)
+    f.o, f.o_strides = o.data_ptr(), _strides3(o)
+    f.dout, f.do_strides = do.data_ptr(), _strides3(do)
+    f.lse, f.delta = lse.data_ptr(), ws.data_ptr()
+    _lib.check(lib.kd_attn_bwd_delta(ctypes.byref(f), st), "kd_attn_bwd_delta")
     outs = [torch.empty((B, H, T, Dp), dtype=torch.bfloat16, device=q.device) for _ in range(6)]
     dqx, dkx, dvx, dq_lo, dk_lo, dv_lo = outs
     a = _attn_args(qx, kx, vx, sm_scale, _lib.KD_PREC_SPLIT)
@@ -473,10 +498,11 @@ def _bwd_x3_op(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: torch.Tenso
     a.dq_strides, a.dk_strides, a.dv_strides = _strides3(dqx), _strides3(dkx), _strides3(dvx)
     a.dq_lo, a.dk_lo, a.dv_lo = dq_lo.data_ptr(), dk_lo.data_ptr(), dv_lo.data_ptr()
     a.delta = ws.data_ptr()
-    lib, st = _lib.load(), _stream(q.device)
     _lib.check(lib.kd_attn_bwd_dq(ctypes.byref(a), *_lib.plan_ref(plan), st), "kd_attn_bwd_dq")
     _lib.check(lib.kd_attn_bwd_dkdv(ctypes.byref(a), *_lib.plan_ref(plan), st), "kd_attn_bwd_dkdv")
-    return _hi_lo(dqx, dq_lo, d, 1), _hi_lo(dkx, dk_lo, d, 2), _hi_lo(dvx, dv_lo, d, 2)
+    grads = [torch.empty((B, H, T, d), dtype=torch.float32, device=q.device) for _ in range(3)]
+    _x3_call(False, [(hi, lo, g, s) for hi, lo, g, s in zip(outs[:3], outs[3:], grads, (1, 2, 2))], B, H, T, d, Dp)
+    return tuple(grads)
 
 
 @_bwd_x3_op.register_fake
@@ -654,8 +680,14 @@ def flash_attention(
 
     if x3:
         # fp32 at the reference's default precision: bf16x3 on the MFMA kernels
-        o, lse, plan_t = _fwd_x3_op(q, k, v, lens, in_span, span_id, is_prefix, float(sm_scale), int(mode),
-                                    bthd=out_layout == "bthd", plan_in=None if plan is None else plan.tensor)
+        bthd, plan_in, got = out_layout == "bthd", None if plan is None else plan.tensor, None
+        if _lib.eager(q, k, v, lens, in_span, span_id, is_prefix, plan_in):
+            got = _lib.native().flash_x3(q, k, v, lens, in_span, span_id, is_prefix, float(sm_scale), int(mode), bthd,
+                                         plan_in)
+        if got is None:
+            got = _fwd_x3_op(q, k, v, lens, in_span, span_id, is_prefix, float(sm_scale), int(mode), bthd=bthd,
+                             plan_in=plan_in)
+        o, lse, plan_t = got
     else:
         # O's rounding residual, kept for the backward's Delta (16-bit O only)
         need_lo = (q.dtype != torch.float32 and torch.is_grad_enabled()

@@ -141,6 +141,42 @@ void kd_struct_sizes4(size_t* span) {
   if (span) *span = sizeof(kd_span_args);
 }
 
+void kd_struct_sizes5(size_t* x3) {
+  if (x3) *x3 = sizeof(kd_x3_args);
+}
+
+static int check_x3(const kd_x3_args* a, bool pack) {
+  if (a == nullptr) return fail(KD_ERR_INVALID, "args is NULL");
+  if (a->n < 1 || a->n > 4) return fail(KD_ERR_INVALID, "n must be in 1 .. 4");
+  if (a->B < 1 || a->H < 1 || a->T < 1) return fail(KD_ERR_INVALID, "B, H and T must be >= 1");
+  if (a->d != 16 && a->d != 32 && a->d != 64) return fail(KD_ERR_UNSUPPORTED, "d must be 16, 32 or 64");
+  if (a->Dp < 3 * a->d || a->Dp > 256 || a->Dp % 8 != 0) return fail(KD_ERR_INVALID, "Dp must hold three rows of d");
+  if (int64_t(a->B) * a->H * a->T > (int64_t(1) << 33)) return fail(KD_ERR_UNSUPPORTED, "too many rows");
+  for (int i = 0; i < a->n; ++i) {
+    const void* f32 = pack ? a->src[i] : a->dst[i];
+    const int64_t* st = pack ? a->src_strides[i] : a->dst_strides[i];
+    if (int r = check_tensor(f32, st, "the fp32 tensor", 1, a->d, 4)) return r;
+    for (const void* p : {pack ? static_cast<const void*>(a->dst[i]) : a->src[i], pack ? f32 : a->lo[i]})
+      if (p == nullptr || !aligned16(p)) return fail(KD_ERR_INVALID, "operands must be given and 16-byte aligned");
+    if (a->sel[i] < (pack ? 0 : 1) || a->sel[i] > (pack ? 1 : 2)) return fail(KD_ERR_INVALID, "bad sel");
+  }
+  return KD_OK;
+}
+
+int kd_x3_pack(const kd_x3_args* a, void* stream) {
+  int r = check_x3(a, true);
+  if (r) return r;
+  r = kd::launch_x3(*a, true, as_stream(stream));
+  return r ? fail(r, "kernel launch failed (x3 pack)") : KD_OK;
+}
+
+int kd_x3_unpack(const kd_x3_args* a, void* stream) {
+  int r = check_x3(a, false);
+  if (r) return r;
+  r = kd::launch_x3(*a, false, as_stream(stream));
+  return r ? fail(r, "kernel launch failed (x3 unpack)") : KD_OK;
+}
+
 static int check_rms(int64_t rows, int32_t D, int32_t dtype) {
   if (rows < 1 || rows > (int64_t(1) << 32)) return fail(KD_ERR_INVALID, "rows must be in 1 .. 2^32");
   if (D < 8 || D > 2048 || D % 8 != 0) return fail(KD_ERR_UNSUPPORTED, "D must be a multiple of 8 in 8 .. 2048");

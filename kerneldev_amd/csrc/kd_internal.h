@@ -73,6 +73,7 @@ int launch_dkdv(const AttnArgs& a, const uint8_t* plan, float* ws, hipStream_t s
 int launch_hadamard(const kd_rot_args& a, hipStream_t st);
 int launch_quant(const kd_quant_args& a, hipStream_t st);
 int launch_absmax(const kd_quant_args& a, float* amax, hipStream_t st);
+int launch_x3(const kd_x3_args& a, bool pack, hipStream_t st);
 int wgrad_pieces(int M, int N, int K);
 int launch_wgrad(const void* dy, const void* x, void* dw, float* part, int M, int N, int K, int dtype, hipStream_t st);
 int launch_rms_fwd(const void* x, void* y, float* rstd, int64_t rows, int D, int dtype, float eps, hipStream_t st);

@@ -118,8 +118,10 @@ struct Meta {
   OptTensor lens, in_span, span_id, is_prefix;
 };
 
-Tensor plan_of(int64_t B, int64_t T, int64_t D, c10::Device on, int64_t mode, const Meta& x) {
-  Tensor plan = bytes_on(on, plan_size(B, T, D), true);
+// clean: zero where the build writes nothing (an op's output carries no stale
+// bytes; a call's own plan need not be cleared, 3 us of a small step)
+Tensor plan_of(int64_t B, int64_t T, int64_t D, c10::Device on, int64_t mode, const Meta& x, bool clean = false) {
+  Tensor plan = bytes_on(on, plan_size(B, T, D), clean);
   kd_meta_args m{};
   m.B = int32_t(B), m.T = int32_t(T), m.D = int32_t(D), m.mode = int32_t(mode);
   auto two = [](int64_t (&to)[2], const Tensor& t) { to[0] = t.stride(0), to[1] = t.stride(1); };
@@ -296,6 +298,131 @@ struct Attention : torch::autograd::Function<Attention> {
   }
 };
 
+// kdattn::fwd_x3 and kdattn::bwd_x3 as one C++ node: fp32 operands of head dim 16
+// or 32 as packed bf16 ones of 64 or 128 (attention.X3_HEAD_DIMS)
+struct AttentionX3 : torch::autograd::Function<AttentionX3> {
+  static int64_t packed_dim(int64_t d) { return d == 16 ? 64 : 128; }
+  static kd_x3_args x3_args(const Tensor& q, int64_t Dp) {
+    kd_x3_args a{};
+    a.B = int32_t(q.size(0)), a.H = int32_t(q.size(1)), a.T = int32_t(q.size(2)), a.d = int32_t(q.size(3));
+    a.Dp = int32_t(Dp);
+    return a;
+  }
+  static Tensor wide(const Tensor& q, int64_t Dp) {
+    return at::empty({q.size(0), q.size(1), q.size(2), Dp}, q.options().dtype(at::kBFloat16));
+  }
+  static variable_list pack(const variable_list& xs, std::initializer_list<int> sel, int64_t Dp) {
+    kd_x3_args a = x3_args(xs[0], Dp);
+    variable_list keep, out;
+    for (const int s : sel) {
+      const int i = a.n++;
+      keep.push_back(kernel_ready(xs[i])), out.push_back(wide(xs[i], Dp));
+      a.src[i] = keep[i].data_ptr(), a.dst[i] = out[i].data_ptr(), a.sel[i] = s;
+      set3(a.src_strides[i], keep[i]);
+    }
+    check(kd_x3_pack(&a, stream_of(xs[0])), "kd_x3_pack");
+    return out;
+  }
+  static void unpack(const variable_list& hi, const variable_list& lo, const variable_list& out,
+                     std::initializer_list<int> sel) {
+    kd_x3_args a = x3_args(out[0], hi[0].size(3));
+    for (const int s : sel) {
+      const int i = a.n++;
+      a.src[i] = hi[i].data_ptr(), a.lo[i] = lo[i].data_ptr(), a.dst[i] = out[i].data_ptr(), a.sel[i] = s;
+      set3(a.dst_strides[i], out[i]);
+    }
+    check(kd_x3_unpack(&a, stream_of(out[0])), "kd_x3_unpack");
+  }
+
+  static variable_list forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v,
+                               const AttnOpts& x) {
+    RECORD_FUNCTION("kdattn::fwd_x3", std::vector<c10::IValue>());
+    const c10::DeviceGuard on(q.device());
+    const int64_t B = q.size(0), H = q.size(1), T = q.size(2), d = q.size(3), Dp = packed_dim(d);
+    const variable_list p = pack({q, k, v}, {0, 1, 1}, Dp);
+    const Tensor plan = x.plan ? *x.plan : plan_of(B, T, Dp, q.device(), x.mode, x.meta);
+    *x.built = plan;
+    const Tensor ox = wide(q, Dp), lo = wide(q, Dp);
+    Tensor lse = at::empty({B, H, T}, q.options());
+    kd_attn_args a = attn_args(p[0], p[1], p[2], x.sm_scale, KD_PREC_SPLIT);
+    a.o = ox.data_ptr();
+    set3(a.o_strides, ox);
+    a.lse = static_cast<float*>(lse.data_ptr());
+    a.o_lo = lo.data_ptr();
+    const int64_t need = kd_attn_fwd_ws_bytes(&a);
+    const Tensor ws = need > 0 ? bytes_on(q.device(), need, false) : Tensor();
+    check(kd_attn_fwd_ws(&a, plan.data_ptr(), plan.numel(), need > 0 ? ws.data_ptr() : nullptr, need, stream_of(q)),
+          "kd_attn_fwd");
+    Tensor o = x.bthd ? at::empty_strided({B, H, T, d}, {T * H * d, d, H * d, 1}, q.options())
+                      : at::empty({B, H, T, d}, q.options());
+    unpack({ox}, {lo}, {o}, {1});
+    ctx->save_for_backward({q, k, v, o, lse, plan});
+    ctx->set_materialize_grads(false);  // (LSE's gradient is ignored)
+    ctx->saved_data["sm_scale"] = x.sm_scale;
+    return {o, lse};
+  }
+
+  static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
+    variable_list out(4);
+    if (!grads[0].defined()) return out;  // only LSE reached the loss
+    RECORD_FUNCTION("kdattn::bwd_x3", std::vector<c10::IValue>());
+    const variable_list s = ctx->get_saved_variables();
+    bool differentiable = false;
+    if (at::GradMode::is_enabled())
+      for (const Tensor& t : {s[0], s[1], s[2], s[3], s[4], grads[0]}) differentiable |= t.requires_grad();
+    variable_list g(3);
+    {
+      at::AutoDispatchBelowADInplaceOrView below;
+      const Tensor& q = s[0];
+      const c10::DeviceGuard on(q.device());
+      const int64_t B = q.size(0), H = q.size(1), T = q.size(2), d = q.size(3), Dp = packed_dim(d);
+      const double sm_scale = ctx->saved_data["sm_scale"].toDouble();
+      Tensor d_o = grads[0];
+      if (d_o.is_neg()) d_o = d_o.resolve_neg();
+      if (d_o._is_zerotensor()) d_o = at::zeros(d_o.sizes(), s[3].options());
+      d_o = kernel_ready(d_o);
+      const Tensor o = kernel_ready(s[3]);
+      const Tensor &lse = s[4], &plan = s[5];
+      const variable_list p = pack({q, s[1], s[2], d_o}, {0, 1, 1, 0}, Dp);
+      const Tensor delta = at::empty({2, B, H, T}, q.options());
+      kd_attn_args f = attn_args(o, o, o, sm_scale, KD_PREC_SPLIT);  // -Delta and -LSE / c from the fp32 O and dO
+      f.o = o.data_ptr(), f.dout = d_o.data_ptr();
+      set3(f.o_strides, o), set3(f.do_strides, d_o);
+      f.lse = static_cast<float*>(lse.data_ptr()), f.delta = static_cast<float*>(delta.data_ptr());
+      check(kd_attn_bwd_delta(&f, stream_of(q)), "kd_attn_bwd_delta");
+      variable_list hi, lo;
+      for (int i = 0; i < 3; ++i)
+        hi.push_back(wide(q, Dp)), lo.push_back(wide(q, Dp)), g[i] = at::empty({B, H, T, d}, q.options());
+      kd_attn_args a = attn_args(p[0], p[1], p[2], sm_scale, KD_PREC_SPLIT);
+      a.lse = f.lse, a.delta = f.delta;
+      a.dout = p[3].data_ptr();
+      set3(a.do_strides, p[3]);
+      a.dq = hi[0].data_ptr(), a.dk = hi[1].data_ptr(), a.dv = hi[2].data_ptr();
+      set3(a.dq_strides, hi[0]), set3(a.dk_strides, hi[1]), set3(a.dv_strides, hi[2]);
+      a.dq_lo = lo[0].data_ptr(), a.dk_lo = lo[1].data_ptr(), a.dv_lo = lo[2].data_ptr();
+      check(kd_attn_bwd_dq(&a, plan.data_ptr(), plan.numel(), stream_of(q)), "kd_attn_bwd_dq");
+      check(kd_attn_bwd_dkdv(&a, plan.data_ptr(), plan.numel(), stream_of(q)), "kd_attn_bwd_dkdv");
+      unpack(hi, lo, g, {1, 2, 2});
+    }
+    if (differentiable) refuse_second(g, "kdattn.bwd_x3.default", {s[0], s[1], s[2], s[3], s[4], grads[0]});
+    for (int i = 0; i < 3; ++i) out[i] = g[i];
+    return out;
+  }
+};
+
+pybind11::object flash_x3(const Tensor& q, const Tensor& k, const Tensor& v, const OptTensor& lens,
+                          const OptTensor& in_span, const OptTensor& span_id, const OptTensor& is_prefix,
+                          double sm_scale, int64_t mode, bool bthd, const OptTensor& plan) {
+  if (!plain_mode() || !plain(q) || !plain(k) || !plain(v) || !plain(lens) || !plain(in_span) || !plain(span_id) ||
+      !plain(is_prefix) || !plain(plan) || q.scalar_type() != at::kFloat || k.scalar_type() != at::kFloat ||
+      v.scalar_type() != at::kFloat || q.numel() == 0 || (q.size(3) != 16 && q.size(3) != 32))
+    return pybind11::none();
+  Tensor used;
+  const AttnOpts x{{lens, in_span, span_id, is_prefix}, plan, {}, sm_scale, mode, KD_PREC_SPLIT, false, bthd, false, &used};
+  const variable_list r = AttentionX3::apply(q, k, v, x);
+  return pybind11::make_tuple(r[0], r[1], used);
+}
+
 // (o, lse, plan), or None where the call is not a plain eager one
 pybind11::object flash(const Tensor& q, const Tensor& k, const Tensor& v, const OptTensor& lens, const OptTensor& in_span,
                        const OptTensor& span_id, const OptTensor& is_prefix, double sm_scale, int64_t mode, bool need_lo,
@@ -315,7 +442,7 @@ pybind11::object plan_from_metadata(int64_t B, int64_t T, int64_t D, int64_t mod
   if (!plain_mode() || !on.is_cuda() || !plain(lens) || !plain(in_span) || !plain(span_id) || !plain(is_prefix))
     return pybind11::none();
   const c10::DeviceGuard guard(on);
-  return pybind11::cast(plan_of(B, T, D, on, mode, Meta{lens, in_span, span_id, is_prefix}));
+  return pybind11::cast(plan_of(B, T, D, on, mode, Meta{lens, in_span, span_id, is_prefix}, true));
 }
 
 pybind11::object plan_from_tokens(const Tensor& tokens, int64_t D, int64_t rule, const OptTensor& lens) {
@@ -576,6 +703,7 @@ pybind11::object span_counts(const Tensor& tokens) {
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("set_kernel_error", [](pybind11::object e) { g_kernel_error = e.release().ptr(); });
   m.def("flash", torch::wrap_pybind_function(flash));
+  m.def("flash_x3", torch::wrap_pybind_function(flash_x3));
   m.def("plan_from_metadata", torch::wrap_pybind_function(plan_from_metadata));
   m.def("plan_from_tokens", torch::wrap_pybind_function(plan_from_tokens));
   m.def("projection", torch::wrap_pybind_function(projection));

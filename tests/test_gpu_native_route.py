@@ -29,6 +29,8 @@ CASES = [
     (2, 2, 200, 64, torch.bfloat16, dict(precision="ieee", causal=False)),
     (1, 2, 129, 32, torch.float32, dict(precision="ieee")),
     (2, 4, 256, 16, torch.float16, {}),
+    (2, 2, 300, 32, torch.float32, {}),
+    (1, 1, 1100, 16, torch.float32, dict(out_layout="bthd")),
 ]
 
 
