@@ -1404,8 +1404,7 @@ int launch_delta(const AttnArgs& a, hipStream_t st) {
 int launch_dq(const AttnArgs& a, const uint8_t* plan, float* ws, hipStream_t st, bool fuse_delta) {
   const SplitArgs sp{ws, ws == nullptr ? 1 : split_pieces(a, SPLIT_DQ)};
   if (use_simt(a)) {
-    int r = fuse_delta ? launch_simt_kernel(1, a, plan, sp, st) : KD_OK;
-    if (!r) r = launch_simt_kernel(2, a, plan, sp, st);
+    const int r = launch_simt_kernel(2, a, plan, sp, st, fuse_delta);
     return r || sp.ns == 1 ? r : launch_combine_dq(a, sp, st);
   }
   if (a.q8 != nullptr) {  // fp8 QK^T: bf16 at head dim 64, 128 or 256 (checked by the C ABI)

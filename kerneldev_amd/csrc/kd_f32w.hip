@@ -8,7 +8,8 @@
 //   dQ        P = exp2(S c - LSE), dS = P (dP - Delta), dQ = sm_scale dS K  (:1173-1336)
 //   dK / dV   dV = P^T dO, dK = sm_scale dS^T Q            (:1339-1525)
 // with c = sm_scale log2(e) folded into the register-resident Q (forward, dQ)
-// or K (dK/dV).  Delta comes from k_delta_simt (kd_simt.hip).
+// or K (dK/dV).  Delta comes from k_delta_simt (kd_simt.hip) or, in a whole
+// backward, from the dQ kernel itself.
 //
 // Why a 16 x 16 product.  With 32 tokens per wave (the 32 x 32 x 2 form,
 // which these kernels replaced) a lane holds WD / 2 floats of each register
@@ -367,7 +368,7 @@ __global__ __launch_bounds__(256, Geo<WD>::WAVES) void k_fwd_f32w(AttnArgs a, co
 
 // ----------------------------------------------------------------------- dQ
 template <int WD>
-__global__ __launch_bounds__(256, Geo<WD>::WAVES) void k_dq_f32w(AttnArgs a, const uint32_t* __restrict__ codes,
+__global__ __launch_bounds__(256, Geo<WD>::WAVES) void k_dq_f32w(AttnArgs a, bool fuse_delta, const uint32_t* __restrict__ codes,
                                                     const uint32_t* __restrict__ list,
                                                     const int32_t* __restrict__ count, int nT, int nblk,
                                                     const uint32_t* __restrict__ order, SplitArgs sp) {
@@ -396,11 +397,28 @@ __global__ __launch_bounds__(256, Geo<WD>::WAVES) void k_dq_f32w(AttnArgs a, con
   // P = exp2(S c - LSE); a fully masked row (LSE = -inf) gets P = 0
   const float l0 = qvalid ? a.lse[int64_t(bh) * T + q] : -__builtin_inff();
   float lse = l0 == -__builtin_inff() ? __builtin_inff() : l0;
-  float ndelta = qvalid ? a.delta[int64_t(bh) * T + q] : 0.f;  // the workspace holds -Delta
+  float ndelta = qvalid && !fuse_delta ? a.delta[int64_t(bh) * T + q] : 0.f;  // the workspace holds -Delta
 
   float qr[NR], dr[NR];
-  load_row16<WD>(qg, a.q_strides[2], q, qvalid, g, cs, qr, a.D);
   load_row16<WD>(dog, a.do_strides[2], q, qvalid, g, 1.f, dr, a.D);
+  if (fuse_delta) {
+    // -Delta = -rowsum(O dO) of this lane's query, from the dO row already
+    // held (the four lane groups hold a quarter each), and stored with
+    // -LSE / c for dK/dV: k_delta_simt's work without its launch and its
+    // second reading of dO.  (Pieces of one row store the same values.)
+    float o[NR], sum = 0.f;  // (o's registers are qr's: it is loaded below)
+    load_row16<WD>(static_cast<const float*>(a.o) + it.b * a.o_strides[0] + it.hh * a.o_strides[1], a.o_strides[2], q,
+                   qvalid, g, 1.f, o, a.D);
+#pragma unroll
+    for (int j = 0; j < NR; ++j) sum = __builtin_fmaf(o[j], dr[j], sum);
+    ndelta = -group_sum(sum);
+    if (qvalid && g == 0) {
+      const int64_t row = int64_t(bh) * T + q;
+      a.delta[row] = ndelta;
+      a.delta[int64_t(a.B) * a.H * T + row] = l0 == -__builtin_inff() ? -__builtin_inff() : -l0 / cs;
+    }
+  }
+  load_row16<WD>(qg, a.q_strides[2], q, qvalid, g, cs, qr, a.D);
 
   const int lb = it.b * nblk + it.blk;
   int n = count[lb];
@@ -592,7 +610,7 @@ __global__ __launch_bounds__(256, Geo<WD>::WAVES) void k_dkdv_f32w(AttnArgs a, c
 }
 
 template <int WD>
-void launch_f32w_d(int which, const AttnArgs& a, const uint8_t* plan, const SplitArgs& sp, hipStream_t st) {
+void launch_f32w_d(int which, bool fuse_delta, const AttnArgs& a, const uint8_t* plan, const SplitArgs& sp, hipStream_t st) {
   const PlanLayout L = plan_layout(a.B, a.T, a.D);
   const uint32_t* codes = reinterpret_cast<const uint32_t*>(plan + L.codes);
   auto lst = [&](size_t off) { return reinterpret_cast<const uint32_t*>(plan + off); };
@@ -602,7 +620,7 @@ void launch_f32w_d(int which, const AttnArgs& a, const uint8_t* plan, const Spli
     hipLaunchKernelGGL(k_fwd_f32w<WD>, dim3(bh2 * unsigned(L.n_fwd_blocks)), dim3(256), 0, st, a, codes,
                        lst(L.fwd_list), cnt(L.fwd_count), L.nT, L.n_fwd_blocks, lst(L.fwd_order), sp);
   else if (which == 2)
-    hipLaunchKernelGGL(k_dq_f32w<WD>, dim3(bh2 * unsigned(L.n_dq_blocks)), dim3(256), 0, st, a, codes,
+    hipLaunchKernelGGL(k_dq_f32w<WD>, dim3(bh2 * unsigned(L.n_dq_blocks)), dim3(256), 0, st, a, fuse_delta, codes,
                        lst(L.dq_list), cnt(L.dq_count), L.nT, L.n_dq_blocks, lst(L.dq_order), sp);
   else
     hipLaunchKernelGGL(k_dkdv_f32w<WD>, dim3(bh2 * unsigned(L.n_dkdv_blocks)), dim3(256), 0, st, a, codes,
@@ -611,13 +629,13 @@ void launch_f32w_d(int which, const AttnArgs& a, const uint8_t* plan, const Spli
 
 }  // namespace
 
-int launch_f32mma(int which, const AttnArgs& a, const uint8_t* plan, const SplitArgs& sp, hipStream_t st) {
+int launch_f32mma(int which, bool fuse_delta, const AttnArgs& a, const uint8_t* plan, const SplitArgs& sp, hipStream_t st) {
   switch (a.D) {
     case 16:  // on the WD = 32 kernels: columns 16-31 read as zeros, not stored
-    case 32: launch_f32w_d<32>(which, a, plan, sp, st); break;
-    case 64: launch_f32w_d<64>(which, a, plan, sp, st); break;
-    case 128: launch_f32w_d<128>(which, a, plan, sp, st); break;
-    default: launch_f32w_d<256>(which, a, plan, sp, st); break;
+    case 32: launch_f32w_d<32>(which, fuse_delta, a, plan, sp, st); break;
+    case 64: launch_f32w_d<64>(which, fuse_delta, a, plan, sp, st); break;
+    case 128: launch_f32w_d<128>(which, fuse_delta, a, plan, sp, st); break;
+    default: launch_f32w_d<256>(which, fuse_delta, a, plan, sp, st); break;
   }
   return hipGetLastError() == hipSuccess ? KD_OK : KD_ERR_LAUNCH;
 }

@@ -89,10 +89,11 @@ int launch_span_bwd(const kd_span_args& a, hipStream_t st);
 // fp32 inputs (kd_simt.hip): Delta on the vector ALUs and the fp32 MFMA
 // kernels; which: 0 forward, 1 Delta, 2 dQ, 3 dK/dV
 bool use_simt(const AttnArgs& a);
-int launch_simt_kernel(int which, const AttnArgs& a, const uint8_t* plan, const SplitArgs& sp, hipStream_t st);
+int launch_simt_kernel(int which, const AttnArgs& a, const uint8_t* plan, const SplitArgs& sp, hipStream_t st,
+                       bool fuse_delta = false);
 // fp32 attention at head dims 16 (on the 32 kernels), 32, 64, 128, 256 on the
 // fp32 MFMA (kd_f32w.hip); which: 0 forward, 2 dQ, 3 dK/dV
-int launch_f32mma(int which, const AttnArgs& a, const uint8_t* plan, const SplitArgs& sp, hipStream_t st);
+int launch_f32mma(int which, bool fuse_delta, const AttnArgs& a, const uint8_t* plan, const SplitArgs& sp, hipStream_t st);
 // Device address of the no-allocation workspace on the current device
 // (kd_noalloc.hip); KD_OK, or a status with *err set.
 int noalloc_workspace(float** out, const char** err);

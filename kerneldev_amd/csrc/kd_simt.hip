@@ -67,8 +67,9 @@ static void launch_delta_f32(const AttnArgs& a, hipStream_t st) {
 bool use_simt(const AttnArgs& a) { return a.dtype == KD_F32; }
 
 // which: 0 forward, 1 Delta, 2 dQ, 3 dK/dV
-int launch_simt_kernel(int which, const AttnArgs& a, const uint8_t* plan, const SplitArgs& sp, hipStream_t st) {
-  if (which != 1) return launch_f32mma(which, a, plan, sp, st);
+int launch_simt_kernel(int which, const AttnArgs& a, const uint8_t* plan, const SplitArgs& sp, hipStream_t st,
+                       bool fuse_delta) {
+  if (which != 1) return launch_f32mma(which, fuse_delta, a, plan, sp, st);
   switch (a.D) {
     case 16: launch_delta_f32<16>(a, st); break;
     case 32: launch_delta_f32<32>(a, st); break;
