@@ -31,8 +31,8 @@ from ._lib import AttnArgs, MetaArgs
 REFERENCE_HEAD_DIMS = (16, 32, 64, 128, 256)  # original_kernel.py:1720
 SUPPORTED_HEAD_DIMS = REFERENCE_HEAD_DIMS
 # bf16 / fp16 at these head dims run on the MFMA kernels with the fused
-# Hadamard epilogues; 16, 32 and 256 run there without them (16 and 32 on
-# the d = 64 kernels, which read the missing columns as zeros).  fp8 scores
+# Hadamard epilogues; 16, 32 and 256 run there without them (16 on
+# the d = 32 kernels, which read the missing columns as zeros).  fp8 scores
 # are built at 64, 128 and 256.  fp32
 # inputs run on the fp32 MFMA kernels at every head dim (kd_f32w.hip; 16 on
 # the d = 32 kernels, which read the missing columns as zeros), except at
@@ -533,7 +533,7 @@ def head_dim_route(dtype: torch.dtype, D: int, precision: str) -> bool:
     """Whether flash_attention runs inputs of this dtype, head dim and precision
     on the bf16x3 ops (fp32 at "tf32" and d = 16, 32); everything else goes to
     the C ABI's kernels as it is, with no padding: 16-bit inputs on the MFMA
-    kernels at every head dim (d = 16, 32 on the d = 64 kernels, which read the
+    kernels at every head dim (d = 16 on the d = 32 kernels, which read the
     missing columns as zeros), fp32 on the fp32 MFMA kernels (d = 16 on the
     d = 32 ones, the same way)."""
     return dtype == torch.float32 and precision == "tf32" and D in X3_ROUTED_HEAD_DIMS

@@ -102,8 +102,8 @@ __global__ __launch_bounds__(256) void k_delta(AttnArgs a) {
 // also each value's rounding residual at the same offsets of glo (the
 // caller's contiguous residual row), so that g + glo carries the fp32 value to
 // about twice the type's significant bits
-// dlim: columns from there on are not stored (head dims 16 and 32 on the
-// D = 64 kernels).  lo32: glo holds fp32 residuals (precision KD_PREC_SPLIT3),
+// dlim: columns from there on are not stored (head dim 16 on the D = 32
+// kernels).  lo32: glo holds fp32 residuals (precision KD_PREC_SPLIT3),
 // so that g + glo is the fp32 value.
 template <class E, int D>
 KD_DEV void store_rows_T(uint16_t* g, const f32x16 (&acc)[D / 32], float scale, int hf, void* glo = nullptr,
@@ -206,7 +206,7 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void k_dq(AttnArgs a, const 
   constexpr bool SP = NSP >= 2, S3 = NSP == 3;
   using TL = Tile<D>;
   using SO = ScoreOp<E, D, Q8>;  // S^T = K Q^T (16-bit, or fp8 from the K8 tile)
-  using TK8 = typename ScoreOp<E, D, true>::TL;
+  using TK8 = typename ScoreOp<E, Q8 ? D : 64, true>::TL;  // (unused without Q8, which is built from D = 64 on)
   // fp8 scores (Q8) take S from the K8 tile, so the 16-bit K tile feeds only
   // dQ^T += K^T dS^T, i.e. only this launch's columns [D0, D0 + DH): it is
   // loaded DH wide (KHALF), which keeps the d = 256 launch's two slots of K,
@@ -253,8 +253,8 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void k_dq(AttnArgs a, const 
   const int qrow = qblock * 128 + wave * 32 + c;
   const bool qvalid = qrow < T;
   SO so;  // B operand: this lane's query row (Q, or its fp8 copy)
-  // bytes of a row of the 16-bit inputs: 2 D, or fewer for head dims 16 and
-  // 32 on the D = 64 kernel, whose other columns are read as zeros
+  // bytes of a row of the 16-bit inputs: 2 D, or fewer for head dim 16 on the
+  // D = 32 kernel, whose other columns are read as zeros
   const uint32_t dbytes = uint32_t(a.D) * 2u;
   if constexpr (Q8) so.load_b(make_rsrc(a.q8 + int64_t(bh) * T * D, uint32_t(T) * D), uint32_t(qrow) * D, hf);
   else so.load_b(rs_q, uint32_t(qrow) * qrb, hf, dbytes);
@@ -527,7 +527,7 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void k_dq(AttnArgs a, const 
     uint16_t* g = static_cast<uint16_t*>(a.dq) + b * a.dq_strides[0] + h * a.dq_strides[1] + qrow * a.dq_strides[2];
     void* glo = lo_row(a.dq_lo, (int64_t(b) * a.H + h) * a.T + qrow, a.D, S3);
     if constexpr (DH == D) {
-      if (a.dqk_signs != nullptr) store_rows_T_unrot<E, D>(g, acc, a.sm_scale, hf, a.dqk_signs);
+      if (D >= 64 && a.dqk_signs != nullptr) store_rows_T_unrot<E, D>(g, acc, a.sm_scale, hf, a.dqk_signs);
       else store_rows_T<E, D>(g, acc, a.sm_scale, hf, glo, a.D, S3);
     } else {  // (no dqk_signs at split widths)
       void* glo_h = glo == nullptr ? nullptr : static_cast<void*>(static_cast<uint8_t*>(glo) + D0 * (S3 ? 4 : 2));
@@ -1035,8 +1035,8 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void k_dkdv_wide(AttnArgs a, 
 
   const int krow = kblock * 128 + wave * 32 + c;
   const bool kvalid = krow < T;
-  // bytes of a row of the 16-bit inputs: 2 D, or fewer for head dims 16 and
-  // 32 on the D = 64 kernel, whose other columns are read as zeros
+  // bytes of a row of the 16-bit inputs: 2 D, or fewer for head dim 16 on the
+  // D = 32 kernel, whose other columns are read as zeros
   const uint32_t dbytes = uint32_t(a.D) * 2u;
   u32x4 bk[Q8 ? 1 : DS], bv[DS];  // this lane's K and V rows (B operands of S^T, dP^T)
   i32x8 bk8[Q8 ? D / 64 : 1];      // fp8: its K8 row instead, k-step st = bytes 64 st + 32 hf .. + 31
@@ -1285,10 +1285,10 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void k_dkdv_wide(AttnArgs a, 
     };
     void* gv_lo = lo_at(a.dv_lo);
     void* gk_lo = lo_at(a.dk_lo);
-    // (a.D < D only for the head dims 16 and 32 on the D = 64 launch, DH == D)
+    // (a.D < D only for head dim 16 on the D = 32 launch, DH == D)
     store_rows_T<E, DH>(gv + D0, acc_v, 1.f, hf, gv_lo, DH == D ? a.D : DH, S3);
     if constexpr (DH == D) {  // all columns here: dK can be rotated back (dqk_signs)
-      if (a.dqk_signs != nullptr) store_rows_T_unrot<E, D>(gk, acc_k, a.sm_scale, hf, a.dqk_signs);
+      if (D >= 64 && a.dqk_signs != nullptr) store_rows_T_unrot<E, D>(gk, acc_k, a.sm_scale, hf, a.dqk_signs);
       else store_rows_T<E, D>(gk, acc_k, a.sm_scale, hf, gk_lo, a.D, S3);
     } else {
       store_rows_T<E, DH>(gk + D0, acc_k, a.sm_scale, hf, gk_lo, DH, S3);  // (no dqk_signs at split widths)
@@ -1335,8 +1335,8 @@ template <class E, int D, bool Q8, int NSP>
 static void launch_dkdv_s(const AttnArgs& a, const uint8_t* plan, const SplitArgs& sp, hipStream_t st) {
   const PlanLayout L = plan_layout(a.B, a.T, a.D);
   const unsigned grid = unsigned(a.B) * a.H * L.n_dkdv_blocks * sp.ns;
-  if constexpr (D == 64) {  // one launch, all four products per wave (fp8 scores too)
-    hipLaunchKernelGGL((k_dkdv_wide<E, D, NSP, 64, 0, Q8>), dim3(grid), dim3(256), 0, st, a,
+  if constexpr (D <= 64) {  // one launch, all four products per wave (fp8 scores too)
+    hipLaunchKernelGGL((k_dkdv_wide<E, D, NSP, D, 0, Q8>), dim3(grid), dim3(256), 0, st, a,
                        reinterpret_cast<const uint32_t*>(plan + L.codes),
                        reinterpret_cast<const uint32_t*>(plan + L.dkdv_list),
                        reinterpret_cast<const int32_t*>(plan + L.dkdv_count),
@@ -1370,15 +1370,21 @@ static void launch_dkdv_t(const AttnArgs& a, const uint8_t* plan, const SplitArg
   }
 }
 
-// head dims 16 and 32 run on the D = 64 kernels (their rows read as zeros past a.D)
+// head dim 16 runs on the D = 32 kernels (its rows read as zeros past a.D).
+// Against the D = 64 kernels, which these two dims ran on before, half of the
+// MFMAs and of the LDS and tile traffic go, and a third wave fits a SIMD: causal
+// bf16 B4 H9 T4538 d32, forward 169 -> 150 us, dQ 235 -> 171, dK/dV 313 -> 228; all
+// keys, B8 H16 T2048 d16, 187 -> 146, 206 -> 148, 298 -> 215.
 #define KD_DISPATCH(FN, ...)                                         \
   do {                                                               \
     if (a.dtype == KD_BF16) {                                        \
-      if (a.D <= 64) FN<BF16, 64>(__VA_ARGS__);                      \
+      if (a.D <= 32) FN<BF16, 32>(__VA_ARGS__);                      \
+      else if (a.D == 64) FN<BF16, 64>(__VA_ARGS__);                 \
       else if (a.D == 128) FN<BF16, 128>(__VA_ARGS__);               \
       else FN<BF16, 256>(__VA_ARGS__);                               \
     } else {                                                         \
-      if (a.D <= 64) FN<F16, 64>(__VA_ARGS__);                       \
+      if (a.D <= 32) FN<F16, 32>(__VA_ARGS__);                       \
+      else if (a.D == 64) FN<F16, 64>(__VA_ARGS__);                  \
       else if (a.D == 128) FN<F16, 128>(__VA_ARGS__);                \
       else FN<F16, 256>(__VA_ARGS__);                                \
     }                                                                \

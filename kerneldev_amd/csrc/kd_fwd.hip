@@ -95,8 +95,8 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void k_fwd(AttnArgs a, const
   const auto rs_q = make_rsrc(qs_base, uint32_t(T) * qrb);
   const u32x4 rs_k = rsrc_words(ks_base, uint32_t(T) * krb);
   const u32x4 rs_v = rsrc_words(vg, uint32_t(T) * vrb);
-  // bytes of a row of the 16-bit inputs: 2 D, or fewer for head dims 16 and
-  // 32 on the D = 64 kernel, whose other columns are read as zeros
+  // bytes of a row of the 16-bit inputs: 2 D, or fewer for head dim 16 on the
+  // D = 32 kernel, whose other columns are read as zeros
   const uint32_t dbytes = uint32_t(a.D) * 2u;
 
   // ---- this lane's query row (the B operand of S^T, kept in registers) ----
@@ -343,7 +343,7 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void k_fwd(AttnArgs a, const
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
           const int d0 = 32 * db + 8 * g + 4 * hf;
-          if (D == 64 && d0 >= a.D) continue;  // head dims 16, 32: only the real columns
+          if (D == 32 && d0 >= a.D) continue;  // head dim 16: only the real columns
           float f[4];
 #pragma unroll
           for (int i = 0; i < 4; ++i) f[i] = o[db][4 * g + i] * inv;
@@ -398,12 +398,14 @@ int launch_fwd(const AttnArgs& a, const uint8_t* plan, float* ws, hipStream_t st
     if (a.D == 64) launch_fwd_p<BF16, 64, true>(a, plan, sp, st);
     else if (a.D == 128) launch_fwd_p<BF16, 128, true>(a, plan, sp, st);
     else launch_fwd_p<BF16, 256, true>(a, plan, sp, st);
-  } else if (a.dtype == KD_BF16) {  // head dims 16 and 32 on the D = 64 kernel
-    if (a.D <= 64) launch_fwd_p<BF16, 64>(a, plan, sp, st);
+  } else if (a.dtype == KD_BF16) {  // head dim 16 on the D = 32 kernel
+    if (a.D <= 32) launch_fwd_p<BF16, 32>(a, plan, sp, st);
+    else if (a.D == 64) launch_fwd_p<BF16, 64>(a, plan, sp, st);
     else if (a.D == 128) launch_fwd_p<BF16, 128>(a, plan, sp, st);
     else launch_fwd_p<BF16, 256>(a, plan, sp, st);
   } else {
-    if (a.D <= 64) launch_fwd_p<F16, 64>(a, plan, sp, st);
+    if (a.D <= 32) launch_fwd_p<F16, 32>(a, plan, sp, st);
+    else if (a.D == 64) launch_fwd_p<F16, 64>(a, plan, sp, st);
     else if (a.D == 128) launch_fwd_p<F16, 128>(a, plan, sp, st);
     else launch_fwd_p<F16, 256>(a, plan, sp, st);
   }

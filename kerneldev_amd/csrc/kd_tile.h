@@ -40,8 +40,8 @@ KD_DEV u32x4 buf_load16(__amdgpu_buffer_rsrc_t r, uint32_t off) {
 // added: a load from it returns zeros, a DMA writes zeros to LDS.
 constexpr uint32_t OFF_OUTSIDE = 0x80000000u;
 
-// Head dims 16 and 32 run on the D = 64 kernels: each row holds dbytes =
-// 2 D_real bytes and the columns from there to 64 are read as zeros, by
+// Head dim 16 runs on the D = 32 kernels: each row holds dbytes =
+// 2 D_real bytes and the columns from there to 32 are read as zeros, by
 // sending the loads of those 16-byte chunks outside the buffer.  col: the
 // chunk's byte offset within the row.
 KD_DEV uint32_t col_masked(uint32_t off, uint32_t col, uint32_t dbytes) { return col < dbytes ? off : OFF_OUTSIDE; }
@@ -82,7 +82,7 @@ struct Tile {
   KD_DEV static int swz(int r) {
     // D = 256: 512-byte rows meet the banks as 256-byte rows do, so the
     // D = 128 swizzle (low four chunk bits) serves them too.  D = 32 (64-byte
-    // rows: the fp8 tiles at head dim 64): the 16 rows a half-wave reads fill
+    // rows; also the fp8 tiles at head dim 64): the 16 rows a half-wave reads fill
     // the 256 bytes of banks 4 times over, rows r and r + 4 k sharing their
     // bank offset, so their chunks are told apart by row bits 2 and 3
     if constexpr (D >= 128) return ((r & 3) << 2) | ((r >> 2) & 3);
