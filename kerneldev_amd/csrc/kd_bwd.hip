@@ -197,12 +197,14 @@ KD_DEV void tr_addrs(int lane, int (&addr)[D / 32][2]) {
 // two launches of 128 columns, each recomputing S and dP, so that the dQ
 // accumulators fit next to the operands of the full head dim)
 // NSP: the parts dS enters dQ in (1, 2 or 3: parts_of the precision)
-template <class E, int D, bool Q8, int NSP, int DH = D, int D0 = 0>
+// PIECES: a workgroup takes a piece of its block's list (SplitArgs)
+template <class E, int D, bool Q8, int NSP, bool PIECES, int DH = D, int D0 = 0>
 __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void k_dq(AttnArgs a, const uint32_t* __restrict__ codes,
                                                const uint32_t* __restrict__ list,
                                                const int32_t* __restrict__ count,
                                                const uint32_t* __restrict__ order, int nT, int nQB,
                                                bool fuse_delta, SplitArgs sp) {
+  const int ns = PIECES ? sp.ns : 1;
   constexpr bool SP = NSP >= 2, S3 = NSP == 3;
   using TL = Tile<D>;
   using SO = ScoreOp<E, D, Q8>;  // S^T = K Q^T (16-bit, or fp8 from the K8 tile)
@@ -232,9 +234,9 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void k_dq(AttnArgs a, const 
             c = lane & 31;
   const int T = a.T, H = a.H;
   const int work = xcd_remap(blockIdx.x, gridDim.x);
-  const int h = work / (a.B * nQB * sp.ns);  // head-major, then the plan's longest-first order
-  int rank = work - h * (a.B * nQB * sp.ns);
-  const int piece = split_piece(sp.ns, &rank);
+  const int h = work / (a.B * nQB * ns);  // head-major, then the plan's longest-first order
+  int rank = work - h * (a.B * nQB * ns);
+  const int piece = split_piece(ns, &rank);
   const int item = int(order[rank]);
   const int b = item / nQB, qblock = item - b * nQB, bh = b * H + h;
 
@@ -330,7 +332,7 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void k_dq(AttnArgs a, const 
   const int lbase = item;  // b nQB + qblock
   int n = count[lbase];
   const uint32_t* ent = list + int64_t(lbase) * nT;
-  split_list(sp.ns, piece, &ent, &n);
+  split_list(ns, piece, &ent, &n);
 
   uint32_t koff[NLK], voff[NL], k8off[NL8];
   TLK::load_offsets(wave, lane, krb, koff, KHALF ? uint32_t(DH) * 2u : dbytes);
@@ -521,7 +523,7 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void k_dq(AttnArgs a, const 
     if (e + 1 < n) step(e + 1, std::integral_constant<int, 1>{});
   }
 
-  if (sp.ns > 1) {  // a piece of the list: the sum as it stands (kd_combine.hip)
+  if (PIECES) {  // a piece of the list: the sum as it stands (kd_combine.hip)
     if (qvalid) store_part<DH>(sp.part + ((int64_t(piece) * a.B * H + bh) * T + qrow) * a.D + D0, acc, hf, DH == D ? a.D : DH);
   } else if (qvalid) {
     uint16_t* g = static_cast<uint16_t*>(a.dq) + b * a.dq_strides[0] + h * a.dq_strides[1] + qrow * a.dq_strides[2];
@@ -1314,15 +1316,20 @@ static void launch_dq_s(const AttnArgs& a, const uint8_t* plan, const SplitArgs&
   auto* list = reinterpret_cast<const uint32_t*>(plan + L.dq_list);
   auto* cnt = reinterpret_cast<const int32_t*>(plan + L.dq_count);
   auto* order = reinterpret_cast<const uint32_t*>(plan + L.dq_order);
-  if constexpr (D == 256) {  // two launches, the column halves of dQ; the first forms Delta
-    hipLaunchKernelGGL((k_dq<E, D, Q8, NSP, 128, 0>), dim3(grid), dim3(256), 0, st, a, codes, list, cnt, order, L.nT,
-                       L.n_dq_blocks, fuse_delta, sp);
-    hipLaunchKernelGGL((k_dq<E, D, Q8, NSP, 128, 128>), dim3(grid), dim3(256), 0, st, a, codes, list, cnt, order, L.nT,
-                       L.n_dq_blocks, false, sp);
-  } else {
-    hipLaunchKernelGGL((k_dq<E, D, Q8, NSP>), dim3(grid), dim3(256), 0, st, a, codes, list, cnt, order, L.nT,
-                       L.n_dq_blocks, fuse_delta, sp);
-  }
+  auto go = [&](auto pieces) {  // (with pieces apart: a run-time test of them cost the whole lists 1.5% at d = 64)
+    constexpr bool P = decltype(pieces)::value;
+    if constexpr (D == 256) {  // two launches, the column halves of dQ; the first forms Delta
+      hipLaunchKernelGGL((k_dq<E, D, Q8, NSP, P, 128, 0>), dim3(grid), dim3(256), 0, st, a, codes, list, cnt, order, L.nT,
+                         L.n_dq_blocks, fuse_delta, sp);
+      hipLaunchKernelGGL((k_dq<E, D, Q8, NSP, P, 128, 128>), dim3(grid), dim3(256), 0, st, a, codes, list, cnt, order,
+                         L.nT, L.n_dq_blocks, false, sp);
+    } else {
+      hipLaunchKernelGGL((k_dq<E, D, Q8, NSP, P>), dim3(grid), dim3(256), 0, st, a, codes, list, cnt, order, L.nT,
+                         L.n_dq_blocks, fuse_delta, sp);
+    }
+  };
+  if (sp.ns > 1) go(std::true_type{});
+  else go(std::false_type{});
 }
 template <class E, int D, bool Q8 = false>
 static void launch_dq_t(const AttnArgs& a, const uint8_t* plan, const SplitArgs& sp, hipStream_t st, bool fuse_delta) {

@@ -50,13 +50,15 @@ template <> constexpr float rescale_log2<F16>() { return 15.f; }
 constexpr int FWD_PF = 4;
 
 // NSP: the parts P enters P V in (1, 2 or 3: parts_of the precision)
-template <class E, int D, bool Q8, int NSP>
+// PIECES: a workgroup takes a piece of its block's list (SplitArgs)
+template <class E, int D, bool Q8, int NSP, bool PIECES>
 __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void k_fwd(AttnArgs a, const uint32_t* __restrict__ codes,
                                                              const uint32_t* __restrict__ list,
                                                              const int32_t* __restrict__ count,
                                                              const uint32_t* __restrict__ order, int nT, int nQB,
                                                              SplitArgs sp) {
   constexpr bool SP = NSP >= 2, S3 = NSP == 3;
+  const int ns = PIECES ? sp.ns : 1;
   constexpr int NW = 4;             // waves per 128-row q-block; each owns 32 rows
   using TL = Tile<D, NW>;           // V tiles (and K tiles on the 16-bit path)
   using SO = ScoreOp<E, D, Q8>;     // S^T = K Q^T, 16-bit or fp8
@@ -75,8 +77,8 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void k_fwd(AttnArgs a, const
             c = lane & 31;
   const int T = a.T, H = a.H;
   int h, rank;  // (fwd_work: per XCD, the plan's longest-first order)
-  fwd_work(blockIdx.x, gridDim.x, a.B * nQB * sp.ns, &h, &rank);
-  const int piece = split_piece(sp.ns, &rank);
+  fwd_work(blockIdx.x, gridDim.x, a.B * nQB * ns, &h, &rank);
+  const int piece = split_piece(ns, &rank);
   const int item = int(order[rank]);
   const int b = item / nQB, qblock = item - b * nQB, bh = b * H + h;
 
@@ -116,7 +118,7 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void k_fwd(AttnArgs a, const
   const int lbase = item;  // b nQB + qblock
   int n = count[lbase];
   const uint32_t* ent = list + int64_t(lbase) * nT;
-  split_list(sp.ns, piece, &ent, &n);
+  split_list(ns, piece, &ent, &n);
 
   uint32_t koff[NLK], voff[NL];
   TK::load_offsets(wave, lane, krb, koff, Q8 ? uint32_t(TK::ROWB) : dbytes);
@@ -320,7 +322,7 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void k_fwd(AttnArgs a, const
   {
     const float l_tot = xhalf_sum(l0 + l1);
     const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-    if (sp.ns > 1) {  // a piece of the row's list: O as it stands, the maximum and the sum (kd_combine.hip)
+    if (PIECES) {  // a piece of the row's list: O as it stands, the maximum and the sum (kd_combine.hip)
       if (qvalid) {
         const int64_t at = (int64_t(piece) * a.B * H + bh) * T + qrow;
         store_part<D>(sp.part + at * a.D, o, hf, a.D);
@@ -370,11 +372,15 @@ static void launch_fwd_t(const AttnArgs& a, const uint8_t* plan, const SplitArgs
   const PlanLayout L = plan_layout(a.B, a.T, a.D);
   const int nQB = L.n_fwd_blocks;
   const unsigned grid = unsigned(a.B) * a.H * nQB * sp.ns;
-  hipLaunchKernelGGL((k_fwd<E, D, Q8, NSP>), dim3(grid), dim3(256), 0, st, a,
-                     reinterpret_cast<const uint32_t*>(plan + L.codes),
-                     reinterpret_cast<const uint32_t*>(plan + L.fwd_list),
-                     reinterpret_cast<const int32_t*>(plan + L.fwd_count),
-                     reinterpret_cast<const uint32_t*>(plan + L.fwd_order), L.nT, nQB, sp);
+  auto go = [&](auto pieces) {  // (with pieces apart: a run-time test of them cost the whole lists 1% at d = 128)
+    hipLaunchKernelGGL((k_fwd<E, D, Q8, NSP, decltype(pieces)::value>), dim3(grid), dim3(256), 0, st, a,
+                       reinterpret_cast<const uint32_t*>(plan + L.codes),
+                       reinterpret_cast<const uint32_t*>(plan + L.fwd_list),
+                       reinterpret_cast<const int32_t*>(plan + L.fwd_count),
+                       reinterpret_cast<const uint32_t*>(plan + L.fwd_order), L.nT, nQB, sp);
+  };
+  if (sp.ns > 1) go(std::true_type{});
+  else go(std::false_type{});
 }
 
 template <class E, int D, bool Q8 = false>
