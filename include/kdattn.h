@@ -212,7 +212,9 @@ typedef struct kd_x3_args {
  * beside its pointer in every entry point that takes a plan.  3.1.0:
  * kd_plan_layout writes 20 offsets (the dK/dV work order added).  3.2.0:
  * kd_absmax added.  3.3.0: fp8 scores (q8 / k8) and kd_quant_fp8 at head
- * dim 256. */
+ * dim 256.  3.4.0: attention with a workspace (kd_attn_fwd_ws, kd_attn_bwd_ws),
+ * kd_signs, kd_span_count, kd_rms_norm, kd_swiglu, kd_weight_grad, kd_x3_pack
+ * and kd_x3_unpack added. */
 int kd_version(void);
 
 /* Message for the last non-zero status returned on this thread. */
