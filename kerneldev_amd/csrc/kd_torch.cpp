@@ -544,6 +544,12 @@ bool flat16(const Tensor& t) {
 bool second_order(const Tensor& d, const Tensor& a, const Tensor& b) {
   return at::GradMode::is_enabled() && (d.requires_grad() || a.requires_grad() || (b.defined() && b.requires_grad()));
 }
+// The same operations serve a cotangent that is not plain: one with a tangent (a
+// later operand of forward-over-reverse differentiation), which the kernels
+// would drop
+bool by_torch(const Tensor& d, const Tensor& a, const Tensor& b) {
+  return d._fw_grad(0).defined() || second_order(d, a, b);
+}
 Tensor ready_grad(Tensor d, const Tensor& like) {
   if (d.is_neg()) d = d.resolve_neg();
   if (d._is_zerotensor()) d = at::zeros(d.sizes(), like.options());
@@ -565,7 +571,7 @@ struct RmsNorm : torch::autograd::Function<RmsNorm> {
   static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
     const variable_list s = ctx->get_saved_variables();
     const Tensor &x = s[0], &rstd = s[1];
-    if (second_order(grads[0], x, Tensor())) {
+    if (by_torch(grads[0], x, Tensor())) {
       const Tensor f = x.to(at::kFloat), d = grads[0].to(at::kFloat);
       const Tensor r = at::rsqrt(f.pow(2).mean(-1, true) + ctx->saved_data["eps"].toDouble());
       return {(r * (d - f * (r * r * (d * f).mean(-1, true)))).to(x.scalar_type()), Tensor()};
@@ -593,7 +599,7 @@ struct Gate : torch::autograd::Function<Gate> {
   static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
     const variable_list s = ctx->get_saved_variables();
     const Tensor &a = s[0], &b = s[1];
-    if (second_order(grads[0], a, b)) {
+    if (by_torch(grads[0], a, b)) {
       const Tensor u = a.to(at::kFloat), v = b.to(at::kFloat), d = grads[0].to(at::kFloat), g = at::sigmoid(u);
       return {(d * v * g * (1 + u * (1 - g))).to(a.scalar_type()), (d * (u * g)).to(a.scalar_type())};
     }
@@ -618,7 +624,7 @@ struct Projection : torch::autograd::Function<Projection> {
     const Tensor &x = s[0], &w = s[1];
     const int64_t N = w.size(0), K = w.size(1), M = x.numel() / K;
     Tensor dx, dw;
-    if (second_order(grads[0], x, w)) {
+    if (by_torch(grads[0], x, w)) {
       dx = at::matmul(grads[0], w);
       dw = at::matmul(grads[0].reshape({M, N}).t(), x.reshape({M, K}));
       return {dx, dw};

@@ -1,0 +1,82 @@
+"""GPU: gradients whose cotangent is not a plain tensor.
+
+A node's backward is handed whatever the layers behind it return: in
+forward-over-reverse differentiation a cotangent with a tangent, under
+``is_grads_batched`` a batch of cotangents.  Compared with fp64 torch (or, where
+the same kernels run, bit for bit with one cotangent at a time)."""
+import pytest
+import torch
+import torch.autograd.forward_ad as fw
+import torch.nn.functional as F
+
+from kerneldev_amd.gpt import Projection, RMSNorm, SwiGLU
+
+pytestmark = pytest.mark.gpu
+
+BF = torch.bfloat16
+
+
+def _randn(dev, *shape, seed=0):
+    return torch.randn(shape, generator=torch.Generator().manual_seed(seed)).to(BF).to(dev)
+
+
+def _norm(x):
+    return x * torch.rsqrt(x.pow(2).mean(-1, keepdim=True) + 1e-6)
+
+
+def _block_layers(dev):
+    """(name, call, operands, the same in fp64) of each layer with a node of its own."""
+    p = Projection(64, 72).to(dev).to(BF)
+    m = SwiGLU(64, 128).to(dev).to(BF)
+    m.w1, m.w2, m.w3 = torch.nn.Identity(), torch.nn.Identity(), torch.nn.Identity()  # the gate alone: silu(x) x
+
+    def gate64(x):
+        return F.silu(x) * x
+
+    return [("norm", RMSNorm(), [_randn(dev, 3, 5, 64)], _norm),
+            ("gate", m, [_randn(dev, 3, 5, 64, seed=1)], gate64),
+            ("projection", p, [_randn(dev, 3, 5, 64, seed=2), p.weight], F.linear)]
+
+
+def _run(name, layer, xs):
+    return layer(xs[0])
+
+
+@pytest.mark.parametrize("which", [0, 1, 2], ids=["norm", "gate", "projection"])
+def test_tangent_of_a_cotangent(dev, which):
+    """The gradients' tangents are the vector-Jacobian product of the cotangent's tangent."""
+    name, layer, xs, ref = _block_layers(dev)[which]
+    xs = [x.detach() for x in xs[:1]] + xs[1:]
+    xs[0].requires_grad_(True)
+    y = _run(name, layer, xs)
+    assert "CppFunction" in type(y.grad_fn).__name__
+    c, t = _randn(dev, *y.shape, seed=3), _randn(dev, *y.shape, seed=4)
+    with fw.dual_level():
+        got = [fw.unpack_dual(g) for g in torch.autograd.grad(y, xs, fw.make_dual(c, t))]
+    x64 = [x.detach().double().requires_grad_(True) for x in xs]
+    y64 = ref(*x64)
+    for cot, part in ((c, "primal"), (t, "tangent")):
+        want = torch.autograd.grad(y64, x64, cot.double(), retain_graph=True)
+        for g, w in zip(got, want):
+            x = getattr(g, part)
+            assert x is not None, f"{name}: no {part}"
+            # fp32 sums rounded once to bf16 (2^-9 each); the library's products may round one partial result more
+            assert (x.double() - w).norm() <= 2.0 ** -8 * w.norm(), (name, part)
+
+
+def test_forward_over_reverse_through_a_block(dev):
+    """Only a later weight is dual: the mixed second derivative of the layers before it."""
+    norm, mlp = RMSNorm(), SwiGLU(64, 128).to(dev).to(BF)
+    x = _randn(dev, 3, 5, 64, seed=5).requires_grad_(True)
+    w, tw = _randn(dev, 64, seed=6), _randn(dev, 64, seed=7)
+    with fw.dual_level():
+        loss = (mlp(norm(x)) * fw.make_dual(w, tw)).sum()
+        g, = torch.autograd.grad(loss, x)
+        tangent = fw.unpack_dual(g).tangent
+    assert tangent is not None
+    x64 = x.detach().double().requires_grad_(True)
+    w1, w2, w3 = (p.weight.detach().double() for p in (mlp.w1, mlp.w2, mlp.w3))
+    n = _norm(x64)
+    want, = torch.autograd.grad((((F.silu(n @ w1.T) * (n @ w3.T)) @ w2.T) * tw.double()).sum(), x64)
+    # six bf16 layers forward and back, each rounding its activations or gradients (2^-9): about 2^-8 sqrt(6) in all
+    assert (tangent.double() - want).norm() <= 2.0 ** -5 * want.norm()
