@@ -14,6 +14,7 @@
 #include <ATen/autocast_mode.h>
 #include <ATen/record_function.h>
 #include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/core/dispatch/Dispatcher.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/core/DeviceGuard.h>
@@ -61,16 +62,40 @@ void* stream_of(const Tensor& t) { return stream_on(t.device()); }
 bool plain(const Tensor& t) {
   using K = c10::DispatchKey;
   static const c10::DispatchKeySet other({K::Python, K::PythonTLSSnapshot, K::Negative, K::Conjugate, K::ZeroTensor,
-                                          K::FuncTorchBatched, K::FuncTorchGradWrapper, K::Functionalize});
+                                          K::Batched, K::FuncTorchBatched, K::FuncTorchGradWrapper, K::Functionalize});
   return t.defined() && t.is_cuda() && t.layout() == at::kStrided && !t.is_nested() &&
          (t.key_set() & other).empty() && !t._fw_grad(0).defined();
 }
 bool plain(const OptTensor& t) { return !t.has_value() || plain(*t); }
-bool plain_mode() {
+bool no_dispatch() {  // no dispatch mode, transform or tracer that has to see operations
   using K = c10::DispatchKey;
-  return !c10::impl::TorchDispatchModeTLS::any_modes_set() && at::impl::PythonTorchFunctionTLS::stack_len() == 0 &&
+  return !c10::impl::TorchDispatchModeTLS::any_modes_set() &&
          !c10::impl::tls_is_dispatch_key_included(K::FuncTorchDynamicLayerFrontMode) &&
          !c10::impl::tls_is_dispatch_key_included(K::Functionalize) && !torch::jit::tracer::isTracing();
+}
+bool plain_mode() { return no_dispatch() && at::impl::PythonTorchFunctionTLS::stack_len() == 0; }
+
+// Whether a backward may hand its cotangent to the kernels.  It is whatever the
+// nodes behind returned: a batch (is_grads_batched), a tensor with a tangent
+// (forward-over-reverse) or a subclass goes through operations that know
+// these -- torch's, or the custom op -- and so does everything under a mode that
+// was entered for the backward alone.  (Lazy negation and zero tensors are made
+// real by the backward itself.)
+bool plain_cotangent(const Tensor& d) {
+  using K = c10::DispatchKey;
+  static const c10::DispatchKeySet other({K::Python, K::PythonTLSSnapshot, K::Batched, K::FuncTorchBatched,
+                                          K::FuncTorchGradWrapper, K::Functionalize});
+  return no_dispatch() && d.is_cuda() && d.layout() == at::kStrided && !d.is_nested() && (d.key_set() & other).empty() &&
+         !d._fw_grad(0).defined();
+}
+
+// The results of a custom op (attention.py, span_head.py) through the dispatcher
+variable_list call_op(const char* name, std::vector<c10::IValue> args) {
+  const auto op = c10::Dispatcher::singleton().findSchemaOrThrow(name, "");
+  op.callBoxed(&args);
+  variable_list out;
+  for (c10::IValue& r : args) out.push_back(std::move(r).toTensor());
+  return out;
 }
 
 // Unit d-stride, 16-byte aligned base, 8-element-multiple strides, rows that
@@ -255,6 +280,16 @@ struct Attention : torch::autograd::Function<Attention> {
     RECORD_FUNCTION("kdattn::bwd", std::vector<c10::IValue>());
     const variable_list s = ctx->get_saved_variables();
     const bool rot = ctx->saved_data["rot"].toBool(), fp8 = ctx->saved_data["fp8"].toBool();
+    if (!plain_cotangent(grads[0])) {
+      auto opt = [&](bool given, size_t i) { return given ? c10::IValue(s[i]) : c10::IValue(); };
+      const size_t i = rot ? 8 : 7;
+      const variable_list g =
+          call_op("kdattn::bwd", {s[0], s[1], s[2], s[3], s[4], grads[0], s[5], ctx->saved_data["sm_scale"].toDouble(),
+                                  s[6].defined() ? s[6] : at::empty({0}, s[3].options()), opt(fp8, i), opt(fp8, i + 1),
+                                  opt(fp8, i + 2), opt(fp8, i + 3), opt(rot, 7), ctx->saved_data["prec"].toInt()});
+      for (int j = 0; j < 3; ++j) out[j] = g[j];
+      return out;
+    }
     bool differentiable = false;  // (create_graph: the op has no second derivative, which its use must report)
     if (at::GradMode::is_enabled())
       for (const Tensor& t : {s[0], s[1], s[2], s[3], s[4], grads[0]}) differentiable |= t.requires_grad();
@@ -367,6 +402,12 @@ struct AttentionX3 : torch::autograd::Function<AttentionX3> {
     if (!grads[0].defined()) return out;  // only LSE reached the loss
     RECORD_FUNCTION("kdattn::bwd_x3", std::vector<c10::IValue>());
     const variable_list s = ctx->get_saved_variables();
+    if (!plain_cotangent(grads[0])) {
+      const variable_list g = call_op("kdattn::bwd_x3", {s[0], s[1], s[2], s[3], s[4], grads[0], s[5],
+                                                         ctx->saved_data["sm_scale"].toDouble()});
+      for (int j = 0; j < 3; ++j) out[j] = g[j];
+      return out;
+    }
     bool differentiable = false;
     if (at::GradMode::is_enabled())
       for (const Tensor& t : {s[0], s[1], s[2], s[3], s[4], grads[0]}) differentiable |= t.requires_grad();
@@ -505,6 +546,10 @@ struct SpanHead : torch::autograd::Function<SpanHead> {
     if (!grads[0].defined()) return out;
     RECORD_FUNCTION("kdattn::span_bwd", std::vector<c10::IValue>());
     const variable_list s = ctx->get_saved_variables();
+    if (!plain_cotangent(grads[0])) {
+      out[0] = call_op("kdattn::span_bwd", {s[0], s[1], grads[0], s[2], s[3], s[4], s[5], s[6]})[0];
+      return out;
+    }
     const bool differentiable = at::GradMode::is_enabled() && (s[1].requires_grad() || grads[0].requires_grad());
     variable_list dh(1);
     {
@@ -535,7 +580,7 @@ pybind11::object span(const Tensor& tokens, const Tensor& h, int64_t n) {
 }
 
 // ------------------------------------------------------- transformer block
-// Under create_graph the backward of both is formed with differentiable torch
+// Under create_graph the backward of each is formed with differentiable torch
 // operations, so that second derivatives exist as they do for the eager forms.
 bool flat16(const Tensor& t) {
   return plain(t) && t.is_contiguous() && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 &&
@@ -544,12 +589,8 @@ bool flat16(const Tensor& t) {
 bool second_order(const Tensor& d, const Tensor& a, const Tensor& b) {
   return at::GradMode::is_enabled() && (d.requires_grad() || a.requires_grad() || (b.defined() && b.requires_grad()));
 }
-// The same operations serve a cotangent that is not plain: one with a tangent (a
-// later operand of forward-over-reverse differentiation), which the kernels
-// would drop
-bool by_torch(const Tensor& d, const Tensor& a, const Tensor& b) {
-  return d._fw_grad(0).defined() || second_order(d, a, b);
-}
+// The same operations serve a cotangent that is not plain
+bool by_torch(const Tensor& d, const Tensor& a, const Tensor& b) { return !plain_cotangent(d) || second_order(d, a, b); }
 Tensor ready_grad(Tensor d, const Tensor& like) {
   if (d.is_neg()) d = d.resolve_neg();
   if (d._is_zerotensor()) d = at::zeros(d.sizes(), like.options());

@@ -80,3 +80,67 @@ def test_forward_over_reverse_through_a_block(dev):
     want, = torch.autograd.grad((((F.silu(n @ w1.T) * (n @ w3.T)) @ w2.T) * tw.double()).sum(), x64)
     # six bf16 layers forward and back, each rounding its activations or gradients (2^-9): about 2^-8 sqrt(6) in all
     assert (tangent.double() - want).norm() <= 2.0 ** -5 * want.norm()
+
+
+def _nodes(dev):
+    """(name, output, inputs) of every C++ node on plain operands."""
+    from kerneldev_amd import flash_attention
+    from kerneldev_amd.span_head import span_scores
+
+    out = []
+    for name, layer, xs, _ in _block_layers(dev):
+        xs = [x.detach().requires_grad_(True) for x in xs[:1]] + xs[1:]
+        out.append((name, layer(xs[0]), xs))
+    for name, dtype, d, kw in (("attention", BF, 64, {}), ("rotated fp8", BF, 128, dict(hadamard=True, qk_dtype="fp8_e4m3")),
+                               ("bf16x3", torch.float32, 32, {})):
+        xs = [_randn(dev, 1, 2, 130, d, seed=10 + i).to(dtype).requires_grad_(True) for i in range(3)]
+        out.append((name, flash_attention(*xs, **kw), xs))
+    tokens = torch.tensor([[2, 3, 9, 9, 4, 9, 3, 9, 4, 9]] * 2, device=dev)
+    h = _randn(dev, 2, 10, 48, seed=20).requires_grad_(True)
+    out.append(("span head", span_scores(tokens, h), [h]))
+    return out
+
+
+NODES = ["norm", "gate", "projection", "attention", "rotated fp8", "bf16x3", "span head"]
+
+
+@pytest.mark.parametrize("which", range(len(NODES)), ids=NODES)
+def test_batched_cotangents(dev, which):
+    name, y, xs = _nodes(dev)[which]
+    assert name == NODES[which] and "CppFunction" in type(y.grad_fn).__name__
+    c = torch.stack([_randn(dev, *y.shape, seed=30 + i) for i in range(3)]).to(y.dtype)
+    got = torch.autograd.grad(y, xs, c, is_grads_batched=True, retain_graph=True)
+    for i in range(3):
+        for g, w in zip(got, torch.autograd.grad(y, xs, c[i], retain_graph=True)):
+            if which < 3:  # torch's operations against the kernels: one rounding of fp32 results each, 2^-9
+                assert (g[i].double() - w.double()).norm() <= 2.0 ** -8 * w.double().norm()
+            else:  # the same kernels
+                assert torch.equal(g[i], w)
+
+
+def test_vectorized_jacobian(dev):
+    x = _randn(dev, 2, 8, seed=40)
+    got = torch.autograd.functional.jacobian(RMSNorm(), x, vectorize=True)
+    want = torch.autograd.functional.jacobian(_norm, x.double())
+    assert (got.double() - want).norm() <= 2.0 ** -8 * want.norm()
+
+
+@pytest.mark.parametrize("which", range(len(NODES)), ids=NODES)
+def test_dispatch_mode_sees_the_backward(dev, which):
+    """A mode entered for the backward alone sees operations, and the gradients are the same."""
+    _, y, xs = _nodes(dev)[which]
+    c = _randn(dev, *y.shape, seed=50).to(y.dtype)
+    want = torch.autograd.grad(y, xs, c, retain_graph=True)
+    seen = []
+
+    class Seen(torch.utils._python_dispatch.TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    with Seen():
+        got = torch.autograd.grad(y, xs, c, retain_graph=True)
+    op = {3: "kdattn.bwd.default", 4: "kdattn.bwd.default", 5: "kdattn.bwd_x3.default", 6: "kdattn.span_bwd.default"}
+    assert (op[which] in seen) if which > 2 else any("mul" in s or "mm" in s for s in seen)
+    for g, w in zip(got, want):
+        assert (g.double() - w.double()).norm() <= (2.0 ** -8 if which < 3 else 0.0) * w.double().norm()
