@@ -589,8 +589,14 @@ bool flat16(const Tensor& t) {
 bool second_order(const Tensor& d, const Tensor& a, const Tensor& b) {
   return at::GradMode::is_enabled() && (d.requires_grad() || a.requires_grad() || (b.defined() && b.requires_grad()));
 }
-// The same operations serve a cotangent that is not plain
-bool by_torch(const Tensor& d, const Tensor& a, const Tensor& b) { return !plain_cotangent(d) || second_order(d, a, b); }
+// The same operations serve a cotangent that is not plain, and saved operands that
+// a hook returned in another layout, type or place than they were saved in
+bool as_saved(const Tensor& t, const Tensor& d) {
+  return flat16(t) && t.scalar_type() == d.scalar_type() && t.device() == d.device();
+}
+bool by_torch(const Tensor& d, const Tensor& a, const Tensor& b) {
+  return !plain_cotangent(d) || second_order(d, a, b) || !as_saved(a, d) || (b.defined() && !as_saved(b, d));
+}
 Tensor ready_grad(Tensor d, const Tensor& like) {
   if (d.is_neg()) d = d.resolve_neg();
   if (d._is_zerotensor()) d = at::zeros(d.sizes(), like.options());
@@ -612,7 +618,8 @@ struct RmsNorm : torch::autograd::Function<RmsNorm> {
   static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
     const variable_list s = ctx->get_saved_variables();
     const Tensor &x = s[0], &rstd = s[1];
-    if (by_torch(grads[0], x, Tensor())) {
+    if (by_torch(grads[0], x, Tensor()) || x.sizes() != grads[0].sizes() || !plain(rstd) || !rstd.is_contiguous() ||
+        rstd.scalar_type() != at::kFloat || rstd.numel() != x.numel() / x.size(-1)) {
       const Tensor f = x.to(at::kFloat), d = grads[0].to(at::kFloat);
       const Tensor r = at::rsqrt(f.pow(2).mean(-1, true) + ctx->saved_data["eps"].toDouble());
       return {(r * (d - f * (r * r * (d * f).mean(-1, true)))).to(x.scalar_type()), Tensor()};
@@ -640,7 +647,7 @@ struct Gate : torch::autograd::Function<Gate> {
   static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
     const variable_list s = ctx->get_saved_variables();
     const Tensor &a = s[0], &b = s[1];
-    if (by_torch(grads[0], a, b)) {
+    if (by_torch(grads[0], a, b) || a.sizes() != grads[0].sizes() || b.sizes() != a.sizes()) {
       const Tensor u = a.to(at::kFloat), v = b.to(at::kFloat), d = grads[0].to(at::kFloat), g = at::sigmoid(u);
       return {(d * v * g * (1 + u * (1 - g))).to(a.scalar_type()), (d * (u * g)).to(a.scalar_type())};
     }
@@ -665,7 +672,7 @@ struct Projection : torch::autograd::Function<Projection> {
     const Tensor &x = s[0], &w = s[1];
     const int64_t N = w.size(0), K = w.size(1), M = x.numel() / K;
     Tensor dx, dw;
-    if (by_torch(grads[0], x, w)) {
+    if (by_torch(grads[0], x, w) || x.size(-1) != K || grads[0].numel() != M * N) {
       dx = at::matmul(grads[0], w);
       dw = at::matmul(grads[0].reshape({M, N}).t(), x.reshape({M, K}));
       return {dx, dw};

@@ -144,3 +144,32 @@ def test_dispatch_mode_sees_the_backward(dev, which):
     assert (op[which] in seen) if which > 2 else any("mul" in s or "mm" in s for s in seen)
     for g, w in zip(got, want):
         assert (g.double() - w.double()).norm() <= (2.0 ** -8 if which < 3 else 0.0) * w.double().norm()
+
+
+@pytest.mark.parametrize("how", ["transposed", "shifted", "other type", "other device"])
+@pytest.mark.parametrize("which", [0, 1, 2], ids=["norm", "gate", "projection"])
+def test_saved_tensors_that_hooks_changed(dev, which, how):
+    """An unpack hook may return the same values in other strides, at an unaligned address or in another type:
+    torch's operations take them as the eager layers did; on another device they raise."""
+    name, layer, xs, ref = _block_layers(dev)[which]
+    xs = [x.detach() for x in xs[:1]] + xs[1:]
+    xs[0].requires_grad_(True)
+
+    def unpack(t):
+        if how == "transposed":
+            return t.transpose(0, 1).contiguous().transpose(0, 1) if t.dim() > 1 else t
+        if how == "shifted":
+            return t.new_empty(t.numel() + 1)[1:].view(t.shape).copy_(t)
+        return t.float() if how == "other type" else t.cpu()
+
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
+        y = layer(xs[0])
+    c = _randn(dev, *y.shape, seed=60)
+    if how == "other device" or (how, name) == ("other type", "projection"):
+        with pytest.raises(RuntimeError):  # (devices, or the two types of a product, differ)
+            torch.autograd.grad(y, xs, c)
+        return
+    x64 = [x.detach().double().requires_grad_(True) for x in xs]
+    want = torch.autograd.grad(ref(*x64), x64, c.double())
+    for g, w in zip(torch.autograd.grad(y, xs, c), want):
+        assert (g.double() - w).norm() <= 2.0 ** -8 * w.norm()
