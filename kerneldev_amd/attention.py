@@ -431,7 +431,7 @@ def _x3_call(pack: bool, tensors, B, H, T, d, Dp):
 
 
 def _x3_packed(tensors, patterns, B, H, T, d, Dp):
-    tensors = [_kernel_ready(x) for x in tensors]
+    tensors = [_kernel_ready(x.to(torch.float32)) for x in tensors]  # (the kernel reads fp32; k and v may be narrower)
     out = [torch.empty((B, H, T, Dp), dtype=torch.bfloat16, device=x.device) for x in tensors]
     _x3_call(True, list(zip(tensors, out, patterns)), B, H, T, d, Dp)
     return out
