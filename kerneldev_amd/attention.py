@@ -660,6 +660,8 @@ def flash_attention(
         # fp8 scores come from bf16 operands: fp32 inputs are rounded to bf16
         # for this path and O cast back
         q, k, v = q.to(torch.bfloat16), k.to(torch.bfloat16), v.to(torch.bfloat16)
+    if k.dtype != q.dtype or v.dtype != q.dtype:  # the kernels read all three as q's type
+        k, v = k.to(q.dtype), v.to(q.dtype)
     from .hadamard import _rot_op, generate_hadamard_signs
 
     fused_signs = None

@@ -32,3 +32,18 @@ def test_bf16x3_with_narrower_keys_and_values(dev, d, T):
     assert torch.equal(o, want)
     for x, a, b in zip(xs, torch.autograd.grad(o, xs, do), torch.autograd.grad(want, ys, do)):
         assert a.dtype == x.dtype and torch.equal(a, b.to(x.dtype))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("q_type,k_type,v_type", [(torch.bfloat16, torch.float16, torch.bfloat16),
+                                                  (torch.float16, torch.float32, torch.float32),
+                                                  (torch.float32, torch.bfloat16, torch.float16)])
+@pytest.mark.parametrize("d,kw", [(64, {}), (128, dict(hadamard=True)), (32, dict(precision="ieee"))])
+def test_keys_and_values_are_taken_in_the_type_of_q(dev, q_type, k_type, v_type, d, kw):
+    g = torch.Generator().manual_seed(d)
+    q, k, v, do = (torch.randn(1, 2, 130, d, generator=g).to(t).to(dev) for t in (q_type, k_type, v_type, q_type))
+    xs, ys = [x.clone().requires_grad_(True) for x in (q, k, v)], [x.to(q_type).requires_grad_(True) for x in (q, k, v)]
+    o, want = flash_attention(*xs, **kw), flash_attention(*ys, **kw)
+    assert o.dtype == q_type and torch.equal(o, want)
+    for x, a, b in zip(xs, torch.autograd.grad(o, xs, do), torch.autograd.grad(want, ys, do)):
+        assert a.dtype == x.dtype and torch.equal(a, b.to(x.dtype))
