@@ -43,10 +43,11 @@ class RMSNorm(nn.Module):
         self.eps = eps
 
     def forward(self, x):
-        if x.is_cuda and _lib.eager(x):
-            y = _lib.native().rms_norm(x, self.eps)  # bf16 / fp16 rows in one kernel, fp32 inside
-            if y is not None:
-                return y
+        if not torch.jit.is_scripting():  # (a script holds the expression below; a symbolic trace's x is not a tensor)
+            if _lib.eager(x) and x.is_cuda:
+                y = _lib.native().rms_norm(x, self.eps)  # bf16 / fp16 rows in one kernel, fp32 inside
+                if y is not None:
+                    return y
         return x * torch.rsqrt(x.pow(2).mean(-1, keepdim=True) + self.eps)
 
 
@@ -58,11 +59,12 @@ class Projection(nn.Linear):
         super().__init__(in_features, out_features, bias=False)
 
     def forward(self, x):
-        if x.is_cuda and _lib.eager(x, self.weight):
-            y = _lib.native().projection(x, self.weight)
-            if y is not None:
-                return y
-        return super().forward(x)
+        if not torch.jit.is_scripting():
+            if _lib.eager(x, self.weight) and x.is_cuda:
+                y = _lib.native().projection(x, self.weight)
+                if y is not None:
+                    return y
+        return F.linear(x, self.weight, self.bias)
 
 
 class SwiGLU(nn.Module):
@@ -76,8 +78,12 @@ class SwiGLU(nn.Module):
 
     def forward(self, x):
         a, b = self.w1(x), self.w3(x)
-        y = _lib.native().swiglu(a, b) if a.is_cuda and _lib.eager(a, b) else None  # silu(a) b in one kernel, fp32 inside
-        return self.w2(F.silu(a) * b if y is None else y)
+        if not torch.jit.is_scripting():
+            if _lib.eager(a, b) and a.is_cuda:
+                y = _lib.native().swiglu(a, b)  # silu(a) b in one kernel, fp32 inside
+                if y is not None:
+                    return self.w2(y)
+        return self.w2(F.silu(a) * b)
 
 
 class MultiHeadAttention(nn.Module):
