@@ -132,7 +132,7 @@ _span_fwd_op.register_autograd(_span_backward, setup_context=_span_setup)
 
 def max_spans(tokens: torch.Tensor) -> int:
     """The reference's ``max_spans``: the largest per-row ``[SPAN]`` count (one host sync)."""
-    if _lib.eager(tokens):
+    if tokens.is_cuda and _lib.eager(tokens):
         counts = _lib.native().span_counts(tokens)
         if counts is not None:
             return max(counts.tolist())

@@ -5,6 +5,7 @@ a script of them has to come out as the torch expressions."""
 import pytest
 import torch
 
+from kerneldev_amd import _lib
 from kerneldev_amd.gpt import Projection, RMSNorm, SwiGLU
 
 LAYERS = [RMSNorm, lambda: SwiGLU(64, 128), lambda: Projection(64, 72)]
@@ -24,3 +25,10 @@ def test_layers_under_tracers(make, how):
     else:
         t = torch.export.export(m, (x,)).module()
     assert torch.equal(t(x), m(x))
+
+
+def test_max_spans_on_the_cpu_needs_no_library(monkeypatch):
+    from kerneldev_amd.span_head import max_spans
+
+    monkeypatch.setattr(_lib, "native", lambda: pytest.fail("the GPU route was asked for"))
+    assert max_spans(torch.tensor([[3, 3, 1], [3, 1, 1]])) == 2
