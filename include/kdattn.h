@@ -69,6 +69,10 @@ extern "C" {
 #define KD_MODE_CAUSAL 1  /* no metadata, causal=True:  i >= j  (:512-513) */
 #define KD_MODE_ALL 2     /* no metadata, causal=False: all True (:514-515) */
 
+/* lengths of the blocks' key (and query) lists (kd_attn_args.lists) */
+#define KD_LISTS_UNEVEN 0 /* they differ: causal and metadata masks */
+#define KD_LISTS_FULL 1   /* every list is full: KD_MODE_ALL */
+
 /* Mask metadata, as the reference's forward adapter receives it
  * (original_kernel.py:1697-1715: lens, in_span, span_id, is_prefix). */
 typedef struct kd_meta_args {
@@ -137,7 +141,8 @@ typedef struct kd_attn_args {
   int32_t dtype;                /* KD_BF16 / KD_F16 / KD_F32 */
   float sm_scale;
   int32_t precision;            /* KD_PREC_SPLIT (0, default) / KD_PREC_SINGLE / KD_PREC_SPLIT3 */
-  int32_t pad_;
+  int32_t lists;                /* KD_LISTS_UNEVEN (0, default) / KD_LISTS_FULL: what the mask makes of
+                                   the key lists, a hint for kd_attn_*_ws_bytes and kd_attn_*_ws */
 } kd_attn_args;
 
 /* Walsh-Hadamard rotation of [B, H, T, D] rows (incoherent processing). */
@@ -214,7 +219,7 @@ typedef struct kd_x3_args {
  * kd_absmax added.  3.3.0: fp8 scores (q8 / k8) and kd_quant_fp8 at head
  * dim 256.  3.4.0: attention with a workspace (kd_attn_fwd_ws, kd_attn_bwd_ws),
  * kd_signs, kd_span_count, kd_rms_norm, kd_swiglu, kd_weight_grad, kd_x3_pack
- * and kd_x3_unpack added. */
+ * and kd_x3_unpack added.  3.5.0: kd_attn_args.lists, a padding word before. */
 int kd_version(void);
 
 /* Message for the last non-zero status returned on this thread. */
@@ -271,7 +276,7 @@ int kd_attn_fwd(const kd_attn_args *a, const void *plan, int64_t plan_bytes, voi
  * run side by side, and a second kernel puts the fp32 partial results
  * together.  kd_attn_fwd_ws_bytes is 0 where that would not pay (then, and
  * with ws NULL, kd_attn_fwd_ws is kd_attn_fwd), -1 on bad arguments; it
- * depends on a's B, H, T, D and dtype only.  The results are the same at every
+ * depends on a's B, H, T, D, dtype, precision and lists only.  The results are the same at every
  * call (the pieces are added in a fixed order) and differ from kd_attn_fwd's
  * by the rounding of fp32 sums.  ws is 16-byte aligned, used by this call
  * alone until its work on the stream is done, and needs no initial contents. */

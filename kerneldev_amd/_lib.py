@@ -21,6 +21,7 @@ KD_BF16, KD_F16, KD_F32 = 0, 1, 2
 KD_I64, KD_I32 = 0, 1
 KD_MODE_FORMULA, KD_MODE_CAUSAL, KD_MODE_ALL = 0, 1, 2
 KD_PREC_SPLIT, KD_PREC_SINGLE, KD_PREC_SPLIT3 = 0, 1, 2
+KD_LISTS_UNEVEN, KD_LISTS_FULL = 0, 1
 KD_NOALLOC_WORKSPACE_FLOATS = 1 << 22
 
 I64x2 = c_int64 * 2
@@ -57,7 +58,7 @@ class AttnArgs(ctypes.Structure):
         ("dq_lo", c_void_p), ("dk_lo", c_void_p), ("dv_lo", c_void_p),
         ("B", c_int32), ("H", c_int32), ("T", c_int32), ("D", c_int32),
         ("dtype", c_int32), ("sm_scale", c_float),
-        ("precision", c_int32), ("pad_", c_int32),
+        ("precision", c_int32), ("lists", c_int32),
     ]
 
 

@@ -174,8 +174,9 @@ def build_plan_from_tokens(tokens: torch.Tensor, head_dim: int, rule: str = "col
     return AttentionPlan(plan, B, T, head_dim)
 
 
-def _attn_args(q, k, v, sm_scale, prec=_lib.KD_PREC_SPLIT) -> AttnArgs:
+def _attn_args(q, k, v, sm_scale, prec=_lib.KD_PREC_SPLIT, full=False) -> AttnArgs:
     a = AttnArgs()
+    a.lists = _lib.KD_LISTS_FULL if full else _lib.KD_LISTS_UNEVEN
     B, H, T, D = q.shape
     a.B, a.H, a.T, a.D = B, H, T, D
     a.dtype = _dtype_code(q.dtype)
@@ -187,6 +188,11 @@ def _attn_args(q, k, v, sm_scale, prec=_lib.KD_PREC_SPLIT) -> AttnArgs:
 
 
 # ----------------------------------------------------------------- custom ops
+def _full_lists(mode, plan_in) -> bool:
+    """Whether every work list is full (no mask); of a caller's plan that is not known."""
+    return mode == _lib.KD_MODE_ALL and plan_in is None
+
+
 def _workspace(nbytes: int, device):
     """Scratch for the partial results of a call whose work lists are cut into pieces, or None."""
     if nbytes < 0:
@@ -273,7 +279,7 @@ def _fwd_op(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, lens: torch.Tenso
     lse = torch.empty((B, H, T), dtype=torch.float32, device=q.device)
     # rounding residual of O, kept for the backward's Delta (see kd_bwd.hip)
     o_lo = torch.empty((B, H, T, D) if need_lo else (0,), dtype=_lo_dtype(q.dtype, prec), device=q.device)
-    a = _attn_args(q, k, v, sm_scale, prec)
+    a = _attn_args(q, k, v, sm_scale, prec, _full_lists(mode, plan_in))
     _set_fp8(a, (q8_o, k8_o, qs_o, ks_o) if quant_fp8 else None)
     a.o, a.o_strides = o.data_ptr(), _strides3(o)
     a.lse = lse.data_ptr()
@@ -308,14 +314,14 @@ def _bwd_op(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: torch.Tensor, 
             do: torch.Tensor, plan: torch.Tensor, sm_scale: float, o_lo: torch.Tensor,
             q8: torch.Tensor | None = None, k8: torch.Tensor | None = None,
             q_scale: torch.Tensor | None = None, k_scale: torch.Tensor | None = None,
-            dqk_signs: torch.Tensor | None = None, prec: int = 0,
+            dqk_signs: torch.Tensor | None = None, prec: int = 0, full: bool = False,
             ) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
     B, H, T, D = q.shape
     operands = (q, k, v)
     q, k, v, o, do = (_kernel_ready(x) for x in (q, k, v, o, do))
     dq, dk, dv = (_grad_like(x, r) for x, r in zip(operands, (q, k, v)))
     delta = torch.empty((2, B, H, T), dtype=torch.float32, device=q.device)  # Delta, LSE for bwd
-    a = _attn_args(q, k, v, sm_scale, prec)
+    a = _attn_args(q, k, v, sm_scale, prec, full)
     a.o, a.o_strides = o.data_ptr(), _strides3(o)
     a.lse = lse.data_ptr()
     a.dout, a.do_strides = do.data_ptr(), _strides3(do)
@@ -333,7 +339,7 @@ def _bwd_op(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: torch.Tensor, 
 
 @_bwd_op.register_fake
 def _bwd_fake(q, k, v, o, lse, do, plan, sm_scale, o_lo, q8=None, k8=None, q_scale=None, k_scale=None,
-              dqk_signs=None, prec=0):
+              dqk_signs=None, prec=0, full=False):
     return torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
 
 
@@ -357,6 +363,7 @@ def _setup_context(ctx, inputs, output):
     ctx.save_for_backward(q, k, v, o, lse, plan, o_lo, *((signs,) if ctx.rot else ()), *extra)
     ctx.sm_scale = sm_scale
     ctx.prec = prec
+    ctx.full = _full_lists(mode, plan_in)
 
 
 def _backward(ctx, do, dlse, dplan, do_lo, *_unused):
@@ -368,7 +375,8 @@ def _backward(ctx, do, dlse, dplan, do_lo, *_unused):
     q, k, v, o, lse, plan, o_lo, *rest = ctx.saved_tensors
     signs = rest.pop(0) if ctx.rot else None
     fp8 = tuple(rest) if ctx.fp8 else (None, None, None, None)
-    dq, dk, dv = _bwd_op(q, k, v, o, lse, do, plan, ctx.sm_scale, o_lo, *fp8, dqk_signs=signs, prec=ctx.prec)
+    dq, dk, dv = _bwd_op(q, k, v, o, lse, do, plan, ctx.sm_scale, o_lo, *fp8, dqk_signs=signs, prec=ctx.prec,
+                         full=ctx.full)
     return (dq, dk, dv) + (None,) * 12
 
 
@@ -450,7 +458,7 @@ def _fwd_x3_op(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, lens: torch.Te
     ox = torch.empty((B, H, T, Dp), dtype=torch.bfloat16, device=q.device)
     ox_lo = torch.empty_like(ox)
     lse = torch.empty((B, H, T), dtype=torch.float32, device=q.device)
-    a = _attn_args(qx, kx, vx, sm_scale, _lib.KD_PREC_SPLIT)
+    a = _attn_args(qx, kx, vx, sm_scale, _lib.KD_PREC_SPLIT, _full_lists(mode, plan_in))
     a.o, a.o_strides = ox.data_ptr(), _strides3(ox)
     a.lse = lse.data_ptr()
     a.o_lo = ox_lo.data_ptr()

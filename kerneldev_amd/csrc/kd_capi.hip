@@ -119,7 +119,7 @@ int check_plan(const void* plan, int64_t plan_bytes, int B, int T, int D) {
 
 extern "C" {
 
-int kd_version(void) { return 30400; }
+int kd_version(void) { return 30500; }
 
 const char* kd_last_error_string(void) { return g_err.c_str(); }
 

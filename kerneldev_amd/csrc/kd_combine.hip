@@ -157,49 +157,73 @@ int launch(const AttnArgs& a, const CombineArgs& c, bool fwd, int outputs, hipSt
 
 }  // namespace
 
-// How many pieces.  A block's list is a serial chain of up to T / 64 tile
+// How many pieces.  A block's list is a serial chain of up to nT = T / 64 tile
 // steps, so with fewer workgroups than the chip holds the longest list is the
 // kernel's time.  Pieces shorten it, and cost the partial results' way through
-// memory (ns rows D floats written and read, at ~5.9 TB/s), a second launch and
-// each piece's own start (4 us together).  The lines below come from sweeps of
-// ns = 1 .. 8 on causal and full masks (us, forward / dQ / dK+dV; bf16 and causal
-// unless said; W = workgroups without pieces):
-//   B1 H12 T1531 d64  (W 144):  37 / 36 / 39   -> 27.5 / 28 / 33  at 3
-//   B1 H8 T4095 d128  (W 256):  110 / 120 / 139 -> 82 / 96 / 116  at 2
-//   B1 H1 T8192 d64   (W 64):   132 / 134 / 160 -> 44 / 57 / 45   at 4
-//   B1 H8 T2048 d256  (W 128):  99 / 170 / 238 -> 61 / 108 / 128  at 3
-//   B2 H8 T1531 d64, full (W 192): 35 -> 37 at 2 and 3, 35 at 4: no gain left
-//   B4 H8 T395 d128   (W 128):  17 -> 22 at 2: lists of 7 tiles are too short
-//   B2 H8 T4096 d64   (W 512):  80 -> 79 at 2, 81 at 3: no pieces from here on
-//   fp32 B1 H8 T2048 d128 (W 256): 170 / 230 / 296 -> 102 / 145 / 188 at 3
-//   fp32 B4 H8 T777 d64   (W 448): 60 / 77 / 90 -> 49 / 64 / 78 at 2
-//   fp32 B8 H8 T395 d128  (W 512): 59 -> 63 at 2, full 75 -> 95
-//   fp32 B2 H8 T4096 d128 (W 1024): 647 -> 626 at 2: long causal lists only
-// 16-bit: pieces of two tiles or more while each has a CU to itself, of six or
-// more up to two a CU (at d = 256, where one fills a CU, up to one and a half).
-// fp32 (two workgroups a block, a tile takes four times as long): one tile a
-// piece, up to two (d = 256), three (128) or four workgroups a CU.  And what a
-// piece saves has to be 1.45 times what it costs.
+// memory (ns rows D floats written and read), a second launch, each piece's own
+// start, and more workgroups on a CU.  The count is the one with the least of
+//   steps of a piece x us a step x (1 + crowd (k - 1) share) + starts + cost
+// where k = workgroups a CU (256 CUs), crowd what each further one on a CU costs a
+// step (full masks, us a step at one, two, three and four workgroups a CU: fp32 d64
+// forward 3.1, 4.9, 6.9, 9.0; bf16 d64 dQ 1.07, 2.06; bf16 d128 dK/dV, whose LDS holds
+// one, 2.2, 5.3), and share how much of that is met by lists of uneven length,
+// where a long list runs beside short ones: all of it for full masks (every list as
+// long), a quarter where an XCD's first 64 workgroups are one head's, longest
+// first, so that the upper half of its lists runs beside the lower, about half to two
+// thirds elsewhere.  It has to save a tenth of the uncut time.
+//
+// Fitted to and checked on every pass of 648 shapes (B 1 and 4, W = 4 .. 1536
+// workgroups, T 512 .. 8192, d 32 .. 256, bf16 and fp32) under full, causal and
+// cocktail masks, timed at each count: 1.26 times faster than uncut in the geometric
+// mean, and 5 of 5832 slower by more than 1.5% (the worst 1.04 x).  The rule before it
+// knew neither k nor the mask: 1.24 times faster, 361 slower, up to 1.43 x.  Some, us
+// (forward / dQ / dK+dV):
+//   bf16 B1 H8 T4095 d128 causal (W 256): 96 / 102 / 135 -> 77 / 88 / 114 at 2
+//   bf16 B1 H16 T2048 d64 causal (W 256): 39 / 36 / 50, 42 / 41 / 56 at 2: uncut
+//   bf16 B1 H12 T1400 d128 full (W 132): dK+dV 53, 76 at 2: uncut
+//   bf16 B1 H1 T8192 d64 causal (W 64): 132 / 134 / 160 -> 44 / 57 / 45 at 4
+//   fp32 B1 H8 T2048 d128 causal (W 256): 168 / 222 / 299 -> 123 / 161 / 214 at 2
+//   fp32 B1 H32 T512 d64 causal (W 256): 28.7 / 35 / 48, 35 / 42 / 51 at 4: uncut
 int split_pieces(const AttnArgs& a, SplitPass pass) {
-  const bool f32 = use_simt(a);
+  const bool f32 = use_simt(a), full = a.lists == KD_LISTS_FULL;
   const int nT = (a.T + 63) / 64, nblk = (nT + 1) / 2;
-  const int64_t rows = int64_t(a.B) * a.H * a.T, W = int64_t(a.B) * a.H * nblk * (f32 ? 2 : 1);
-  const int d = a.D <= 32 ? 0 : a.D == 64 ? 1 : a.D == 128 ? 2 : 3;
-  // us a tile step takes a workgroup that has its CU to itself
-  constexpr float step16[4] = {1.0f, 1.0f, 1.7f, 3.0f}, step32[4] = {2.0f, 3.0f, 5.3f, 10.6f};
-  constexpr float pass16[3] = {1.0f, 1.1f, 1.25f}, pass32[3] = {1.0f, 1.3f, 1.8f};
-  constexpr int64_t room32[4] = {1024, 1024, 768, 512};
-  const float step = f32 ? step32[d] * pass32[pass] : step16[d] * pass16[pass];
-  const int outs = pass == SPLIT_DKDV ? 2 : 1;
-  for (int ns = f32 ? 6 : 4; ns > 1; --ns) {
-    const int64_t wg = W * ns;
-    const bool room = f32 ? nT >= ns && (wg <= (ns > 4 ? 256 : room32[d]) || (wg <= 2048 && nT >= 32 * ns))
-                          : (wg <= 256 && nT >= 2 * ns) || (wg <= (a.D == 256 ? 384 : 512) && nT >= 6 * ns);
-    const float saved = step * float(nT) * (1.f - 1.f / float(ns));
-    const float cost = 4.f + 1.4e-6f * float(ns * outs) * float(rows) * float(a.D);
-    if (room && saved > 1.45f * cost) return ns;
+  const int64_t rows = int64_t(a.B) * a.H * a.T, per_head = int64_t(a.B) * nblk * (f32 ? 2 : 1), W = per_head * a.H;
+  const int d = a.D <= 32 ? 0 : a.D == 64 ? 1 : a.D == 128 ? 2 : 3, outs = pass == SPLIT_DKDV ? 2 : 1;
+  if (W > (f32 ? 2048 : 512)) return 1;  // (several a CU already; 16-bit lists are cut in three and more there at a loss)
+  constexpr float step16[4][3] = {{1.0f, 0.85f, 1.2f}, {1.15f, 1.07f, 1.55f}, {1.6f, 1.7f, 2.2f}, {3.0f, 5.2f, 6.7f}};
+  constexpr float crowd16[4][3] = {
+      {0.5f, 0.55f, 0.65f}, {0.75f, 0.95f, 0.95f}, {0.95f, 1.15f, 1.5f}, {1.2f, 1.25f, 1.2f}};
+  constexpr float step32[4] = {2.1f, 3.1f, 5.3f, 10.2f}, pass32[3] = {1.0f, 1.27f, 1.75f};
+  constexpr float crowd32[4] = {0.5f, 0.65f, 0.83f, 1.02f};
+  const float single = a.precision == KD_PREC_SINGLE ? 0.7f : 1.f;  // P and dS rounded once: fewer products
+  const float step = f32 ? step32[d] * pass32[pass] : step16[d][pass] * single, crowd = f32 ? crowd32[d] : crowd16[d][pass];
+  const float start = (f32 ? 0.75f : 0.5f) * (1.f + 0.4f * float(d));
+  auto us = [&](int ns) {
+    const int k = int((W * ns + 255) / 256);
+    float share = 1.f;
+    if (!full) {
+      if (ns == 1) share = k == 2 ? 0.35f : 0.67f;
+      else if (k > 2) share = 0.67f;
+      else if (a.H % 8 == 0 && per_head * ns >= 64 && nT >= 16) share = 0.25f;
+      else share = pass == SPLIT_FWD && !f32 ? 0.6f : 0.5f;
+    }
+    const float t = float((nT + ns - 1) / ns) * step * (1.f + crowd * float(k - 1) * share) + start * float(k);
+    return ns == 1 ? t : t + 4.5f + 1.4e-6f * float(ns * outs) * float(rows) * float(a.D);
+  };
+  const float whole = us(1);
+  float least = 0.9f * whole;
+  int best = 1;
+  for (int ns = 2; ns <= (f32 ? 6 : 4); ++ns) {
+    // two steps a piece; fp32, whose steps are longer, one where each piece has its CU to itself
+    if (nT < (f32 && W * ns <= 256 ? 1 : 2) * ns) continue;
+    if (const float t = us(ns); t < least) least = t, best = ns;
   }
-  return 1;
+  // fp32 lists of uneven length and 64 steps or more, whole heads an XCD: the lists of
+  // an XCD's last head are the kernel's tail however many come before.  Causal, forward
+  // and whole backward: B2 H8 T4096 d128 (W 1024) 647 / 2060 -> 625 / 1969, B1 H8 T8192 d128
+  // 1278 / 4069 -> 1192 / 3746, B1 H16 T4096 d64 433 / 1263 -> 351 / 1125.  Not at d = 256 (1364 -> 1435).
+  if (best == 1 && f32 && !full && a.D <= 128 && a.H % 8 == 0 && nT >= 64 && W <= 1024) best = 2;
+  return best;
 }
 
 int64_t split_floats(const AttnArgs& a, SplitPass pass) {

@@ -163,8 +163,10 @@ Tensor plan_of(int64_t B, int64_t T, int64_t D, c10::Device on, int64_t mode, co
   return plan;
 }
 
-kd_attn_args attn_args(const Tensor& q, const Tensor& k, const Tensor& v, double sm_scale, int64_t prec) {
+kd_attn_args attn_args(const Tensor& q, const Tensor& k, const Tensor& v, double sm_scale, int64_t prec,
+                       bool full = false) {
   kd_attn_args a{};
+  a.lists = full ? KD_LISTS_FULL : KD_LISTS_UNEVEN;
   a.B = int32_t(q.size(0)), a.H = int32_t(q.size(1)), a.T = int32_t(q.size(2)), a.D = int32_t(q.size(3));
   a.dtype = dtype_code(q.scalar_type());
   a.sm_scale = float(sm_scale);
@@ -227,6 +229,7 @@ struct AttnOpts {
   int64_t mode, prec;
   bool need_lo, bthd, fp8;
   Tensor* built;  // the plan used, for the caller
+  bool full() const { return mode == KD_MODE_ALL && !plan; }  // (attention._full_lists)
 };
 
 // kdattn::fwd and kdattn::bwd (attention.py) as one C++ node
@@ -251,7 +254,7 @@ struct Attention : torch::autograd::Function<Attention> {
                       : at::empty({B, H, T, D}, q.options());
     Tensor lse = at::empty({B, H, T}, f32), o_lo;
     if (x.need_lo) o_lo = at::empty({B, H, T, D}, x.prec == KD_PREC_SPLIT3 ? f32 : q.options());
-    kd_attn_args a = attn_args(q, k, v, x.sm_scale, x.prec);
+    kd_attn_args a = attn_args(q, k, v, x.sm_scale, x.prec, x.full());
     if (x.fp8) set_fp8(a, q8, k8, qs, ks);
     a.o = o.data_ptr();
     set3(a.o_strides, o);
@@ -271,6 +274,7 @@ struct Attention : torch::autograd::Function<Attention> {
     ctx->saved_data["prec"] = x.prec;
     ctx->saved_data["rot"] = x.signs.has_value();
     ctx->saved_data["fp8"] = x.fp8;
+    ctx->saved_data["full"] = x.full();
     return {o, lse};
   }
 
@@ -286,7 +290,8 @@ struct Attention : torch::autograd::Function<Attention> {
       const variable_list g =
           call_op("kdattn::bwd", {s[0], s[1], s[2], s[3], s[4], grads[0], s[5], ctx->saved_data["sm_scale"].toDouble(),
                                   s[6].defined() ? s[6] : at::empty({0}, s[3].options()), opt(fp8, i), opt(fp8, i + 1),
-                                  opt(fp8, i + 2), opt(fp8, i + 3), opt(rot, 7), ctx->saved_data["prec"].toInt()});
+                                  opt(fp8, i + 2), opt(fp8, i + 3), opt(rot, 7), ctx->saved_data["prec"].toInt(),
+                                  ctx->saved_data["full"].toBool()});
       for (int j = 0; j < 3; ++j) out[j] = g[j];
       return out;
     }
@@ -307,7 +312,8 @@ struct Attention : torch::autograd::Function<Attention> {
       const Tensor* ready[3] = {&q, &k, &v};
       for (int i = 0; i < 3; ++i) g[i] = grad_like(s[i], *ready[i]);
       const Tensor delta = at::empty({2, B, H, T}, q.options().dtype(at::kFloat));
-      kd_attn_args a = attn_args(q, k, v, ctx->saved_data["sm_scale"].toDouble(), ctx->saved_data["prec"].toInt());
+      kd_attn_args a = attn_args(q, k, v, ctx->saved_data["sm_scale"].toDouble(), ctx->saved_data["prec"].toInt(),
+                                 ctx->saved_data["full"].toBool());
       a.o = o.data_ptr();
       set3(a.o_strides, o);
       a.lse = static_cast<float*>(lse.data_ptr());
@@ -379,7 +385,7 @@ struct AttentionX3 : torch::autograd::Function<AttentionX3> {
     *x.built = plan;
     const Tensor ox = wide(q, Dp), lo = wide(q, Dp);
     Tensor lse = at::empty({B, H, T}, q.options());
-    kd_attn_args a = attn_args(p[0], p[1], p[2], x.sm_scale, KD_PREC_SPLIT);
+    kd_attn_args a = attn_args(p[0], p[1], p[2], x.sm_scale, KD_PREC_SPLIT, x.full());
     a.o = ox.data_ptr();
     set3(a.o_strides, ox);
     a.lse = static_cast<float*>(lse.data_ptr());

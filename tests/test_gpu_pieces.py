@@ -115,3 +115,14 @@ def test_pieces_capture(dev):
         g.replay()
         torch.cuda.synchronize()
         assert all(torch.equal(x, y) for x, y in zip(got, want)) and torch.isfinite(other).all()
+
+
+@pytest.mark.parametrize("B,H,T,D,dtype", [(1, 2, 1000, 64, BF), (1, 12, 700, 128, HF), (1, 2, 300, 32, F32)])
+def test_full_lists_against_the_oracle(dev, B, H, T, D, dtype):
+    """No mask: the lists are marked full, in the forward and the backward, which choose their own piece counts."""
+    a = _args(B, H, T, D, dtype)
+    a.lists = _lib.KD_LISTS_FULL
+    lib = _lib.load()
+    assert lib.kd_attn_fwd_ws_bytes(ctypes.byref(a)) > 0 or lib.kd_attn_bwd_ws_bytes(ctypes.byref(a)) > 0
+    q, k, v, do = qkvdo(B, H, T, D, seed=T, dtype=dtype)
+    _case(dict(name=f"full {B} {H} {T} {D}", q=q, k=k, v=v, do=do, causal=False), dev)
