@@ -154,3 +154,16 @@ def test_projection_forms(dev):
     g64, = torch.autograd.grad((2 * (z.detach().double() @ w64.T) @ w64).sum(), w64)
     assert (gw.double() - g64).norm() <= 0.05 * g64.norm()
     assert set(p.state_dict()) == {"weight"}
+
+
+@pytest.mark.parametrize("D,own", [(8, False), (24, False), (32, True)])
+def test_many_narrow_rows(dev, D, own):
+    """Both sides of the rule on narrow rows: torch's expressions past 2^17 of them, unless they are 32 wide."""
+    for rows, want in ((1 << 17, True), ((1 << 17) + 1, own)):
+        x = torch.randn(rows, D, device=dev).bfloat16().requires_grad_(True)
+        y = RMSNorm()(x)
+        assert ("CppFunction" in type(y.grad_fn).__name__) == want
+        ref = x.detach().double()
+        ref = ref * torch.rsqrt(ref.pow(2).mean(-1, keepdim=True) + 1e-6)
+        # torch's form rounds the square, the mean, the factor and the product to bf16 (2^-9 each)
+        assert (y.detach().double() - ref).norm() <= 2.0 ** -7 * ref.norm()
