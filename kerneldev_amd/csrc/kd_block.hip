@@ -7,6 +7,8 @@
 // at the end (the eager forms round after every operation and move each
 // intermediate through memory; B8 T2048, D 768 and hidden 2048, bf16, us:
 // norm 36 -> 10 forward, 100 -> 14 backward; gate 61 -> 33 and 96 -> 51).
+#include <algorithm>
+
 #include "kd_internal.h"
 
 namespace kd {
@@ -146,16 +148,25 @@ int by_type(int dtype, F f) {
   return hipGetLastError() == hipSuccess ? KD_OK : KD_ERR_LAUNCH;
 }
 
+// A launch holds less than 2^32 threads: longer inputs go in several.  f(first, count)
+template <class F>
+void in_launches(int64_t n, int64_t most, F f) {
+  for (int64_t i = 0; i < n; i += most) f(i, std::min(most, n - i));
+}
+constexpr int64_t LAUNCH_ROWS = int64_t(1) << 25;   // 64 threads a row
+constexpr int64_t LAUNCH_WORDS = int64_t(1) << 31;  // a thread a word of eight
+
 }  // namespace
 
 int launch_rms_fwd(const void* x, void* y, float* rstd, int64_t rows, int D, int dtype, float eps, hipStream_t st) {
   return by_type(dtype, [&](auto e) {
     using E = decltype(e);
     const int words = D / 8;
-    const dim3 grid(unsigned((rows + 3) / 4));
     auto go = [&](auto k) {
-      hipLaunchKernelGGL(k, grid, dim3(256), 0, st, static_cast<const u32x4*>(x), static_cast<u32x4*>(y), rstd, rows,
-                         words, eps);
+      in_launches(rows, LAUNCH_ROWS, [&](int64_t r, int64_t n) {
+        hipLaunchKernelGGL(k, dim3(unsigned((n + 3) / 4)), dim3(256), 0, st, static_cast<const u32x4*>(x) + r * words,
+                           static_cast<u32x4*>(y) + r * words, rstd == nullptr ? rstd : rstd + r, n, words, eps);
+      });
     };
     if (words <= 64) go(k_rms_fwd<E, 1>);
     else if (words <= 128) go(k_rms_fwd<E, 2>);
@@ -168,10 +179,12 @@ int launch_rms_bwd(const void* x, const void* dy, const float* rstd, void* dx, i
   return by_type(dtype, [&](auto e) {
     using E = decltype(e);
     const int words = D / 8;
-    const dim3 grid(unsigned((rows + 3) / 4));
     auto go = [&](auto k) {
-      hipLaunchKernelGGL(k, grid, dim3(256), 0, st, static_cast<const u32x4*>(x), static_cast<const u32x4*>(dy), rstd,
-                         static_cast<u32x4*>(dx), rows, words);
+      in_launches(rows, LAUNCH_ROWS, [&](int64_t r, int64_t n) {
+        hipLaunchKernelGGL(k, dim3(unsigned((n + 3) / 4)), dim3(256), 0, st, static_cast<const u32x4*>(x) + r * words,
+                           static_cast<const u32x4*>(dy) + r * words, rstd + r, static_cast<u32x4*>(dx) + r * words, n,
+                           words);
+      });
     };
     if (words <= 64) go(k_rms_bwd<E, 1>);
     else if (words <= 128) go(k_rms_bwd<E, 2>);
@@ -181,17 +194,23 @@ int launch_rms_bwd(const void* x, const void* dy, const float* rstd, void* dx, i
 
 int launch_gate_fwd(const void* a, const void* b, void* y, int64_t n, int dtype, hipStream_t st) {
   return by_type(dtype, [&](auto e) {
-    hipLaunchKernelGGL(k_gate_fwd<decltype(e)>, dim3(unsigned((n + 2047) / 2048)), dim3(256), 0, st,
-                       static_cast<const uint16_t*>(a), static_cast<const uint16_t*>(b), static_cast<uint16_t*>(y), n);
+    in_launches(n, 8 * LAUNCH_WORDS, [&](int64_t i, int64_t m) {
+      hipLaunchKernelGGL(k_gate_fwd<decltype(e)>, dim3(unsigned((m + 2047) / 2048)), dim3(256), 0, st,
+                         static_cast<const uint16_t*>(a) + i, static_cast<const uint16_t*>(b) + i,
+                         static_cast<uint16_t*>(y) + i, m);
+    });
   });
 }
 
 int launch_gate_bwd(const void* a, const void* b, const void* dy, void* da, void* db, int64_t n, int dtype,
                     hipStream_t st) {
   return by_type(dtype, [&](auto e) {
-    hipLaunchKernelGGL(k_gate_bwd<decltype(e)>, dim3(unsigned((n + 2047) / 2048)), dim3(256), 0, st,
-                       static_cast<const uint16_t*>(a), static_cast<const uint16_t*>(b),
-                       static_cast<const uint16_t*>(dy), static_cast<uint16_t*>(da), static_cast<uint16_t*>(db), n);
+    in_launches(n, 8 * LAUNCH_WORDS, [&](int64_t i, int64_t m) {
+      hipLaunchKernelGGL(k_gate_bwd<decltype(e)>, dim3(unsigned((m + 2047) / 2048)), dim3(256), 0, st,
+                         static_cast<const uint16_t*>(a) + i, static_cast<const uint16_t*>(b) + i,
+                         static_cast<const uint16_t*>(dy) + i, static_cast<uint16_t*>(da) + i,
+                         static_cast<uint16_t*>(db) + i, m);
+    });
   });
 }
 

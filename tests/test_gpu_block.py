@@ -167,3 +167,21 @@ def test_many_narrow_rows(dev, D, own):
         ref = ref * torch.rsqrt(ref.pow(2).mean(-1, keepdim=True) + 1e-6)
         # torch's form rounds the square, the mean, the factor and the product to bf16 (2^-9 each)
         assert (y.detach().double() - ref).norm() <= 2.0 ** -7 * ref.norm()
+
+
+def test_more_rows_than_a_launch_holds(dev):
+    """2^26 rows of a wave each are 2^32 threads: the rows at every launch's ends, forward and backward."""
+    rows, D = (1 << 26) + 5, 32
+    x = torch.randn(rows, D, device=dev, dtype=torch.bfloat16, generator=torch.Generator(dev).manual_seed(1))
+    dy = torch.randn(rows, D, device=dev, dtype=torch.bfloat16, generator=torch.Generator(dev).manual_seed(2))
+    x.requires_grad_(True)
+    y = RMSNorm()(x)
+    assert "CppFunction" in type(y.grad_fn).__name__
+    dx, = torch.autograd.grad(y, x, dy)
+    at = torch.cat([torch.arange(max(0, i - 64), min(rows, i + 64)) for i in (0, 1 << 25, 1 << 26, rows)]).to(dev)
+    x64 = x.detach()[at].double().requires_grad_(True)
+    y64 = x64 * torch.rsqrt(x64.pow(2).mean(-1, keepdim=True) + 1e-6)
+    want, = torch.autograd.grad(y64, x64, dy[at].double())
+    # one rounding of fp32 results: 2^-9
+    assert (y.detach()[at].double() - y64.detach()).norm() <= 2.0 ** -8 * y64.detach().norm()
+    assert (dx[at].double() - want).norm() <= 2.0 ** -8 * want.norm()
