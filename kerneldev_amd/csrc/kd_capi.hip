@@ -151,7 +151,10 @@ static int check_x3(const kd_x3_args* a, bool pack) {
   if (a->B < 1 || a->H < 1 || a->T < 1) return fail(KD_ERR_INVALID, "B, H and T must be >= 1");
   if (a->d != 16 && a->d != 32 && a->d != 64) return fail(KD_ERR_UNSUPPORTED, "d must be 16, 32 or 64");
   if (a->Dp < 3 * a->d || a->Dp > 256 || a->Dp % 8 != 0) return fail(KD_ERR_INVALID, "Dp must hold three rows of d");
-  if (int64_t(a->B) * a->H * a->T > (int64_t(1) << 33)) return fail(KD_ERR_UNSUPPORTED, "too many rows");
+  // one thread a word of eight columns; a launch holds less than 2^32 threads, and wraps past that without an error
+  const int64_t rows = int64_t(a->B) * a->H * a->T;
+  if (rows > (int64_t(1) << 31) || rows * ((pack ? a->Dp : a->d) / 8) > (int64_t(1) << 32) - 256)
+    return fail(KD_ERR_UNSUPPORTED, "too many rows");
   for (int i = 0; i < a->n; ++i) {
     const void* f32 = pack ? a->src[i] : a->dst[i];
     const int64_t* st = pack ? a->src_strides[i] : a->dst_strides[i];
@@ -257,6 +260,7 @@ int kd_signs(const uint64_t* bits, int32_t d, float* signs, void* stream) {
 int kd_span_count(const kd_span_args* a, int32_t* counts, void* stream) {
   if (a == nullptr) return fail(KD_ERR_INVALID, "args is NULL");
   if (a->B < 1 || a->T < 1) return fail(KD_ERR_INVALID, "B and T must be >= 1");
+  if (a->B >= (1 << 26)) return fail(KD_ERR_UNSUPPORTED, "B must be < 2^26");  // a wave a row, 2^32 threads a launch
   if (a->tokens_dtype != KD_I64 && a->tokens_dtype != KD_I32) return fail(KD_ERR_INVALID, "bad tokens dtype");
   if (a->tokens == nullptr || counts == nullptr) return fail(KD_ERR_INVALID, "tokens and counts are required");
   if (a->tokens_strides[0] < 0 || a->tokens_strides[1] < 0) return fail(KD_ERR_INVALID, "negative token strides");
