@@ -146,3 +146,13 @@ def test_span_count(dev, dtype):
         tokens = torch.randint(0, 6, (B, T), generator=g).to(dtype)
         assert max_spans(tokens.to(dev)) == max_spans(tokens)
         assert max_spans(tokens.T.contiguous().T.to(dev)) == max_spans(tokens)
+
+
+@pytest.mark.parametrize("B,T,own", [(1, 8192, True), (1, 8193, False), (1024, 8, True), (1025, 8, False)])
+def test_span_count_route(dev, B, T, own):
+    """Both sides of the count kernel's limits, and the same count."""
+    from kerneldev_amd import _lib
+
+    tokens = torch.randint(0, 6, (B, T), generator=torch.Generator().manual_seed(T))
+    assert (_lib.native().span_counts(tokens.to(dev)) is not None) == own
+    assert max_spans(tokens.to(dev)) == max_spans(tokens)
