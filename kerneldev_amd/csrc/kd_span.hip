@@ -5,13 +5,12 @@
 // the zipped [SPAN] / [ES] position lists, taking x_embed[i, st+1:ed].mean(0)
 // when st + 1 < ed (model.py:287-293), and scores each span by its dot
 // product with the hidden state at the row's first [MASK] (:264-270, :296).
-// Here, up to FUSE_T tokens, FUSE_D columns and FUSE_NT scanned tokens, one workgroup per (row, span)
+// Here, where one_launch says so, one workgroup per (row, span)
 // finds its own span's markers (block scans give the j-th [SPAN] and the j-th
 // [ES] of the row), sums the interior in fp32 (eight waves over interleaved
 // rows, combined in a fixed order) and dots the mean with the context vector:
 // one launch of 10.7 us at B8 T2048 D768 with 8 spans, where the same in three
-// (k_span_find, k_span_pool, k_span_score, which longer and wider rows keep, as
-// every workgroup would scan the whole row) takes 20 us.  The backward spreads
+// (k_span_find, k_span_pool, k_span_score) takes 20 us.  The backward spreads
 // d score over the interior rows and the [MASK] row in a fixed order, so the
 // results are deterministic.
 #include "kd_internal.h"
@@ -152,16 +151,12 @@ __global__ __launch_bounds__(256) void k_span_score(kd_span_args a) {
   if (threadIdx.x == 0) a.scores[int64_t(b) * n + j] = s;
 }
 
-// Rows of up to FUSE_T tokens and FUSE_D columns: k_span_find, k_span_pool and
-// k_span_score in one launch, grid (n_spans + 1, B), 512 threads.  Block (j, b)
-// scans row b itself (thread i a contiguous run of tokens, two block scans for
-// the ordinals), keeps the positions of the j-th [SPAN] and [ES] and the first
+// k_span_find, k_span_pool and k_span_score in one launch (where: one_launch),
+// grid (n_spans + 1, B), 512 threads.  Block (j, b) scans row b itself (thread i
+// a contiguous run of tokens, two block scans for the ordinals), keeps the positions of the j-th [SPAN] and [ES] and the first
 // [MASK], then sums its interior 256 columns at a time (wave w the rows lo + w,
 // lo + w + 8, ..., lane l the columns 4 l .. 4 l + 3) and its score.  The sums
 // run in the order of the three kernels.  Block (n, b) writes h_ctx.
-constexpr int FUSE_T = 16384, FUSE_D = 2048;
-constexpr int64_t FUSE_NT = 1 << 20;  // span columns times tokens: what the blocks of a row scan
-
 template <class E, bool VEC>
 __global__ __launch_bounds__(512) void k_span_all(kd_span_args a) {
   __shared__ float s_part[8][256];
@@ -252,9 +247,7 @@ __global__ __launch_bounds__(512) void k_span_all(kd_span_args a) {
 // dh's strides and every base allow it; without, columns d0 + l + 64 k.  25 MB of
 // dh at B8 T2048 D768: 32 us with one row a wave and 2-byte stores, 23.6 with
 // 16-byte stores, 14.6 with four rows a wave and the [MASK] row's loads overlapped.
-constexpr int BWD_R = 4;
-
-template <class E, bool VEC>
+template <class E, bool VEC, int BWD_R>
 __global__ __launch_bounds__(256) void k_span_bwd(kd_span_args a) {
   const int lane = threadIdx.x & 63;
   const int b = blockIdx.y, n = a.n_spans, D = a.D;
@@ -320,11 +313,29 @@ bool multiple(const void* p, const int64_t* strides, int D, int of) {  // a base
   return reinterpret_cast<uintptr_t>(p) % (2 * of) == 0 && strides[0] % of == 0 && strides[1] % of == 0 && D % of == 0;
 }
 
+// Where one launch is the faster one.  Each of its (n + 1) B workgroups scans its
+// row's T tokens and walks the columns 256 at a time, where k_span_find scans a row once and
+// k_span_pool has a workgroup for every 256 columns; without 8-byte loads (vec) its
+// columns take up to six times as long.  So the scans have to be few (2^21
+// tokens) or small beside the columns that a row is pooled over, and the columns one
+// group without vec, four with it, eight where the workgroups fill a quarter of the chip.  us, one
+// launch / three: B8 T2048 D768 n8 8.9 / 15.4; B1 T2048 n1 L1945 D768 47 / 112, D2048 209 / 109, D770 290 / 108;
+// B64 T16384 n60 D64 274 / 70; B64 T4096 n4 D2048 124 / 366.  Over 1902 timed shapes none is
+// slower than three launches by 2%.
+bool one_launch(const kd_span_args& a, bool vec) {
+  const int64_t n = a.n_spans, blocks = (n + 1) * a.B;
+  const bool small_scan = 16 * (n + 1) <= a.D;
+  if (a.T > 16384 || n * a.T > (1 << 20)) return false;
+  if (a.D <= (vec ? 1024 : 256)) return blocks * a.T <= (1 << 21) || small_scan;
+  return vec && a.D <= 2048 && blocks >= 64 && small_scan;
+}
+
 template <class E>
 void launch_span_e(const kd_span_args& a, hipStream_t st) {
-  if (a.T <= FUSE_T && a.D <= FUSE_D && int64_t(a.n_spans) * a.T <= FUSE_NT) {
+  const bool vec = multiple(a.h, a.h_strides, a.D, 4);
+  if (one_launch(a, vec)) {
     const dim3 grid(unsigned(a.n_spans + 1), unsigned(a.B));
-    if (multiple(a.h, a.h_strides, a.D, 4)) hipLaunchKernelGGL((k_span_all<E, true>), grid, dim3(512), 0, st, a);
+    if (vec) hipLaunchKernelGGL((k_span_all<E, true>), grid, dim3(512), 0, st, a);
     else hipLaunchKernelGGL((k_span_all<E, false>), grid, dim3(512), 0, st, a);
     return;
   }
@@ -334,12 +345,19 @@ void launch_span_e(const kd_span_args& a, hipStream_t st) {
   hipLaunchKernelGGL(k_span_score, dim3(unsigned(a.n_spans), unsigned(a.B)), dim3(256), 0, st, a);
 }
 
+template <class E, int R>
+void launch_span_bwd_r(const kd_span_args& a, hipStream_t st) {
+  const dim3 grid(unsigned((a.T + 4 * R - 1) / (4 * R)), unsigned(a.B));
+  auto aligned = [](const float* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+  if (multiple(a.dh, a.dh_strides, a.D, 8) && aligned(a.h_ctx) && aligned(a.h_spans))
+    hipLaunchKernelGGL((k_span_bwd<E, true, R>), grid, dim3(256), 0, st, a);
+  else
+    hipLaunchKernelGGL((k_span_bwd<E, false, R>), grid, dim3(256), 0, st, a);
+}
+
 template <class E>
 void launch_span_bwd_e(const kd_span_args& a, hipStream_t st) {
-  const dim3 grid(unsigned((a.T + 4 * BWD_R - 1) / (4 * BWD_R)), unsigned(a.B));
-  auto aligned = [](const float* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
-  if (multiple(a.dh, a.dh_strides, a.D, 8) && aligned(a.h_ctx) && aligned(a.h_spans)) hipLaunchKernelGGL((k_span_bwd<E, true>), grid, dim3(256), 0, st, a);
-  else hipLaunchKernelGGL((k_span_bwd<E, false>), grid, dim3(256), 0, st, a);
+  launch_span_bwd_r<E, 4>(a, st);
 }
 
 }  // namespace

@@ -4,8 +4,9 @@ Replaces the head of KernelDev's ``GPTModel.forward`` (``model.py:263-298``):
 the hidden state at each row's first ``[MASK]`` is dotted with the mean hidden
 state of every span interior.  The reference fills ``h_spans`` with a Python
 double loop over rows and over the zipped ``[SPAN]`` / ``[ES]`` positions
-(``:287-293``); here ``kd_span_scores`` does the pooling and the scores in two
-kernel launches and ``kd_span_scores_bwd`` returns ``d h``.
+(``:287-293``); here ``kd_span_scores`` does the pooling and the scores in one
+kernel launch (three where rows are long or wide) and ``kd_span_scores_bwd``
+returns ``d h``.
 
 Pairing: the j-th ``[SPAN]`` of a row goes with the row's j-th ``[ES]``, as the
 reference's ``zip(st_indices, ed_indices)`` does when a row holds as many of

@@ -156,3 +156,20 @@ def test_span_count_route(dev, B, T, own):
     tokens = torch.randint(0, 6, (B, T), generator=torch.Generator().manual_seed(T))
     assert (_lib.native().span_counts(tokens.to(dev)) is not None) == own
     assert max_spans(tokens.to(dev)) == max_spans(tokens)
+
+
+@pytest.mark.parametrize("B,T,D,n", [(1, 700, 256, 3), (1, 700, 258, 3), (1, 700, 1024, 3), (1, 700, 1028, 3),
+                                     (16, 300, 1028, 3), (15, 300, 1028, 3), (16, 300, 2048, 3), (16, 300, 2052, 3),
+                                     (1, 8192, 64, 128), (1, 8200, 64, 128), (1, 1500, 64, 70), (64, 1200, 16, 27)])
+def test_lines_of_the_one_launch_rule(dev, B, T, D, n):
+    """Both sides of each line of the one-launch rule: the widths with and without 8-byte loads, the workgroups that
+    eight column groups need, and the scanned tokens."""
+    g = torch.Generator().manual_seed(T + D)
+    rows = []
+    for b in range(B):
+        row = [X] * int(torch.randint(0, 5, (1,), generator=g)) + [MASK]
+        for _ in range(n):
+            row += [SPAN] + [X] * int(torch.randint(0, max(1, (T - 8) // n - 3), (1,), generator=g)) + [ES]
+        rows.append(row + [X] * (T - len(row)))
+    h = torch.randn(B, T, D, generator=g).to(torch.bfloat16)
+    _check(torch.tensor(rows, dtype=torch.int64), h, dev, seed=D)
