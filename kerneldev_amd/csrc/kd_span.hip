@@ -236,7 +236,7 @@ __global__ __launch_bounds__(512) void k_span_all(kd_span_args a) {
   if (tid == 0) a.scores[int64_t(b) * n + j] = (s_red[0] + s_red[1]) + (s_red[2] + s_red[3]);
 }
 
-// grid (ceil(T / 16), B), one wave per BWD_R rows t of dh, each written in full:
+// grid (ceil(T / (4 BWD_R)), B), one wave per BWD_R rows t of dh, each written in full:
 //   dh[t] = sum_{j: lo_j <= t < hi_j} ds_j h_ctx / (hi_j - lo_j)   (ascending j)
 //         + [t == mask] sum_j ds_j h_span_j                          (ascending j)
 // Columns go in groups of 512.  The spans containing t are found 64 at a time
@@ -355,9 +355,13 @@ void launch_span_bwd_r(const kd_span_args& a, hipStream_t st) {
     hipLaunchKernelGGL((k_span_bwd<E, false, R>), grid, dim3(256), 0, st, a);
 }
 
+// Up to 8192 rows a wave takes one, so that there are waves for every CU: us, one
+// row a wave / four: B1 T2048 D768 6.5 / 8.0, D2048 6.8 / 14.3, B4 T2048 D2048 11.3 / 18; B16 T1024 D1024 with 60
+// spans 34 / 27, B64 T2048 D768 63 / 58.
 template <class E>
 void launch_span_bwd_e(const kd_span_args& a, hipStream_t st) {
-  launch_span_bwd_r<E, 4>(a, st);
+  if (int64_t(a.B) * a.T <= 8192) launch_span_bwd_r<E, 1>(a, st);
+  else launch_span_bwd_r<E, 4>(a, st);
 }
 
 }  // namespace

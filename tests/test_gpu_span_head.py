@@ -173,3 +173,12 @@ def test_lines_of_the_one_launch_rule(dev, B, T, D, n):
         rows.append(row + [X] * (T - len(row)))
     h = torch.randn(B, T, D, generator=g).to(torch.bfloat16)
     _check(torch.tensor(rows, dtype=torch.int64), h, dev, seed=D)
+
+
+@pytest.mark.parametrize("B,T", [(1, 8192), (1, 8193), (2, 4097), (3, 2730)])
+def test_backward_rows_a_wave(dev, B, T):
+    """Both sides of the backward's 8192 rows, with ends that are no multiple of its 4 or 16 rows a workgroup."""
+    row = [X] * 3 + [MASK, SPAN] + [X] * (T // 2) + [ES, X, SPAN, X, X, ES]
+    tokens = torch.tensor([row + [X] * (T - len(row))] * B, dtype=torch.int64)
+    h = torch.randn(B, T, 40, generator=torch.Generator().manual_seed(T)).to(torch.bfloat16)
+    _check(tokens, h, dev, seed=T)
