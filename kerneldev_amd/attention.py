@@ -21,7 +21,6 @@ There is no CPU or PyTorch fallback: a missing library raises.
 from __future__ import annotations
 
 import ctypes
-import math
 
 import torch
 
@@ -405,23 +404,6 @@ X3_HEAD_DIMS = {16: 64, 32: 128, 64: 256}
 X3_ROUTED_HEAD_DIMS = (16, 32)
 
 
-def _x3(x: torch.Tensor, pattern: str, Dp: int) -> torch.Tensor:
-    """[B, H, T, d] fp32 -> contiguous bf16 [B, H, T, Dp]: the parts named by pattern ('h', 'l'), then zeros."""
-    xh = x.to(torch.bfloat16)
-    xl = (x - xh.to(torch.float32)).to(torch.bfloat16)
-    parts = [xh if c == "h" else xl for c in pattern]
-    pad = Dp - len(pattern) * x.shape[-1]
-    if pad:
-        parts.append(xh.new_zeros(x.shape[:-1] + (pad,)))
-    return torch.cat(parts, dim=-1)
-
-
-def _hi_lo(hi: torch.Tensor, lo: torch.Tensor, d: int, second: int) -> torch.Tensor:
-    """fp32 (hi + lo)[..., 0:d] + (hi + lo)[..., second * d:(second + 1) * d]."""
-    x = hi.to(torch.float32).add_(lo.to(torch.float32))
-    return x[..., :d] + x[..., second * d:(second + 1) * d]
-
-
 def _x3_call(pack: bool, tensors, B, H, T, d, Dp):
     """kd_x3_pack of ``(x, y, pattern)`` or kd_x3_unpack of ``(hi, lo, out, second)``, all in one launch."""
     a = _lib.X3Args()
@@ -774,6 +756,3 @@ def tile_masks(plan: torch.Tensor, B: int, T: int, D: int):
 
 def mask_mode(in_span=None, span_id=None, is_prefix=None, attention_mask=None, causal=True) -> int:
     return _mode(in_span, span_id, is_prefix, attention_mask is not None, causal)
-
-
-LOG2E = math.log2(math.e)

@@ -1,5 +1,6 @@
 """CPU: the operand layout of the bf16x3 path for fp32 inputs, and which kernels
-flash_attention picks per dtype and head dim (kerneldev_amd.attention).
+flash_attention picks per dtype and head dim (kerneldev_amd.attention).  The
+layout is proven on its torch form; test_gpu_x3.py holds the kernels to that form.
 
 The kernels see Q' = [Qh, Qh, Ql], K' = [Kh, Kl, Kh], V' = [Vh, Vl, Vh],
 dO' = [dOh, dOh, dOl] (zero-padded) and compute every product of the
@@ -12,7 +13,8 @@ block (the mistakes this layout invites) is off by O(1) or by 2^-8.
 import pytest
 import torch
 
-from kerneldev_amd.attention import X3_HEAD_DIMS, _hi_lo, _x3
+from kerneldev_amd.attention import X3_HEAD_DIMS
+from x3_reference import hi_lo, x3
 
 
 def _rel(x, ref):
@@ -26,7 +28,7 @@ def test_every_product_through_the_expanded_operands(d):
     q, k, v, do = (torch.randn(1, 1, T, d, generator=g) * 3 for _ in range(4))
     p = torch.softmax(torch.randn(T, T, generator=g, dtype=torch.float64), dim=-1)
     ds = torch.randn(T, T, generator=g, dtype=torch.float64)
-    qx, kx, vx, dox = (_x3(x, pat, Dp)[0, 0].double() for x, pat in ((q, "hhl"), (k, "hlh"), (v, "hlh"), (do, "hhl")))
+    qx, kx, vx, dox = (x3(x, pat, Dp)[0, 0].double() for x, pat in ((q, "hhl"), (k, "hlh"), (v, "hlh"), (do, "hhl")))
     q, k, v, do = (x[0, 0].double() for x in (q, k, v, do))
     assert qx.shape == (T, Dp) and (qx[:, 3 * d:] == 0).all()
     bound = 2.0 ** -15
@@ -36,17 +38,17 @@ def test_every_product_through_the_expanded_operands(d):
     zero = torch.zeros(T, Dp, dtype=torch.float64)
     # outputs: O = P V' in blocks [0, d) + [d, 2d); dQ = dS K' in [0, d) + [d, 2d);
     # dK = dS^T Q' and dV = P^T dO' in [0, d) + [2d, 3d)
-    assert _rel(_hi_lo(p @ vx, zero, d, 1), p @ v) < bound
-    assert _rel(_hi_lo(ds @ kx, zero, d, 1), ds @ k) < bound
-    assert _rel(_hi_lo(ds.T @ qx, zero, d, 2), ds.T @ q) < bound
-    assert _rel(_hi_lo(p.T @ dox, zero, d, 2), p.T @ do) < bound
+    assert _rel(hi_lo(p @ vx, zero, d, 1), p @ v) < bound
+    assert _rel(hi_lo(ds @ kx, zero, d, 1), ds @ k) < bound
+    assert _rel(hi_lo(ds.T @ qx, zero, d, 2), ds.T @ q) < bound
+    assert _rel(hi_lo(p.T @ dox, zero, d, 2), p.T @ do) < bound
 
 
 def test_hi_lo_adds_the_residual():
     x = torch.randn(2, 3, 5, 64, dtype=torch.float32)
     hi = x.to(torch.bfloat16)
     lo = (x - hi.float()).to(torch.bfloat16)
-    got = _hi_lo(hi, lo, 16, 2)
+    got = hi_lo(hi, lo, 16, 2)
     want = (hi.float() + lo.float())[..., :16] + (hi.float() + lo.float())[..., 32:48]
     assert torch.equal(got, want)
     assert _rel(got.double(), (x[..., :16] + x[..., 32:48]).double()) < 2.0 ** -15
