@@ -646,12 +646,12 @@ def flash_attention(
     in_dtype = q.dtype
     if in_dtype not in (torch.bfloat16, torch.float16, torch.float32):
         raise ValueError(f"unsupported dtype {in_dtype}")
+    if k.dtype != in_dtype or v.dtype != in_dtype:  # the kernels read all three as q's type
+        k, v = k.to(in_dtype), v.to(in_dtype)
     if qk_dtype == "fp8_e4m3" and in_dtype == torch.float32:
         # fp8 scores come from bf16 operands: fp32 inputs are rounded to bf16
         # for this path and O cast back
         q, k, v = q.to(torch.bfloat16), k.to(torch.bfloat16), v.to(torch.bfloat16)
-    if k.dtype != q.dtype or v.dtype != q.dtype:  # the kernels read all three as q's type
-        k, v = k.to(q.dtype), v.to(q.dtype)
     from .hadamard import _rot_op, generate_hadamard_signs
 
     fused_signs = None
