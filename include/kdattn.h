@@ -19,7 +19,7 @@
  *     (b, h, t) strides multiples of 8 elements, the t stride >= D and
  *     T * t_stride * element size < 2^31 bytes.
  *   - Head dims 16, 32, 64, 128, 256 (original_kernel.py:1720).  bf16 / fp16
- *     run on the MFMA kernels at every head dim (16 and 32 on the D = 64
+ *     run on the MFMA kernels at every head dim (16 on the D = 32
  *     kernels, which read the columns past D as zeros and store only the D
  *     real ones; dqk_signs at 64, 128 only; fp8 scores at 64, 128, 256 for bf16); fp32 inputs
  *     on the fp32 MFMA kernels at every head dim (16 on the D = 32 kernels,

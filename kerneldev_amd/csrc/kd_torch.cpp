@@ -8,8 +8,10 @@
 // step: 309 us a forward and backward at fp32 B2 H4 T256 d64, whose kernels
 // run for 78 us.  The same work here -- the same checks, allocations, kernels
 // and saved tensors, under a C++ autograd::Function -- takes 104 us (fp16 B4
-// H8 T777 d32: 322 -> 88; span_scores of B8 T2048 D768: 226 -> 96).  Every entry returns None where the call is not plain (see
-// plain()), and the caller then goes through the custom op.
+// H8 T777 d32: 322 -> 88; span_scores of B8 T2048 D768: 226 -> 96).  Every
+// entry returns None where the call is not plain (see plain()), and the caller
+// then goes through the custom op; a backward does the same where its
+// cotangent is not (plain_cotangent()).
 #include <ATen/ATen.h>
 #include <ATen/autocast_mode.h>
 #include <ATen/record_function.h>
