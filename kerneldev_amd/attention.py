@@ -154,6 +154,8 @@ def build_plan_from_tokens(tokens: torch.Tensor, head_dim: int, rule: str = "col
         raise ValueError(f"head_dim must be one of {SUPPORTED_HEAD_DIMS}")
     if lens is not None and (lens.dtype != torch.int32 or lens.dim() != 1 or lens.shape[0] != tokens.shape[0]):
         raise ValueError("lens must be an int32 tensor of shape [batch]")
+    if lens is not None and lens.device != tokens.device:  # (the kernel reads it)
+        raise ValueError("lens must be on the same device as tokens")
     B, T = tokens.shape
     if _lib.eager(tokens, lens):
         plan = _lib.native().plan_from_tokens(tokens, head_dim, RULES[rule], lens)

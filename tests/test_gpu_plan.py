@@ -252,3 +252,11 @@ def test_flash_attention_with_shared_plan(dev):
         flash_attention(q0, k0, v0, plan=plan, in_span=meta[0])
     with pytest.raises(ValueError, match="plan is for"):
         flash_attention(q0[:, :, :512], k0[:, :, :512], v0[:, :, :512], plan=plan)
+
+
+def test_plan_from_tokens_refuses_lens_on_the_host(dev):
+    from kerneldev_amd.attention import build_plan_from_tokens
+
+    tokens = torch.zeros(2, 64, dtype=torch.int64, device=dev)
+    with pytest.raises(ValueError, match="same device"):
+        build_plan_from_tokens(tokens, 64, lens=torch.tensor([3, 5], dtype=torch.int32))
