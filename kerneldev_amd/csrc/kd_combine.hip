@@ -178,7 +178,7 @@ int launch(const AttnArgs& a, const CombineArgs& c, bool fwd, int outputs, hipSt
 // mean, and 5 of 5832 slower by more than 1.5% (the worst 1.04 x).  The rule before it
 // knew neither k nor the mask: 1.24 times faster, 361 slower, up to 1.43 x.  Some, us
 // (forward / dQ / dK+dV):
-//   bf16 B1 H8 T4095 d128 causal (W 256): 96 / 102 / 135 -> 77 / 88 / 114 at 2
+//   bf16 B1 H8 T4096 d128 causal (W 256): 96 / 102 / 135 -> 77 / 88 / 114 at 2
 //   bf16 B1 H16 T2048 d64 causal (W 256): 39 / 36 / 50, 42 / 41 / 56 at 2: uncut
 //   bf16 B1 H12 T1400 d128 full (W 132): dK+dV 53, 76 at 2: uncut
 //   bf16 B1 H1 T8192 d64 causal (W 64): 132 / 134 / 160 -> 44 / 57 / 45 at 4

@@ -153,10 +153,11 @@ __global__ __launch_bounds__(256) void k_span_score(kd_span_args a) {
 
 // k_span_find, k_span_pool and k_span_score in one launch (where: one_launch),
 // grid (n_spans + 1, B), 512 threads.  Block (j, b) scans row b itself (thread i
-// a contiguous run of tokens, two block scans for the ordinals), keeps the positions of the j-th [SPAN] and [ES] and the first
-// [MASK], then sums its interior 256 columns at a time (wave w the rows lo + w,
-// lo + w + 8, ..., lane l the columns 4 l .. 4 l + 3) and its score.  The sums
-// run in the order of the three kernels.  Block (n, b) writes h_ctx.
+// a contiguous run of tokens, two block scans for the ordinals), keeps the
+// positions of the j-th [SPAN] and [ES] and the first [MASK], then sums its
+// interior 256 columns at a time (wave w the rows lo + w, lo + w + 8, ..., lane l
+// the columns 4 l .. 4 l + 3) and its score.  The sums run in the order of the
+// three kernels.  Block (n, b) writes h_ctx.
 template <class E, bool VEC>
 __global__ __launch_bounds__(512) void k_span_all(kd_span_args a) {
   __shared__ float s_part[8][256];
@@ -314,14 +315,15 @@ bool multiple(const void* p, const int64_t* strides, int D, int of) {  // a base
 }
 
 // Where one launch is the faster one.  Each of its (n + 1) B workgroups scans its
-// row's T tokens and walks the columns 256 at a time, where k_span_find scans a row once and
-// k_span_pool has a workgroup for every 256 columns; without 8-byte loads (vec) its
-// columns take up to six times as long.  So the scans have to be few (2^21
-// tokens) or small beside the columns that a row is pooled over, and the columns one
-// group without vec, four with it, eight where the workgroups fill a quarter of the chip.  us, one
-// launch / three: B8 T2048 D768 n8 8.9 / 15.4; B1 T2048 n1 L1945 D768 47 / 112, D2048 209 / 109, D770 290 / 108;
-// B64 T16384 n60 D64 274 / 70; B64 T4096 n4 D2048 124 / 366.  Over 1902 timed shapes none is
-// slower than three launches by 2%.
+// row's T tokens and walks the columns 256 at a time, where k_span_find scans a
+// row once and k_span_pool has a workgroup for every 256 columns; without 8-byte
+// loads (vec) its columns take up to six times as long.  So the scans have to be
+// few (2^21 tokens) or small beside the columns that a row is pooled over, and the
+// columns one group without vec, four with it, eight where the workgroups fill a
+// quarter of the chip.  us, one launch / three: B8 T2048 D768 n8 8.9 / 15.4; B1 T2048
+// n1 L1945 D768 47 / 112, D2048 209 / 109, D770 290 / 108; B64 T16384 n60 D64 274 / 70;
+// B64 T4096 n4 D2048 124 / 366.  Over 1902 timed shapes none is slower than three
+// launches by 2%.
 bool one_launch(const kd_span_args& a, bool vec) {
   const int64_t n = a.n_spans, blocks = (n + 1) * a.B;
   const bool small_scan = 16 * (n + 1) <= a.D;
