@@ -720,31 +720,16 @@ pybind11::object swiglu(const Tensor& a, const Tensor& b) {
   return pybind11::cast(Gate::apply(a, b));
 }
 
-// Where the weight gradient's own kernel is the faster one, for dW [N, K] over M
-// tokens.  P: the dW it computes, whole 128 x 128 tiles.  The library takes 18 to
-// 19 us up to about 2000 tokens whatever the size (it splits the tokens over the
-// chip) and grows from there; the own kernel takes 9 us where it is small and grows with M P.
-// So: a small P always; any P while M P is small; large M, unless most of a tile
-// is padding.  us, own / library, bf16: 768 x 768 over 2048 tokens 15.4 / 18.4, over 16384
-// 30 / 91; 2048 x 768 over 768 16.1 / 18.2, over 1536 20.3 / 18.6, over 2048 22.3 / 19.9, over 2560
-// 22.4 / 23.4, over 16384 63 / 132; 2048 x 1024 over 1024 19.4 / 18.4; 2048 x 512 over 2560 20.3 / 19.4,
-// over 4096 22.5 / 28.0; 512 x 2048 over 2560 17.9 / 19.3; 64 x 32768 over 4096 56 / 52.  Over 1270
-// timed (M, N, K) none is slower than the library's by 1%, and the mean gain is 1.26.
-bool weight_grad_pays(int64_t M, int64_t N, int64_t K) {
-  const int64_t P = (N + 127) / 128 * 128 * ((K + 127) / 128 * 128), Mi = int64_t(1) << 20;
-  if (N * K > 2 * Mi) return false;
-  if (P <= 3 * Mi / 4 || (P <= Mi && N <= 512)) return true;
-  if (M * P <= int64_t(1450000000)) return true;
-  return M >= (P > Mi ? 2560 : 3200) && P <= 9 * Mi / 4 && P <= 2 * N * K;
-}
-
+// Where the weight gradient's own kernel is the faster one: up to 2^21 weights
+// (us, own against library, bf16: 768 x 768 over 16384 tokens 31 / 93, over 2048
+// 15 / 19, over 128 8 / 19; 2048 x 768 over 16384 58 / 120, over 2048 21.6 / 19.8;
+// beyond, 4096 x 1024 over 2048 31 / 29, over 512 21.5 / 19)
 pybind11::object projection(const Tensor& x, const Tensor& w) {
   if (!block_mode() || !at::GradMode::is_enabled() || !w.requires_grad() || !flat16(x) || !flat16(w) || w.dim() != 2 ||
       x.dim() < 2 || x.size(-1) != w.size(1) || x.scalar_type() != w.scalar_type() || x.device() != w.device())
     return pybind11::none();
   const int64_t N = w.size(0), K = w.size(1), M = x.numel() / K;
-  if (N % 8 != 0 || K % 8 != 0 || !weight_grad_pays(M, N, K) || M * std::max(N, K) >= (int64_t(1) << 30))
-    return pybind11::none();
+  if (N % 8 != 0 || K % 8 != 0 || N * K > (1 << 21) || M * std::max(N, K) >= (int64_t(1) << 30)) return pybind11::none();
   return pybind11::cast(Projection::apply(x, w));
 }
 
@@ -793,7 +778,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("plan_from_metadata", torch::wrap_pybind_function(plan_from_metadata));
   m.def("plan_from_tokens", torch::wrap_pybind_function(plan_from_tokens));
   m.def("projection", torch::wrap_pybind_function(projection));
-  m.def("weight_grad_pays", &weight_grad_pays);
   m.def("rms_norm", torch::wrap_pybind_function(rms_norm));
   m.def("swiglu", torch::wrap_pybind_function(swiglu));
   m.def("signs", torch::wrap_pybind_function(signs));
