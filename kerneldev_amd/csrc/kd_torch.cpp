@@ -720,10 +720,16 @@ pybind11::object swiglu(const Tensor& a, const Tensor& b) {
   return pybind11::cast(Gate::apply(a, b));
 }
 
-// Where the weight gradient's own kernel is the faster one: up to 2^21 weights
-// (us, own against library, bf16: 768 x 768 over 16384 tokens 31 / 93, over 2048
-// 15 / 19, over 128 8 / 19; 2048 x 768 over 16384 58 / 120, over 2048 21.6 / 19.8;
-// beyond, 4096 x 1024 over 2048 31 / 29, over 512 21.5 / 19)
+// Where the weight gradient's own kernel is the faster one: up to 2^21 weights.
+// Alone on the GPU, own against library in us, bf16: 768 x 768 over 16384 tokens
+// 30 / 91, over 2048 15.4 / 18.4, over 128 10 / 18; 2048 x 768 over 16384 63 / 132, over
+// 2048 22.3 / 19.9, over 768 16.1 / 18.2; 2048 x 1024 over 1536 22.8 / 18.7; beyond, 4096 x 1024
+// over 2048 31 / 29, over 512 21.5 / 19.  A large dW over 1000 to 2500 tokens is the
+// library's by 1 to 4 us there, but its product costs the host 12 us more than the own
+// kernel's two launches, and a layer of that size is the host's: a block of B2
+// T1024, 768 and 2048 wide, forward and backward 796 us with the own products, 884 with
+// the library's from this node (GPU 449 / 484); of B3 T627, 1536 wide, 731 us, and
+// 849 with w1, w2 and w3 as torch's own linear.
 pybind11::object projection(const Tensor& x, const Tensor& w) {
   if (!block_mode() || !at::GradMode::is_enabled() || !w.requires_grad() || !flat16(x) || !flat16(w) || w.dim() != 2 ||
       x.dim() < 2 || x.size(-1) != w.size(1) || x.scalar_type() != w.scalar_type() || x.device() != w.device())
